@@ -404,6 +404,58 @@ __global__ void k_perm_in(int n, const int* __restrict__ perm, const double* __r
 // one thread per element; per sample F = x_e G_s, one SVD shared by every
 // projection, contribution sum_energies w A_s^T vec(p(F)).
 // -----------------------------------------------------------------------------
+// P = sum of the weighted projections of F (the muscle's with fiber mf, level ma)
+template <class TC>
+__device__ __forceinline__ void sample_projection(const DevMaterials& m, int e, double wc, double wv, double wm,
+                                                  const double (&mf)[3], double ma, const double (&F)[9], double (&P)[9]) {
+    // F in FP64 (positions minus the sum of their gradients cancel to
+    // O(1)); the SVD and the projections in TC
+    TC Fc[9];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) Fc[i] = (TC)F[i];
+    TC U[9], sg[3], V[9];
+    svd3(Fc, U, sg, V);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) P[i] = 0.0;
+    if (wc != 0.0) {
+        const TC one[3] = {TC(1), TC(1), TC(1)};
+        TC R[9];
+        udv(U, one, V, R);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) P[i] += wc * (double)R[i];
+    }
+    if (wv != 0.0) {
+        TC D[3], sd[3], Pv[9];
+        volume_D(sg, D);
+        sd[0] = sg[0] + D[0]; sd[1] = sg[1] + D[1]; sd[2] = sg[2] + D[2];
+        udv(U, sd, V, Pv);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) P[i] += wv * (double)Pv[i];
+    }
+    for (int h = 0; h < m.n_nh; ++h) {
+        const double wn = m.wn[h][e];
+        if (wn == 0.0) continue;
+        TC ss[3], Pn[9];
+        nh_prox((TC)m.nh_mu[h], (TC)m.nh_la[h], (TC)m.nh_k[h], sg, ss);
+        udv(U, ss, V, Pn);
+#pragma unroll
+        for (int i = 0; i < 9; ++i) P[i] += wn * (double)Pn[i];
+    }
+    if (wm != 0.0) {
+        // muscle (ProjectToManifold, pd_muscle_energy.cpp:118-125): Bp = a F m / |F m|,
+        // contribution w M^T Bp = w Bp m^T (FP64 in both precisions)
+        double Fm[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) Fm[i] = F[i] * mf[0] + F[i + 3] * mf[1] + F[i + 6] * mf[2];
+        const double l = sqrt(Fm[0] * Fm[0] + Fm[1] * Fm[1] + Fm[2] * Fm[2]);
+        const double r = l <= DBL_EPSILON ? 0.0 : wm * ma / l;
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) P[i + 3 * j] += r * Fm[i] * mf[j];
+    }
+}
+
 template <int EDIM, class TC>
 __global__ void __launch_bounds__(256) k_local_step(DevMaterials m, const double* __restrict__ q,
                                                     double* __restrict__ elem_out) {
@@ -438,53 +490,8 @@ __global__ void __launch_bounds__(256) k_local_step(DevMaterials m, const double
                 F[1 + 3 * jj] += x[k][1] * g;
                 F[2 + 3 * jj] += x[k][2] * g;
             }
-        // F in FP64 (positions minus the sum of their gradients cancel to
-        // O(1)); the SVD and the projections in TC
-        TC Fc[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) Fc[i] = (TC)F[i];
-        TC U[9], sg[3], V[9];
-        svd3(Fc, U, sg, V);
         double P[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) P[i] = 0.0;
-        if (wc != 0.0) {
-            const TC one[3] = {TC(1), TC(1), TC(1)};
-            TC R[9];
-            udv(U, one, V, R);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) P[i] += wc * (double)R[i];
-        }
-        if (wv != 0.0) {
-            TC D[3], sd[3], Pv[9];
-            volume_D(sg, D);
-            sd[0] = sg[0] + D[0]; sd[1] = sg[1] + D[1]; sd[2] = sg[2] + D[2];
-            udv(U, sd, V, Pv);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) P[i] += wv * (double)Pv[i];
-        }
-        for (int h = 0; h < m.n_nh; ++h) {
-            const double wn = m.wn[h][e];
-            if (wn == 0.0) continue;
-            TC ss[3], Pn[9];
-            nh_prox((TC)m.nh_mu[h], (TC)m.nh_la[h], (TC)m.nh_k[h], sg, ss);
-            udv(U, ss, V, Pn);
-#pragma unroll
-            for (int i = 0; i < 9; ++i) P[i] += wn * (double)Pn[i];
-        }
-        if (wm != 0.0) {
-            // muscle (ProjectToManifold, pd_muscle_energy.cpp:118-125): Bp = a F m / |F m|,
-            // contribution w M^T Bp = w Bp m^T (FP64 in both precisions)
-            double Fm[3];
-#pragma unroll
-            for (int i = 0; i < 3; ++i) Fm[i] = F[i] * mf[0] + F[i + 3] * mf[1] + F[i + 6] * mf[2];
-            const double l = sqrt(Fm[0] * Fm[0] + Fm[1] * Fm[1] + Fm[2] * Fm[2]);
-            const double r = l <= DBL_EPSILON ? 0.0 : wm * ma / l;
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-#pragma unroll
-                for (int i = 0; i < 3; ++i) P[i + 3 * j] += r * Fm[i] * mf[j];
-        }
+        sample_projection<TC>(m, e, wc, wv, wm, mf, ma, F, P);
 #pragma unroll
         for (int k = 0; k < EDIM; ++k)
 #pragma unroll
@@ -494,6 +501,84 @@ __global__ void __launch_bounds__(256) k_local_step(DevMaterials m, const double
     double* o = elem_out + (int64_t)e * EDIM * 3;
 #pragma unroll
     for (int k = 0; k < EDIM; ++k) { o[3 * k] = acc[k][0]; o[3 * k + 1] = acc[k][1]; o[3 * k + 2] = acc[k][2]; }
+}
+
+// lanes per element of the per-sample kernels
+template <int EDIM> struct Lanes { static constexpr int N = EDIM == 8 ? 8 : 1; };
+
+// Sum over the element's lanes of its per-vertex vectors: afterwards a[0] of lane s is
+// the sum for vertex s (hex: three halving exchanges, 21 values moved instead of the 72
+// of a butterfly over all 24). A tet's one lane keeps its four vectors.
+template <int EDIM>
+__device__ inline void group_sum(double (&a)[EDIM][3], int s) {
+    if constexpr (EDIM == 8) {
+#pragma unroll
+        for (int off = 4; off >= 1; off /= 2) {
+            const bool hi = (s & off) != 0;
+#pragma unroll
+            for (int k = 0; k < off; ++k)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const double keep = hi ? a[k + off][i] : a[k][i], send = hi ? a[k][i] : a[k + off][i];
+                    a[k][i] = keep + __shfl_xor(send, off, WAVE);
+                }
+        }
+    }
+}
+
+// writes the element's vectors (hex: lane s its vertex s, so the 24 values are contiguous)
+template <int EDIM>
+__device__ inline void group_write(const double (&a)[EDIM][3], int e, int s, double* __restrict__ elem_out) {
+    constexpr int K = Lanes<EDIM>::N == 1 ? EDIM : 1;
+    double* o = elem_out + ((int64_t)e * EDIM + s) * 3;
+#pragma unroll
+    for (int k = 0; k < K; ++k) { o[3 * k] = a[k][0]; o[3 * k + 1] = a[k][1]; o[3 * k + 2] = a[k][2]; }
+}
+
+// The same with one thread per sample: eight neighbouring lanes share a hex. The SVD is
+// a chain of dependent FP64 operations of about 6 us and the thread per element runs
+// eight of them in a row, which sets the time of every mesh that does not fill the chip:
+// 47 -> 10 us at 256 hexes, 60 -> 13 us at 2,048, 100 -> 91 us at 131,072. Bodies with a
+// frictional boundary keep the thread per element: their iteration amplifies round-off
+// (two orders of these sums end up to 4e-2 apart in the velocities after 12 iterations
+// of a press), and their contact solves outweigh the local step.
+template <int EDIM, class TC>
+__global__ void __launch_bounds__(256) k_local_step_samples(DevMaterials m, const double* __restrict__ q,
+                                                            double* __restrict__ elem_out) {
+    constexpr int S = Lanes<EDIM>::N;
+    const int e = (blockIdx.x * blockDim.x + threadIdx.x) / S, s = threadIdx.x % S;
+    if (e >= m.ne) return;  // whole groups of S lanes leave together
+    double x[EDIM][3];
+#pragma unroll
+    for (int k = 0; k < EDIM; ++k) {
+        const int v = m.elems[k * m.ne + e];
+        x[k][0] = q[3 * v]; x[k][1] = q[3 * v + 1]; x[k][2] = q[3 * v + 2];
+    }
+    const double wc = m.wc ? m.wc[e] : 0.0;
+    const double wv = m.wv ? m.wv[e] : 0.0;
+    const double wm = m.mw ? m.mw[e] : 0.0;
+    double mf[3] = {0.0, 0.0, 0.0}, ma = 0.0;
+    if (wm != 0.0) { mf[0] = m.mfib[e]; mf[1] = m.mfib[m.ne + e]; mf[2] = m.mfib[2 * m.ne + e]; ma = m.mact[e]; }
+    const double* G = m.G + (int64_t)e * m.g_stride + s * EDIM * 3;
+    double F[9], P[9], acc[EDIM][3];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) F[i] = 0.0;
+#pragma unroll
+    for (int k = 0; k < EDIM; ++k)
+#pragma unroll
+        for (int jj = 0; jj < 3; ++jj) {
+            const double g = G[k * 3 + jj];
+            F[0 + 3 * jj] += x[k][0] * g;
+            F[1 + 3 * jj] += x[k][1] * g;
+            F[2 + 3 * jj] += x[k][2] * g;
+        }
+    sample_projection<TC>(m, e, wc, wv, wm, mf, ma, F, P);
+#pragma unroll
+    for (int k = 0; k < EDIM; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) acc[k][i] = P[i] * G[k * 3] + P[i + 3] * G[k * 3 + 1] + P[i + 6] * G[k * 3 + 2];
+    group_sum<EDIM>(acc, s);
+    group_write<EDIM>(acc, e, s, elem_out);
 }
 
 __global__ void k_gather_rhs(int nv, const int* __restrict__ inc_ptr, const int* __restrict__ inc_idx,
@@ -1053,11 +1138,12 @@ template <int EDIM, class TW>
 __global__ void __launch_bounds__(64) k_kpd_build(DevMaterials m, const double* __restrict__ kc, const double* __restrict__ kv,
                                                   KnPtrs kn, const double* __restrict__ q, int filter, double theta,
                                                   double lo, int* __restrict__ nfilt, TW* __restrict__ W) {
-    // one thread per (sample, element), elements fastest: the writes of W
-    // (element-minor: entry j of sample s at (81 s + j) ne + e) are coalesced
+    // one thread per (element, sample), samples fastest: the writes of W
+    // (sample-minor: entry j of sample s at (j ne + e) samples + s) are coalesced,
+    // and so are the reads of k_kpd_apply, whose lanes lie the same way
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= (int64_t)m.ne * m.samples) return;
-    const int e = (int)(gid % m.ne), s = (int)(gid / m.ne);
+    const int e = (int)(gid / m.samples), s = (int)(gid % m.samples);
     const double* G = m.G + (int64_t)e * m.g_stride + s * EDIM * 3;
     double F[9];
 #pragma unroll
@@ -1130,7 +1216,8 @@ __global__ void __launch_bounds__(64) k_kpd_build(DevMaterials m, const double* 
             for (int i = 0; i < 9; ++i) col[i] += w * dP[i];
         }
     };
-    TW* out = W + (int64_t)s * 81 * m.ne + e;
+    TW* out = W + gid;
+    const int64_t total = (int64_t)m.ne * m.samples;
     if (filter != 0) {
         // The proximal maps are isotropic, so in the basis E_kl = u_k v_l^T of
         // the SVD of F the block splits into a 3x3 stretch block (E_00, E_11,
@@ -1244,7 +1331,7 @@ __global__ void __launch_bounds__(64) k_kpd_build(DevMaterials m, const double* 
                             cl[i + 3 * j] = US[i] * V[j] + US[i + 3] * V[j + 3] + US[i + 6] * V[j + 6];
                     muscle_col(c, cl);
 #pragma unroll
-                    for (int i = 0; i < 9; ++i) out[(int64_t)(i + 9 * c) * m.ne] = (TW)cl[i];
+                    for (int i = 0; i < 9; ++i) out[(i + 9 * c) * total] = (TW)cl[i];
                 }
                 return;
             }
@@ -1258,54 +1345,54 @@ __global__ void __launch_bounds__(64) k_kpd_build(DevMaterials m, const double* 
         op(dF, col);
         muscle_col(c, col);
 #pragma unroll
-        for (int i = 0; i < 9; ++i) out[(int64_t)(i + 9 * c) * m.ne] = (TW)col[i];
+        for (int i = 0; i < 9; ++i) out[(i + 9 * c) * total] = (TW)col[i];
     }
 }
 
+// One thread per sample, as in the local step; a thread's 81 entries of W are
+// read coalesced across the lanes (entry j of sample s of element e at
+// (j ne + e) samples + s).
 template <int EDIM, class TW>
 __global__ void __launch_bounds__(128) k_kpd_apply(DevMaterials m, const TW* __restrict__ W, const double* __restrict__ dq,
                                                    double* __restrict__ elem_out) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int S = Lanes<EDIM>::N;
+    const int e = (blockIdx.x * blockDim.x + threadIdx.x) / S, s = threadIdx.x % S;
     if (e >= m.ne) return;
     double x[EDIM][3], acc[EDIM][3];
 #pragma unroll
     for (int k = 0; k < EDIM; ++k) {
         const int v = m.elems[k * m.ne + e];
         x[k][0] = dq[3 * v]; x[k][1] = dq[3 * v + 1]; x[k][2] = dq[3 * v + 2];
-        acc[k][0] = acc[k][1] = acc[k][2] = 0.0;
     }
-    const double* Ge = m.G + (int64_t)e * m.g_stride;
-    for (int s = 0; s < m.samples; ++s) {
-        const double* G = Ge + s * EDIM * 3;
-        double dF[9];
+    const double* G = m.G + (int64_t)e * m.g_stride + s * EDIM * 3;
+    double dF[9];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) dF[i] = 0.0;
+    for (int i = 0; i < 9; ++i) dF[i] = 0.0;
 #pragma unroll
-        for (int k = 0; k < EDIM; ++k)
+    for (int k = 0; k < EDIM; ++k)
 #pragma unroll
-            for (int jj = 0; jj < 3; ++jj) {
-                const double g = G[k * 3 + jj];
-                dF[0 + 3 * jj] += x[k][0] * g;
-                dF[1 + 3 * jj] += x[k][1] * g;
-                dF[2 + 3 * jj] += x[k][2] * g;
-            }
-        const TW* Ws = W + (int64_t)s * 81 * m.ne + e;  // element-minor: coalesced across the wave
-        double y[9];
-#pragma unroll
-        for (int r = 0; r < 9; ++r) {
-            double a = 0;
-#pragma unroll
-            for (int c = 0; c < 9; ++c) a += (double)Ws[(int64_t)(r + 9 * c) * m.ne] * dF[c];
-            y[r] = a;
+        for (int jj = 0; jj < 3; ++jj) {
+            const double g = G[k * 3 + jj];
+            dF[0 + 3 * jj] += x[k][0] * g;
+            dF[1 + 3 * jj] += x[k][1] * g;
+            dF[2 + 3 * jj] += x[k][2] * g;
         }
+    const int64_t total = (int64_t)m.ne * S;
+    const TW* Ws = W + (int64_t)e * S + s;
+    double y[9];
 #pragma unroll
-        for (int k = 0; k < EDIM; ++k)
+    for (int r = 0; r < 9; ++r) {
+        double a = 0;
 #pragma unroll
-            for (int i = 0; i < 3; ++i) acc[k][i] += y[i] * G[k * 3] + y[i + 3] * G[k * 3 + 1] + y[i + 6] * G[k * 3 + 2];
+        for (int c = 0; c < 9; ++c) a += (double)Ws[(r + 9 * c) * total] * dF[c];
+        y[r] = a;
     }
-    double* o = elem_out + (int64_t)e * EDIM * 3;
 #pragma unroll
-    for (int k = 0; k < EDIM; ++k) { o[3 * k] = acc[k][0]; o[3 * k + 1] = acc[k][1]; o[3 * k + 2] = acc[k][2]; }
+    for (int k = 0; k < EDIM; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) acc[k][i] = y[i] * G[k * 3] + y[i + 3] * G[k * 3 + 1] + y[i + 6] * G[k * 3 + 2];
+    group_sum<EDIM>(acc, s);
+    group_write<EDIM>(acc, e, s, elem_out);
 }
 
 // dl/d(mat_w) per merged type (PdEnergyForceDifferential require_dw,
@@ -1652,8 +1739,16 @@ void launch_perm_in(hipStream_t s, int n, const int* perm, const double* r, cons
     template void launch_contact_scatter<TV>(hipStream_t, const ContactPieces&, const int*, const int*, const TV*,          \
                                              const double*, double*, int, TV*);
 
-void launch_local_step(hipStream_t s, const DevMaterials& m, const double* q, double* elem_out, int block, bool fp32) {
+void launch_local_step(hipStream_t s, const DevMaterials& m, const double* q, double* elem_out, int block, bool fp32,
+                       bool samples) {
     if (block != 64 && block != 128 && block != 256) throw std::invalid_argument("local-step block must be 64, 128 or 256");
+    // a tet has one sample: both kernels would do the same
+    if (samples && m.edim == 8) {
+        const dim3 g(blocks_for((int64_t)m.ne * m.samples, block)), b(block);
+        if (fp32) hipLaunchKernelGGL((k_local_step_samples<8, float>), g, b, 0, s, m, q, elem_out);
+        else hipLaunchKernelGGL((k_local_step_samples<8, double>), g, b, 0, s, m, q, elem_out);
+        return;
+    }
     const dim3 g(blocks_for(m.ne, block)), b(block);
     if (m.edim == 8) {
         if (fp32) hipLaunchKernelGGL((k_local_step<8, float>), g, b, 0, s, m, q, elem_out);
@@ -1946,7 +2041,7 @@ void launch_kpd_build(hipStream_t s, const DevMaterials& m, const double* kc, co
 template <class TW>
 void launch_kpd_apply(hipStream_t s, const DevMaterials& m, const TW* W, const double* dq, double* elem_out) {
     if (m.edim == 8)
-        hipLaunchKernelGGL((k_kpd_apply<8, TW>), dim3(blocks_for(m.ne, 128)), dim3(128), 0, s, m, W, dq, elem_out);
+        hipLaunchKernelGGL((k_kpd_apply<8, TW>), dim3(blocks_for((int64_t)m.ne * 8, 128)), dim3(128), 0, s, m, W, dq, elem_out);
     else
         hipLaunchKernelGGL((k_kpd_apply<4, TW>), dim3(blocks_for(m.ne, 128)), dim3(128), 0, s, m, W, dq, elem_out);
 }
@@ -2021,89 +2116,87 @@ template <int EDIM>
 __global__ void __launch_bounds__(128) k_pd_energy_force(DevMaterials m, const double* __restrict__ kc,
                                                          const double* __restrict__ kv, const double* __restrict__ q,
                                                          double* __restrict__ energy, double* __restrict__ elem_out) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int S = Lanes<EDIM>::N;
+    const int e = (blockIdx.x * blockDim.x + threadIdx.x) / S, s = threadIdx.x % S;
     if (e >= m.ne) return;
     double x[EDIM][3], acc[EDIM][3];
 #pragma unroll
     for (int k = 0; k < EDIM; ++k) {
         const int v = m.elems[k * m.ne + e];
         x[k][0] = q[3 * v]; x[k][1] = q[3 * v + 1]; x[k][2] = q[3 * v + 2];
-        acc[k][0] = acc[k][1] = acc[k][2] = 0.0;
     }
     const double wc = kc ? kc[e] : 0.0, wv = kv ? kv[e] : 0.0;
     const double wm = m.mw ? m.mw[e] : 0.0;
     double mf[3] = {0.0, 0.0, 0.0}, ma = 0.0;
     if (wm != 0.0) { mf[0] = m.mfib[e]; mf[1] = m.mfib[m.ne + e]; mf[2] = m.mfib[2 * m.ne + e]; ma = m.mact[e]; }
     double en = 0.0;
-    const double* Ge = m.G + (int64_t)e * m.g_stride;
-    for (int s = 0; s < m.samples; ++s) {
-        const double* G = Ge + s * EDIM * 3;
-        double F[9];
+    const double* G = m.G + (int64_t)e * m.g_stride + s * EDIM * 3;
+    double F[9];
 #pragma unroll
-        for (int i = 0; i < 9; ++i) F[i] = 0.0;
+    for (int i = 0; i < 9; ++i) F[i] = 0.0;
 #pragma unroll
-        for (int k = 0; k < EDIM; ++k)
+    for (int k = 0; k < EDIM; ++k)
 #pragma unroll
-            for (int jj = 0; jj < 3; ++jj) {
-                const double g = G[k * 3 + jj];
-                F[0 + 3 * jj] += x[k][0] * g;
-                F[1 + 3 * jj] += x[k][1] * g;
-                F[2 + 3 * jj] += x[k][2] * g;
-            }
-        double P[9];
-#pragma unroll
-        for (int i = 0; i < 9; ++i) P[i] = 0.0;
-        if (wc != 0.0 || wv != 0.0) {
-            double U[9], sg[3], V[9];
-            svd3(F, U, sg, V);
-            if (wc != 0.0) {
-                const double one[3] = {1.0, 1.0, 1.0};
-                double R[9], n2 = 0.0;
-                udv(U, one, V, R);
-#pragma unroll
-                for (int i = 0; i < 9; ++i) { const double d = F[i] - R[i]; n2 += d * d; P[i] += wc * d; }
-                en += 0.5 * wc * n2;
-            }
-            if (wv != 0.0) {
-                double D[3], sd[3], Pv[9], n2 = 0.0;
-                volume_D(sg, D);
-                sd[0] = sg[0] + D[0]; sd[1] = sg[1] + D[1]; sd[2] = sg[2] + D[2];
-                udv(U, sd, V, Pv);
-#pragma unroll
-                for (int i = 0; i < 9; ++i) { const double d = F[i] - Pv[i]; n2 += d * d; P[i] += wv * d; }
-                en += 0.5 * wv * n2;
-            }
+        for (int jj = 0; jj < 3; ++jj) {
+            const double g = G[k * 3 + jj];
+            F[0 + 3 * jj] += x[k][0] * g;
+            F[1 + 3 * jj] += x[k][1] * g;
+            F[2 + 3 * jj] += x[k][2] * g;
         }
-        if (wm != 0.0) {
-            double Fm[3];
+    double P[9];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) Fm[i] = F[i] * mf[0] + F[i + 3] * mf[1] + F[i + 6] * mf[2];
-            const double l = sqrt(Fm[0] * Fm[0] + Fm[1] * Fm[1] + Fm[2] * Fm[2]);
-            en += 0.5 * wm * (l - ma) * (l - ma);
-            if (l > DBL_EPSILON) {
-                const double r = wm * (1.0 - ma / l);
+    for (int i = 0; i < 9; ++i) P[i] = 0.0;
+    if (wc != 0.0 || wv != 0.0) {
+        double U[9], sg[3], V[9];
+        svd3(F, U, sg, V);
+        if (wc != 0.0) {
+            const double one[3] = {1.0, 1.0, 1.0};
+            double R[9], n2 = 0.0;
+            udv(U, one, V, R);
 #pragma unroll
-                for (int j = 0; j < 3; ++j)
-#pragma unroll
-                    for (int i = 0; i < 3; ++i) P[i + 3 * j] += r * Fm[i] * mf[j];
-            }
+            for (int i = 0; i < 9; ++i) { const double d = F[i] - R[i]; n2 += d * d; P[i] += wc * d; }
+            en += 0.5 * wc * n2;
         }
+        if (wv != 0.0) {
+            double D[3], sd[3], Pv[9], n2 = 0.0;
+            volume_D(sg, D);
+            sd[0] = sg[0] + D[0]; sd[1] = sg[1] + D[1]; sd[2] = sg[2] + D[2];
+            udv(U, sd, V, Pv);
 #pragma unroll
-        for (int k = 0; k < EDIM; ++k)
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                acc[k][i] -= P[i] * G[k * 3] + P[i + 3] * G[k * 3 + 1] + P[i + 6] * G[k * 3 + 2];
+            for (int i = 0; i < 9; ++i) { const double d = F[i] - Pv[i]; n2 += d * d; P[i] += wv * d; }
+            en += 0.5 * wv * n2;
+        }
     }
-    energy[e] = en;
-    double* o = elem_out + (int64_t)e * EDIM * 3;
+    if (wm != 0.0) {
+        double Fm[3];
 #pragma unroll
-    for (int k = 0; k < EDIM; ++k) { o[3 * k] = acc[k][0]; o[3 * k + 1] = acc[k][1]; o[3 * k + 2] = acc[k][2]; }
+        for (int i = 0; i < 3; ++i) Fm[i] = F[i] * mf[0] + F[i + 3] * mf[1] + F[i + 6] * mf[2];
+        const double l = sqrt(Fm[0] * Fm[0] + Fm[1] * Fm[1] + Fm[2] * Fm[2]);
+        en += 0.5 * wm * (l - ma) * (l - ma);
+        if (l > DBL_EPSILON) {
+            const double r = wm * (1.0 - ma / l);
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+#pragma unroll
+                for (int i = 0; i < 3; ++i) P[i + 3 * j] += r * Fm[i] * mf[j];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < EDIM; ++k)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            acc[k][i] = -(P[i] * G[k * 3] + P[i + 3] * G[k * 3 + 1] + P[i + 6] * G[k * 3 + 2]);
+#pragma unroll
+    for (int off = 1; off < S; off *= 2) en += __shfl_xor(en, off, WAVE);
+    if (s == 0) energy[e] = en;
+    group_sum<EDIM>(acc, s);
+    group_write<EDIM>(acc, e, s, elem_out);
 }
 
 void launch_pd_energy_force(hipStream_t s, const DevMaterials& m, const double* kc, const double* kv, const double* q,
                             double* energy, double* elem_out) {
     if (m.edim == 8)
-        hipLaunchKernelGGL(k_pd_energy_force<8>, dim3(blocks_for(m.ne, 128)), dim3(128), 0, s, m, kc, kv, q, energy, elem_out);
+        hipLaunchKernelGGL(k_pd_energy_force<8>, dim3(blocks_for((int64_t)m.ne * 8, 128)), dim3(128), 0, s, m, kc, kv, q, energy, elem_out);
     else
         hipLaunchKernelGGL(k_pd_energy_force<4>, dim3(blocks_for(m.ne, 128)), dim3(128), 0, s, m, kc, kv, q, energy, elem_out);
 }

@@ -1564,7 +1564,7 @@ Body::TuneResult Body::autotune(double dt, int threads, int reps) {
     unit_items_ = kTuneUnits[best];
     best = 0;
     for (int i = 0; i < 3; ++i) {
-        res.local_ms[i] = time_ms([&] { launch_local_step(stream_, mat_, d_q_.p, d_elem_.p, kTuneBlocks[i]); });
+        res.local_ms[i] = time_ms([&] { launch_local_step(stream_, mat_, d_q_.p, d_elem_.p, kTuneBlocks[i], false, K_ == 0); });
         if (res.local_ms[i] < res.local_ms[best]) best = i;
     }
     local_block_ = kTuneBlocks[best];
@@ -1611,7 +1611,7 @@ void Body::contact_scatter(const double* f, DevBuf<TV>& y) {
 }
 
 void Body::local_rhs(const double* q, double inv_h2m) {
-    launch_local_step(stream_, mat_, q, d_elem_.p, local_block_, local_fp32_);
+    launch_local_step(stream_, mat_, q, d_elem_.p, local_block_, local_fp32_, K_ == 0);
     launch_gather_rhs(stream_, nv_, d_inc_ptr_.p, d_inc_idx_.p, d_elem_.p, d_c_dir_.p, d_qtilde_.p, inv_h2m, d_pdrhs_.p, d_b_.p);
 }
 
