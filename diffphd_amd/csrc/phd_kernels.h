@@ -113,22 +113,53 @@ void launch_gather_vertex(hipStream_t s, int nv, const int* inc_ptr, const int* 
 void launch_dots(hipStream_t s, int n, const DotArgs& args, double* partial, double* out);
 int dots_partial_size();
 // out = x + alpha * (y - z) ... generic axpby: out = a*x + b*y (+ c*z)
-// Anderson history push: dQ = x - x_last, dG = g - g_last (skipped when dQ is null),
-// then x_last = x, g_last = g.
-void launch_aa_push(hipStream_t s, int n, const double* x, const double* g, double* x_last, double* g_last, double* dQ,
-                    double* dG);
 void launch_axpbypcz(hipStream_t s, int n, double a, const double* x, double b, const double* y, double c,
                      const double* z, double* out);
-// out = q_prev + g - sum_i gamma_i (dQ_i + dG_i)
-void launch_aa_combine(hipStream_t s, int n, const double* q_prev, const double* g, int m, const double* const* dQ,
-                       const double* const* dG, const double* gamma, double* out);
 void launch_set_dirichlet(hipStream_t s, int nd, const int* ddof, const double* dval, double* q);
 void launch_zero_dirichlet(hipStream_t s, int nd, const int* ddof, double* q);
-// NaN/Inf -> 0 (returned count ignored), scaling done separately
-void launch_nan_to_zero(hipStream_t s, int n, double* x);
 void launch_scale(hipStream_t s, int n, double a, double* x);
-// x *= clip / |x| if |x| = sqrt(norm2[0]) is finite and > clip (norm2 on the device)
-void launch_clip_scale(hipStream_t s, int n, double clip, const double* norm2, double* x);
+
+// ---- one iteration around the global solve (phd_iter.hip) ---------------------
+constexpr int kAAMax = 6;       // Anderson differences combined at once (aa_window <= 6)
+constexpr int kAASlots = 7;     // difference buffers of the pool
+constexpr int kIterRows = 512;  // most block partials per sum
+constexpr int kIterHead = 8;    // doubles before the block sums of launch_iter_combine's output
+constexpr int kIterPartials = (2 * kAAMax + 1) * kIterRows;
+constexpr int kIterOut = kIterHead + 4 * kIterRows;
+int iter_rows(int n);  // block partials of a vector of n entries
+// The Anderson history as the kernels see it: m differences (oldest first, the
+// newest last: dq / dg, also Q[m - 1] / G[m - 1]), their pool slots, the last iterate.
+struct AAHist {
+    int m = 0, push = 0, replay = 0;
+    int slot[kAAMax] = {};
+    const double* Q[kAAMax] = {};
+    const double* G[kAAMax] = {};
+    double *dq = nullptr, *dg = nullptr, *x_last = nullptr, *g_last = nullptr;
+};
+// Right-hand side and residual of one iteration (see k_iter_residual); F and
+// vcand (candidate of a vertex or -1) may be null, pmask as in launch_residual.
+struct IterResidual {
+    int nv = 0, width = 0;
+    const int *inc_ptr = nullptr, *inc_idx = nullptr, *Ai = nullptr, *ipos = nullptr, *vcand = nullptr;
+    const double *elem = nullptr, *c_dir = nullptr, *rhs = nullptr, *Ax = nullptr, *x = nullptr, *F = nullptr;
+    const unsigned char *dmask = nullptr, *pmask = nullptr;
+    double inv_h2m = 0;
+    double *pd_rhs = nullptr, *x_prev = nullptr;
+};
+// fwd: rhs is q~ and pd_rhs, c_dir are used; else b = rhs + the contributions.
+// w[d * ldw + ipos[v]] = the residual (the S product's input), x_prev = x.
+template <class TV>
+void launch_iter_residual(hipStream_t s, const IterResidual& a, bool fwd, TV* w, int ldw);
+// x <- 0 where not finite; part[0 .. iter_rows(n)) = block sums of x.x
+void launch_iter_norm(hipStream_t s, int n, double* x, double* part);
+// norm_part (may be null): x is first scaled to |x| <= clip; part: kIterPartials doubles
+void launch_iter_push(hipStream_t s, int n, const AAHist& h, double* x, const double* x_prev, double clip,
+                      const double* norm_part, double* part);
+// out: kIterOut doubles of pinned host memory; gram_in / gram_out (kAASlots^2
+// doubles each, not the same array): the Gram matrix before and after this step
+void launch_iter_combine(hipStream_t s, int n, bool fwd, const AAHist& h, const double* part, const double* gram_in,
+                         double* gram_out, const double* x_prev, double* x, const unsigned char* fix, const double* fixval,
+                         const double* pd_rhs, double* pd_prev, double* out);
 
 // ---- contact -----------------------------------------------------------------
 // normals / tangents at the frame-start positions (GetLocalFrame)
@@ -160,8 +191,6 @@ void launch_contact_gather(hipStream_t s, const ContactPieces& pc, const int* cp
 template <class TV>
 void launch_contact_scatter(hipStream_t s, const ContactPieces& pc, const int* rc_row, const int* rc_c, const TV* rc_val,
                             const double* f, double* part, int n, TV* y);
-// add f[3c + d] at node c: r[3 node + d] += f
-void launch_add_node_force(hipStream_t s, int K, const int* nodes, const double* f, double* r);
 // M[i][j] = om_i (n_i . n_j) H[i][j] om_j + (i == j) E_i  (row-major, TM = float or double)
 template <class TM>
 void launch_assemble_msys(hipStream_t s, int K, const double* H, const double* nrm, const double* om, const double* E, TM* M);

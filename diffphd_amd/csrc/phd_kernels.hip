@@ -767,36 +767,6 @@ __global__ void k_axpbypcz(int n, double a, const double* __restrict__ x, double
     out[i] = r;
 }
 
-// Anderson history push: with a previous iterate, dQ = x - x_last and dG = g - g_last;
-// then x_last = x and g_last = g (each thread reads its entries before it writes them).
-__global__ void k_aa_push(int n, const double* __restrict__ x, const double* __restrict__ g, double* __restrict__ x_last,
-                          double* __restrict__ g_last, double* __restrict__ dQ, double* __restrict__ dG) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double xi = x[i], gi = g[i];
-    if (dQ) {
-        dQ[i] = xi - x_last[i];
-        dG[i] = gi - g_last[i];
-    }
-    x_last[i] = xi;
-    g_last[i] = gi;
-}
-
-struct AAPtrs {
-    const double* dQ[8];
-    const double* dG[8];
-    double gamma[8];
-};
-
-__global__ void k_aa_combine(int n, const double* __restrict__ q_prev, const double* __restrict__ g, int m, AAPtrs p,
-                             double* __restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double c = q_prev[i] + g[i];
-    for (int a = 0; a < m; ++a) c -= (p.dQ[a][i] + p.dG[a][i]) * p.gamma[a];
-    out[i] = c;
-}
-
 __global__ void k_set_dirichlet(int nd, const int* __restrict__ ddof, const double* __restrict__ dval, double* __restrict__ q) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nd) q[ddof[i]] = dval[i];
@@ -804,18 +774,6 @@ __global__ void k_set_dirichlet(int nd, const int* __restrict__ ddof, const doub
 __global__ void k_zero_dirichlet(int nd, const int* __restrict__ ddof, double* __restrict__ q) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < nd) q[ddof[i]] = 0.0;
-}
-__global__ void k_nan_to_zero(int n, double* __restrict__ x) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !isfinite(x[i])) x[i] = 0.0;
-}
-// x *= clip / |x| when |x| = sqrt(*norm2) is finite and above clip (the norm
-// comes from a device reduction, so no host round trip is needed).
-__global__ void k_clip_scale(int n, double clip, const double* __restrict__ norm2, double* __restrict__ x) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double nn = sqrt(*norm2);
-    if (isfinite(nn) && nn > clip) x[i] *= clip / nn;
 }
 __global__ void k_scale(int n, double a, double* __restrict__ x) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1077,15 +1035,6 @@ __global__ void k_contact_scatter_fin(int nrows, const int* __restrict__ piece_p
     y[k] += (TV)a0;
     y[n + k] += (TV)a1;
     y[2 * n + k] += (TV)a2;
-}
-
-__global__ void k_add_node_force(int K, const int* __restrict__ nodes, const double* __restrict__ f, double* __restrict__ r) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= K) return;
-    const int v = nodes[c];
-    r[3 * v] += f[3 * c];
-    r[3 * v + 1] += f[3 * c + 1];
-    r[3 * v + 2] += f[3 * c + 2];
 }
 
 template <class TM>
@@ -1796,17 +1745,6 @@ void launch_axpbypcz(hipStream_t s, int n, double a, const double* x, double b, 
                      const double* z, double* out) {
     hipLaunchKernelGGL(k_axpbypcz, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a, x, b, y, c, z, out);
 }
-void launch_aa_push(hipStream_t s, int n, const double* x, const double* g, double* x_last, double* g_last, double* dQ,
-                    double* dG) {
-    if (n == 0) return;
-    hipLaunchKernelGGL(k_aa_push, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, x, g, x_last, g_last, dQ, dG);
-}
-void launch_aa_combine(hipStream_t s, int n, const double* q_prev, const double* g, int m, const double* const* dQ,
-                       const double* const* dG, const double* gamma, double* out) {
-    AAPtrs p;
-    for (int a = 0; a < m && a < 8; ++a) { p.dQ[a] = dQ[a]; p.dG[a] = dG[a]; p.gamma[a] = gamma[a]; }
-    hipLaunchKernelGGL(k_aa_combine, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, q_prev, g, m, p, out);
-}
 void launch_set_dirichlet(hipStream_t s, int nd, const int* ddof, const double* dval, double* q) {
     if (nd == 0) return;
     hipLaunchKernelGGL(k_set_dirichlet, dim3(blocks_for(nd, 256)), dim3(256), 0, s, nd, ddof, dval, q);
@@ -1814,12 +1752,6 @@ void launch_set_dirichlet(hipStream_t s, int nd, const int* ddof, const double* 
 void launch_zero_dirichlet(hipStream_t s, int nd, const int* ddof, double* q) {
     if (nd == 0) return;
     hipLaunchKernelGGL(k_zero_dirichlet, dim3(blocks_for(nd, 256)), dim3(256), 0, s, nd, ddof, q);
-}
-void launch_nan_to_zero(hipStream_t s, int n, double* x) {
-    hipLaunchKernelGGL(k_nan_to_zero, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, x);
-}
-void launch_clip_scale(hipStream_t s, int n, double clip, const double* norm2, double* x) {
-    hipLaunchKernelGGL(k_clip_scale, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, clip, norm2, x);
 }
 void launch_scale(hipStream_t s, int n, double a, double* x) {
     hipLaunchKernelGGL(k_scale, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, a, x);
@@ -2008,10 +1940,6 @@ template void launch_assemble_msys_idx<double>(hipStream_t, int, const int*, con
                                                const double*, const double*, double*);
 void launch_copy(hipStream_t s, int64_t n16, const void* a, void* b) {
     hipLaunchKernelGGL(k_copy, dim3((unsigned)((n16 + 1023) / 1024)), dim3(256), 0, s, n16, (const float4*)a, (float4*)b);
-}
-void launch_add_node_force(hipStream_t s, int K, const int* nodes, const double* f, double* r) {
-    if (K == 0) return;
-    hipLaunchKernelGGL(k_add_node_force, dim3(blocks_for(K, 128)), dim3(128), 0, s, K, nodes, f, r);
 }
 template <class TM>
 void launch_assemble_msys(hipStream_t s, int K, const double* H, const double* nrm, const double* om, const double* E, TM* M) {

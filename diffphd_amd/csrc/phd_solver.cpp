@@ -118,7 +118,8 @@ Body::Body(int device) : device_(device) {
     hip_check(hipSetDevice(device_), "hipSetDevice");
     scratch_ = scratch_address(device_);
     hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
-    hip_check(hipHostMalloc((void**)&pin_small_, kPinSmallBytes, hipHostMallocDefault), "hipHostMalloc");
+    hip_check(hipHostMalloc((void**)&pin_small_, kPinSmallBytes + kIterOut * sizeof(double),
+                            hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
     rocblas_handle h;
     check(rocblas_create_handle(&h) == rocblas_status_success, "rocblas_create_handle failed");
     rocblas_set_stream(h, stream_);
@@ -1163,6 +1164,7 @@ void Body::setup(double dt, int threads) {
         hip_check(hipGetLastError(), "expand S launch");
     }
     d_perm_.upload(factor_.perm);
+    d_iperm_.upload(factor_.iperm);
     {  // A in ELL form for the residual kernel (entries in CSR row order, zero padding)
         ell_w_ = 0;
         for (int v = 0; v < nv_; ++v) ell_w_ = std::max(ell_w_, Ap_[v + 1] - Ap_[v]);
@@ -1182,6 +1184,12 @@ void Body::setup(double dt, int threads) {
     d_ddof_.upload(ddof_);
     d_dval_.upload(dval_);
     d_dval_full_.upload(dval_full_);
+    d_fix_.release();
+    if (!ddof_.empty()) {
+        std::vector<unsigned char> fix(dofs_, 0);
+        for (int d : ddof_) fix[d] = 1;
+        d_fix_.upload(fix);
+    }
     // constant Dirichlet part of the local step: sum_e w_e (vol/s) sum_s A_s^T F_bound,s
     c_dir_.assign(dofs_, 0.0);
     if (!dirichlet_.empty()) {
@@ -1249,6 +1257,9 @@ void Body::setup(double dt, int threads) {
     d_elem_.alloc((size_t)ne_ * edim_ * 3);
     d_dot_partial_.alloc(dots_partial_size());
     d_dot_out_.alloc(32);
+    d_iter_part_.alloc(kIterPartials);
+    d_iter_norm_.alloc(kIterRows);
+    for (auto& g : d_aa_gram_) g.alloc(kAASlots * kAASlots);
     w32_.alloc((size_t)3 * spmv_ldw(nv_)); y32_.alloc((size_t)3 * nv_);
     w64_.alloc((size_t)3 * spmv_ldw(nv_)); y64_.alloc((size_t)3 * nv_);
     // k_perm_in writes columns < n only; the padding stays zero from here on
@@ -1274,6 +1285,11 @@ void Body::setup_contact(int threads) {
     if (!boundary_.faces.empty()) d_mesh_faces_.upload(boundary_.faces);
     if (K_ == 0) return;
     d_cand_.upload(cand_);
+    {
+        std::vector<int> vc(nv_, -1);
+        for (int c = 0; c < K_; ++c) vc[cand_[c]] = c;
+        d_vcand_.upload(vc);
+    }
     // paths: contact c in column iperm[v] walks its ancestors
     std::vector<int> cp_ptr(K_ + 1, 0), cp_row, cp_col;
     for (int c = 0; c < K_; ++c) {
@@ -1364,9 +1380,10 @@ void Body::setup_contact(int threads) {
         launch_to_float(stream_, (int64_t)K_ * K_, d_H_.p, d_H32_.p);
         hip_check(hipStreamSynchronize(stream_), "contact H");
     }
+    // the diagonal as one strided copy (a copy per candidate took 3 us each)
     std::vector<double> Hdiag(K_);
-    for (int c = 0; c < K_; ++c)
-        hip_check(hipMemcpy(&Hdiag[c], d_H_.p + (size_t)c * K_ + c, sizeof(double), hipMemcpyDeviceToHost), "H diag");
+    hip_check(hipMemcpy2D(Hdiag.data(), sizeof(double), d_H_.p, ((size_t)K_ + 1) * sizeof(double), sizeof(double), K_,
+                          hipMemcpyDeviceToHost), "H diag");
     Hdiag_ = Hdiag;
     d_Hdiag_.upload(Hdiag);
     for (auto* b : {&d_nrm_, &d_t1_, &d_t2_, &d_F_, &d_dF_, &d_uC_, &d_tmpK3_, &d_qframeC_, &d_Fg_, &d_Fn_, &d_hprev_})
@@ -1581,6 +1598,11 @@ Body::TuneResult Body::autotune(double dt, int threads, int reps) {
 template <class TV>
 void Body::spmv_S(const double* r, DevBuf<TV>& w, DevBuf<TV>& y, DevBuf<TV>& part, const TV* V) {
     launch_perm_in<TV>(stream_, nv_, d_perm_.p, r, nullptr, w.p);
+    spmv_rows(w, y, part, V);
+}
+
+template <class TV>
+void Body::spmv_rows(DevBuf<TV>& w, DevBuf<TV>& y, DevBuf<TV>& part, const TV* V) {
     hipEvent_t a = nullptr, b = nullptr;
     if (timing) { a = next_event(); b = next_event(); (void)hipEventRecord(a, stream_); }
     launch_spmv_rows_grp<TV>(stream_, (int)plan_.gu_group.size(), d_gu_group_.p, d_gu_chunk_.p, d_fd_.p, d_base_.p,
@@ -1627,9 +1649,13 @@ std::vector<double> Body::dots(const std::vector<std::pair<const double*, const 
     return std::vector<double>(pd, pd + a.m);
 }
 
-void Body::kpd_apply(const double* x, double* out, int precision) {
+void Body::kpd_elements(const double* x, int precision) {
     if (precision == 1) launch_kpd_apply<float>(stream_, mat_, d_W32_.p, x, d_elem_.p);
     else launch_kpd_apply<double>(stream_, mat_, d_W64_.p, x, d_elem_.p);
+}
+
+void Body::kpd_apply(const double* x, double* out, int precision) {
+    kpd_elements(x, precision);
     launch_gather_vertex(stream_, nv_, d_inc_ptr_.p, d_inc_idx_.p, d_elem_.p, out);
 }
 
@@ -1894,7 +1920,7 @@ struct DevAnderson {
     bool replay = false;          // the replay's variant: reg 1e-10 max(tr / m, 1), no restart
     std::deque<int> diffs;        // pool indices of the differences, oldest first
     std::vector<int> free_slots;
-    double gram[7][7] = {};       // dG_a . dG_b by pool index, filled as differences arrive
+    int gram_at = 0;              // which of the body's two Gram arrays is current
     void init(int w, int n_, DevBuf<double>* q, DevBuf<double>* g) {
         window = std::min(w, 6);
         n = n_;
@@ -1914,62 +1940,87 @@ struct DevAnderson {
 // One Anderson step (forward_gpu.cpp:1346-1379, backward_gpu.cpp:822-851)
 // on the map x -> x + g at x = xprev: records the newest difference pair
 // (x - x_last, g - g_last), forms the Gram matrix of the g differences from
-// the entries cached as the differences arrived (one new row per call), solves
-// the regularized least squares and writes xprev + g - sum gamma_a (dQ_a + dG_a)
-// into out. `extra` dot pairs ride along in the same reduction. Returns false
-// when nothing was combined: fewer than two iterates, or a restart because
-// |gamma| >= 10 (the history is then dropped, the current iterate included).
-bool Body::anderson_step(DevAnderson& aa, const double* xprev, const double* g, double* out,
-                         const std::vector<std::pair<const double*, const double*>>& extra,
-                         std::vector<double>* extra_out) {
-    const int n3 = aa.n;
-    // the newest difference pair and the new last iterate in one pass
-    double *dq = nullptr, *dg = nullptr;
-    if (aa.have_last) {
-        const int pi = aa.free_slots.back();
-        aa.free_slots.pop_back();
-        dq = aa.Q[pi].p;
-        dg = aa.G[pi].p;
-        aa.diffs.push_back(pi);
+// the entries kept as the differences arrived (one new row per call), solves
+// the regularized least squares and replaces xnew by
+// xprev + g - sum gamma_a (dQ_a + dG_a). The host waits once, for the sums of
+// the convergence test and the restart flag that ride along.
+bool Body::iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew, double clip, double* sums, double* gg) {
+    const int n3 = dofs_;
+    AAHist h;
+    h.push = aa.window > 0 ? 1 : 0;
+    h.replay = aa.replay ? 1 : 0;
+    if (h.push) {
+        if (aa.have_last) {
+            aa.diffs.push_back(aa.free_slots.back());
+            aa.free_slots.pop_back();
+        }
+        h.m = (int)aa.diffs.size();
+        for (int a = 0; a < h.m; ++a) {
+            h.slot[a] = aa.diffs[a];
+            h.Q[a] = aa.Q[aa.diffs[a]].p;
+            h.G[a] = aa.G[aa.diffs[a]].p;
+        }
+        if (h.m > 0) {
+            h.dq = aa.Q[aa.diffs.back()].p;
+            h.dg = aa.G[aa.diffs.back()].p;
+        }
+        h.x_last = aa.Q[7].p;
+        h.g_last = aa.G[7].p;
+        aa.have_last = true;
     }
-    launch_aa_push(stream_, n3, xprev, g, aa.Q[7].p, aa.G[7].p, dq, dg);
-    aa.have_last = true;
-    const int m = (int)aa.diffs.size();
-    std::vector<std::pair<const double*, const double*>> pr;
-    if (m >= 1) {
-        const int nw = aa.diffs.back();
-        for (int a = 0; a < m; ++a) pr.push_back({aa.G[aa.diffs[a]].p, aa.G[nw].p});
-        for (int a = 0; a < m; ++a) pr.push_back({aa.G[aa.diffs[a]].p, g});
+    if (!fwd) launch_iter_norm(stream_, n3, xnew, d_iter_norm_.p);
+    launch_iter_push(stream_, n3, h, xnew, xprev, clip, !fwd && clip > 0 ? d_iter_norm_.p : nullptr, d_iter_part_.p);
+    launch_iter_combine(stream_, n3, fwd, h, d_iter_part_.p, d_aa_gram_[aa.gram_at].p, d_aa_gram_[1 - aa.gram_at].p, xprev,
+                        xnew, d_fix_.p, d_dval_full_.p, d_pdrhs_.p, d_pdrhs_prev_.p, pin_iter());
+    if (h.m > 0) aa.gram_at = 1 - aa.gram_at;
+    hip_check(hipStreamSynchronize(stream_), "iteration");
+    const double* out = pin_iter();
+    const int rows = iter_rows(n3);
+    for (int k = 0; k < (fwd ? 4 : 1); ++k) {
+        sums[k] = 0;
+        for (int r = 0; r < rows; ++r) sums[k] += out[kIterHead + k * kIterRows + r];
     }
-    for (const auto& e : extra) pr.push_back(e);
-    if (pr.empty()) return false;
-    const std::vector<double> dd = dots(pr);
-    if (extra_out) extra_out->assign(dd.begin() + 2 * m, dd.end());
-    if (m == 0) return false;
-    const int nw = aa.diffs.back();
-    for (int a = 0; a < m; ++a) aa.gram[aa.diffs[a]][nw] = aa.gram[nw][aa.diffs[a]] = dd[a];
-    std::vector<double> GtG(m * m), rr(m);
-    double sq = 0;
-    for (int a = 0; a < m; ++a) {
-        for (int b = 0; b < m; ++b) GtG[a * m + b] = aa.gram[aa.diffs[a]][aa.diffs[b]];
-        rr[a] = dd[m + a];
-        sq += GtG[a * m + a];
-    }
-    const double reg = aa.replay ? 1e-10 * std::max(sq / std::max(m, 1), 1.0) : std::max(1e-6 * sq / std::max(m, 1), 1e-12);
-    for (int a = 0; a < m; ++a) GtG[a * m + a] += reg;
-    const std::vector<double> gamma = small_ldlt_solve(GtG, m, rr);
-    if (!aa.replay && nrm2(gamma) >= 10.0) {
+    if (gg) *gg = out[1];
+    if (h.m == 0) return false;
+    if (out[0] == 0.0) {
         aa.clear();
         return false;
     }
-    std::vector<const double*> pq(m), pg(m);
-    for (int a = 0; a < m; ++a) { pq[a] = aa.Q[aa.diffs[a]].p; pg[a] = aa.G[aa.diffs[a]].p; }
-    launch_aa_combine(stream_, n3, xprev, g, m, pq.data(), pg.data(), gamma.data(), out);
     while ((int)aa.diffs.size() > aa.window - 1) {
         aa.free_slots.push_back(aa.diffs.front());
         aa.diffs.pop_front();
     }
     return true;
+}
+
+IterResidual Body::iter_args(const double* rhs, double* x, double* xprev, double inv_h2m, const double* F) {
+    IterResidual a;
+    a.nv = nv_;
+    a.width = ell_w_;
+    a.inc_ptr = d_inc_ptr_.p;
+    a.inc_idx = d_inc_idx_.p;
+    a.Ai = d_Aie_.p;
+    a.Ax = d_Axe_.p;
+    a.vcand = d_vcand_.p;
+    a.elem = d_elem_.p;
+    a.c_dir = d_c_dir_.p;
+    a.rhs = rhs;
+    a.x = x;
+    a.F = F;
+    a.dmask = d_dmask_.p;
+    a.pmask = d_pmask_.p;
+    a.inv_h2m = inv_h2m;
+    a.pd_rhs = d_pdrhs_.p;
+    a.x_prev = xprev;
+    return a;
+}
+
+template <class TV>
+void Body::iter_residual(bool fwd, const double* rhs, double* x, double* xprev, double inv_h2m, const double* F,
+                         DevBuf<TV>& w) {
+    IterResidual a = iter_args(rhs, x, xprev, inv_h2m, F);
+    a.ipos = d_iperm_.p;
+    launch_iter_residual<TV>(stream_, a, fwd, w.p, spmv_ldw(nv_));
 }
 
 // ---------------------------------------------------------------------------
@@ -2093,16 +2144,19 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
     for (int iter = 0; iter < max_pd_iter; ++iter) {
         {
             PhaseTimer tl(this, kFwdLocal);
-            local_rhs(d_q_.p, inv_h2m);
+            launch_local_step(stream_, mat_, d_q_.p, d_elem_.p, local_block_, local_fp32_, K_ == 0);
         }
-        hip_check(hipMemcpyAsync(d_qprev_.p, d_q_.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "q_prev");
-        // residual of the global system with the previous contact impulses
+        // residual of the global system with the previous contact impulses; q_prev = q
         {
             PhaseTimer ts(this, kFwdSolve);
-            launch_residual(stream_, nv_, ell_w_, d_Aie_.p, d_Axe_.p, d_b_.p, d_q_.p, d_dmask_.p, d_r_.p, d_pmask_.p);
-            if (K > 0) launch_add_node_force(stream_, K, d_cand_.p, d_F_.p, d_r_.p);
-            if (precision == 1) spmv_S<float>(d_r_.p, w32_, y32_, part32_, V32_.p);
-            else spmv_S<double>(d_r_.p, w64_, y64_, part64_, V64_.p);
+            const double* F = K > 0 ? d_F_.p : nullptr;
+            if (precision == 1) {
+                iter_residual<float>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w32_);
+                spmv_rows<float>(w32_, y32_, part32_, V32_.p);
+            } else {
+                iter_residual<double>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w64_);
+                spmv_rows<double>(w64_, y64_, part64_, V64_.p);
+            }
         }
         if (K > 0) {
             PhaseTimer tc(this, kFwdContact);
@@ -2195,20 +2249,13 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
             partial_dirichlet(d_q_.p, d_qprev_.p, d_dval_full_.p);
         }
         ++iters;
-        // Anderson acceleration
-        if (aa_window > 0) {
+        // Anderson acceleration and the sums of the dual gate (:1382-1397)
+        double gd[4];
+        {
             PhaseTimer ta(this, kFwdAA);
-            launch_axpbypcz(stream_, n3, 1.0, d_q_.p, -1.0, d_qprev_.p, 0.0, nullptr, d_g_.p);
-            if (anderson_step(aa, d_qprev_.p, d_g_.p, d_q_.p, {}, nullptr))
-                launch_set_dirichlet(stream_, (int)ddof_.size(), d_ddof_.p, d_dval_.p, d_q_.p);
+            iterate(aa, true, d_qprev_.p, d_q_.p, 0.0, gd, nullptr);
         }
-        // dual gate (:1382-1397)
         PhaseTimer tg(this, kFwdGate);
-        launch_axpbypcz(stream_, n3, 1.0, d_q_.p, -1.0, d_qprev_.p, 0.0, nullptr, d_g_.p);
-        launch_axpbypcz(stream_, n3, 1.0, d_pdrhs_.p, -1.0, d_pdrhs_prev_.p, 0.0, nullptr, d_tmp_.p);
-        const std::vector<double> gd = dots({{d_g_.p, d_g_.p}, {d_qprev_.p, d_qprev_.p}, {d_tmp_.p, d_tmp_.p},
-                                             {d_pdrhs_prev_.p, d_pdrhs_prev_.p}});
-        hip_check(hipMemcpyAsync(d_pdrhs_prev_.p, d_pdrhs_.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "prev");
         const double abs_err = std::sqrt(gd[0]), rhs_norm = std::sqrt(gd[1]), rc = std::sqrt(gd[2]), rr = std::sqrt(gd[3]);
         if (verbose > 0) printf("alg_phd PD iter %d  dq=%g  dpd_rhs=%g\n", iter, abs_err, rc);
         if (iter > 0 && abs_err <= rel_tol * rhs_norm + abs_tol && rc <= rel_tol * rr + abs_tol) { converged = true; break; }
@@ -2412,17 +2459,6 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
     d_zero.alloc(n3);
     hip_check(hipMemsetAsync(d_zero.p, 0, sizeof(double) * n3, stream_), "zero");
 
-    // safe_clip (backward_gpu.cpp:809-816) on a device vector
-    auto safe_clip = [&](double* x) {
-        launch_nan_to_zero(stream_, n3, x);
-        if (clip > 0) {  // |x| reduced and applied on the device: no host round trip
-            DotArgs a;
-            a.m = 1;
-            a.a[0] = a.b[0] = x;
-            launch_dots(stream_, n3, a, d_dot_partial_.p, d_dot_out_.p);
-            launch_clip_scale(stream_, n3, clip, d_dot_out_.p, x);
-        }
-    };
     // Constrained solve data (Woodbury basis); nb == 0 means the plain backbone.
     int nb = 0;
     DevBuf<double> d_G, d_Gx, d_dirs, d_Gs64;
@@ -2444,12 +2480,15 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
         aa.init(aa_window, n3, d_hist_q_, d_hist_g_);
         int it_used = 0;
         for (int i = 0; i < max_it; ++i) {
-            hip_check(hipMemcpyAsync(d_sprev.p, d_s.p, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "sprev");
-            kpd_apply(d_s.p, d_kz_.p, precision);
-            launch_axpbypcz(stream_, n3, 1.0, d_rhs.p, 1.0, d_kz_.p, 0.0, nullptr, d_tmp_.p);
-            launch_residual(stream_, nv_, ell_w_, d_Aie_.p, d_Axe_.p, d_tmp_.p, d_s.p, d_dmask_.p, d_r_.p, d_pmask_.p);
-            if (precision == 1) spmv_S<float>(d_r_.p, w32_, y32_, part32_, V32_.p);
-            else spmv_S<double>(d_r_.p, w64_, y64_, part64_, V64_.p);
+            // s_prev = s; r = rhs + K s - A s
+            kpd_elements(d_s.p, precision);
+            if (precision == 1) {
+                iter_residual<float>(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, w32_);
+                spmv_rows<float>(w32_, y32_, part32_, V32_.p);
+            } else {
+                iter_residual<double>(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, w64_);
+                spmv_rows<double>(w64_, y64_, part64_, V64_.p);
+            }
             if (nb > 0) {
                 // s <- s + A^-1 r - A^-1 J^T G^-1 J (A^-1 r + s) on the device: project the
                 // candidate vectors on the basis, apply G^-1 (formed once per frame, FP32
@@ -2468,18 +2507,17 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
             if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_sprev.p, d_zero.p, d_s.p);
             else spmv_ST<double>(y64_, xpart64_, V64_.p, d_sprev.p, d_zero.p, d_s.p);
             partial_dirichlet(d_s.p, d_sprev.p, nullptr);
-            safe_clip(d_s.p);
-            launch_axpbypcz(stream_, n3, 1.0, d_s.p, -1.0, d_sprev.p, 0.0, nullptr, d_g_.p);
-            double err;
-            if (aa_window > 0) {
-                std::vector<double> e2;
-                if (anderson_step(aa, d_sprev.p, d_g_.p, d_s.p, {{d_g_.p, d_g_.p}}, &e2)) safe_clip(d_s.p);
-                err = std::sqrt(e2[0]);
-            } else {
-                err = std::sqrt(dots({{d_g_.p, d_g_.p}})[0]);
+            // safe_clip (backward_gpu.cpp:809-816) before and after the Anderson
+            // step: non-finite entries to 0, then |s| <= clip
+            double ss, gg;
+            const bool combined = iterate(aa, false, d_sprev.p, d_s.p, clip, &ss, &gg);
+            const double err = std::sqrt(gg);
+            double sn = std::sqrt(ss);
+            if (combined && clip > 0 && std::isfinite(sn) && sn > clip) {
+                launch_scale(stream_, n3, clip / sn, d_s.p);
+                sn = clip;
             }
             it_used = i + 1;
-            const double sn = std::sqrt(dots({{d_s.p, d_s.p}})[0]);
             if (i > 0 && err < rel_tol * sn + abs_tol) { *conv = true; break; }
             if (div) {
                 err_min = std::min(err_min, err);

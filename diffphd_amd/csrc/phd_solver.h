@@ -308,6 +308,8 @@ private:
     // Pinned host memory for the few scalars read back per iteration (the
     // contact set sizes, the dense solve's pivot flag, the dot products).
     static constexpr size_t kPinSmallBytes = 4096;
+    // followed by the sums that launch_iter_combine writes there
+    double* pin_iter() { return reinterpret_cast<double*>(static_cast<char*>(pin_small_) + kPinSmallBytes); }
     void* pin_small_ = nullptr;
     // scene
     int edim_ = 8, nv_ = 0, ne_ = 0, dofs_ = 0, samples_ = 8;
@@ -424,6 +426,9 @@ private:
     void warm_start(const double* v, double dt, double inv_h2m, bool learned);
     DevBuf<double> d_hist_q_[8], d_hist_g_[8];
     DevBuf<double> d_dot_partial_, d_dot_out_;
+    DevBuf<double> d_iter_part_, d_iter_norm_, d_aa_gram_[2];
+    DevBuf<int> d_iperm_, d_vcand_;
+    DevBuf<unsigned char> d_fix_;  // Dirichlet DOFs (empty without any)
     DevBuf<float> w32_, y32_, part32_, xpart32_;
     DevBuf<double> w64_, y64_, part64_, xpart64_;
     // contact
@@ -483,9 +488,21 @@ private:
     void contact_scatter(const double* f, DevBuf<TV>& y);
     void local_rhs(const double* q, double inv_h2m);
     void kpd_apply(const double* x, double* out, int precision);
+    void kpd_elements(const double* x, int precision);  // its per-element part, into d_elem_
     std::vector<double> dots(const std::vector<std::pair<const double*, const double*>>& pairs);
-    bool anderson_step(DevAnderson& aa, const double* xprev, const double* g, double* out,
-                       const std::vector<std::pair<const double*, const double*>>& extra, std::vector<double>* extra_out);
+    // The Anderson step on x -> x + g with x = xprev, xnew = x + g, in place on
+    // xnew, and the iteration's sums: fwd sums[4] = |x' - x|^2, |x|^2, |dpd|^2,
+    // |pd_prev|^2 (x' the combined iterate), else sums[0] = x'.x'; gg = g.g.
+    // clip > 0 (adjoint): xnew is scaled to that norm first. Returns whether x'
+    // was combined: not with fewer than two iterates, nor after a restart
+    // (|gamma| >= 10), which drops the history, the current iterate included.
+    bool iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew, double clip, double* sums, double* gg);
+    // r = b - A x of one iteration into w (see IterResidual)
+    IterResidual iter_args(const double* rhs, double* x, double* xprev, double inv_h2m, const double* F);
+    template <class TV>
+    void iter_residual(bool fwd, const double* rhs, double* x, double* xprev, double inv_h2m, const double* F, DevBuf<TV>& w);
+    template <class TV>
+    void spmv_rows(DevBuf<TV>& w, DevBuf<TV>& y, DevBuf<TV>& part, const TV* V);
     bool solve_contact_system(int n, int precision, const int* J, bool plain_w = false);
     void forward_impl(const double* q, const double* v, const double* f_ext, double dt,
                       const std::map<std::string, double>& opt, double* q_next, double* v_next, std::vector<int>& active,
