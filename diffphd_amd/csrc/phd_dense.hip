@@ -60,87 +60,9 @@ template <class TV> struct V16;
 template <> struct V16<float> { using type = float4; static constexpr int N = 4; };
 template <> struct V16<double> { using type = double2; static constexpr int N = 2; };
 
-constexpr int kColStride = 2 * CB + 4;  // one published pivot column, see k_chol_step
 constexpr int kTSB = CB + 4;             // row stride of the published L columns (16-byte aligned rows)
 
-// Pivot of step j from the window's column j (wave 0): publishes the column
-// into buffer j & 1, L(r, j) at CB + r - j for r > j so that L(j + m, j) sits
-// at CB + m for every j, and 1 / L(j, j) at CB (the slot of the diagonal,
-// which no update reads). Returns L(r, j) for r > j, 1 / L(j, j) on lane j and
-// zero above it (lanes r <= j only ever touch their own upper triangle).
-template <class TV>
-__device__ __forceinline__ TV panel_pivot(int j, TV zj, TV* colS, int r, bool& bad_any) {
-    TV* cb = colS + (j & 1) * kColStride;
-    const TV p = lane_bcast(zj, j);
-    const bool bad = !(p > TV(0));
-    bad_any |= bad;
-    const TV inv = bad ? TV(1) : pivot_rsqrt(p);
-    const TV coef = (r > j) ? zj * inv : (r == j ? inv : TV(0));
-    cb[CB + r - j] = coef;
-    if (r == CB - 1) {  // the two slots past the column, stale from step j - 2
-        cb[2 * CB - j] = TV(0);
-        cb[2 * CB + 1 - j] = TV(0);
-    }
-    return coef;
-}
-
-template <class TV>
-__device__ __forceinline__ void read16(const TV* src, TV (&c)[16]) {
-    using VT = typename V16<TV>::type;
-    constexpr int VN = V16<TV>::N;
-#pragma unroll
-    for (int e = 0; e < 16 / VN; ++e) {
-        const VT t = reinterpret_cast<const VT*>(src)[e];
-        memcpy(c + VN * e, &t, sizeof(VT));
-    }
-}
-
-// Steps [j, j + 16) of the panel chain. Window z[m] = column j + m of the
-// lane's row; columns past 63 never matter, and from step j on only
-// m <= 63 - j can reach one, so this quarter of the steps stops at m = MB.
-// Role 0 (the diagonal wave) takes L(j + 1, j) from lane j + 1 by readlane,
-// updates its column j + 1 and publishes the pivot of step j + 1 before the
-// rest of step j's update, so the pivot chain never waits on LDS. Role 1
-// solves its block row against the published columns; role 2 only keeps the
-// barriers. The published column is read in chunks of 16, each chunk's reads
-// issued before the previous chunk's update so the LDS latency overlaps the
-// FMAs.
-template <class TV, int MB>
-__device__ __forceinline__ void panel_quarter(int& j, TV (&z)[CB], TV* colS, int role, int r, bool& bad_any, TV& coef,
-                                              TV* out, int64_t out_ld) {
-    constexpr int NQ = (MB + 1) / 16;
-    for (int jj = 0; jj < 16; ++jj, ++j) {
-        __syncthreads();
-        if (role == 2) continue;
-        const bool diag_wave = role == 0;
-        const TV* cb = colS + (j & 1) * kColStride + CB;
-        TV c[2][16];
-        read16<TV>(cb, c[0]);
-        if (NQ > 1) read16<TV>(cb + 16, c[1]);
-        const bool chain = diag_wave && (j + 1 < CB);
-        TV z0 = TV(0), coef_next = TV(0);
-        if (chain) {
-            z0 = z[1] - coef * lane_bcast(coef, j + 1);
-            coef_next = panel_pivot<TV>(j + 1, z0, colS, r, bad_any);
-        }
-        if (!diag_wave) {
-            coef = z[0] * c[0][0];
-            out[r + (int64_t)j * out_ld] = coef;
-        }
-        z[0] = chain ? z0 : z[1] - coef * c[0][1];
-#pragma unroll
-        for (int m = 2; m < 16; ++m) z[m - 1] = z[m] - coef * c[0][m];
-#pragma unroll
-        for (int q = 1; q < NQ; ++q) {
-            if (q + 1 < NQ) read16<TV>(cb + 16 * (q + 1), c[(q + 1) & 1]);
-#pragma unroll
-            for (int e = 0; e < 16; ++e) z[16 * q + e - 1] = z[16 * q + e] - coef * c[q & 1][e];
-        }
-        if (diag_wave) coef = coef_next;
-    }
-}
-
-// ---- The panel in 16-column sub-blocks ------------------------------------
+// ---- The FP32 panel in 16-column sub-blocks --------------------------------
 // The diagonal wave (lane r holds row r of the diagonal block in z) factors
 // sub-block SB's 16 columns with readlane pivots and rank-1 updates restricted
 // to those columns, so a step waits on register broadcasts only; L(r, j)
@@ -173,28 +95,6 @@ __device__ __forceinline__ void diag_publish(const TV (&z)[CB], int r, TV inv_mi
 
 __device__ __forceinline__ float vget(const float4& t, int e) { return e == 0 ? t.x : e == 1 ? t.y : e == 2 ? t.z : t.w; }
 __device__ __forceinline__ double vget(const double2& t, int e) { return e == 0 ? t.x : t.y; }
-
-// Rank-16 update of the columns right of sub-block SB: z[m] -= sum_j z[j] L(m, j)
-// over the sub-block's j (z[j] = L(r, j) in the diagonal wave, X(r, j) in the
-// block-row wave); L(m, j) read as broadcast 16-byte vectors. FP64 only: the
-// FP32 panel runs these updates on the matrix cores (diag_trail_mfma,
-// row_trail_mfma), which keeps LDS latency off the panel's critical path.
-template <class TV, int SB>
-__device__ __forceinline__ void panel_trail(TV (&z)[CB], const TV (*Lt)[kTSB]) {
-    using VT = typename V16<TV>::type;
-    constexpr int VN = V16<TV>::N;
-    constexpr int M0 = 16 * (SB + 1);
-#pragma unroll
-    for (int jj = 0; jj < 16; ++jj) {
-        const TV x = z[16 * SB + jj];
-#pragma unroll
-        for (int m = M0; m < CB; m += VN) {
-            const VT t = *reinterpret_cast<const VT*>(&Lt[16 * SB + jj][m]);
-#pragma unroll
-            for (int e = 0; e < VN; ++e) z[m + e] -= x * vget(t, e);
-        }
-    }
-}
 
 // The block-row wave's forward substitution on sub-block SB: X(r, j) =
 // (B(r, j) - sum_{i<j} X(r, i) L(j, i)) / L(j, j), right-looking within the
@@ -250,20 +150,24 @@ __device__ __forceinline__ void stage_block(const TV* __restrict__ M, int64_t ld
     }
 }
 
-// acc[p] = sum_l A[l][tx] B[l][16 ty + p]: thread (tx, ty) of 256 owns row tx
-// and columns 16 ty .. 16 ty + 15 of a rank-64 product tile (a wave holds one
-// column group, so B is read as broadcast 16-byte vectors).
-template <class TV>
-__device__ __forceinline__ void tile_product(const TV (*A)[kTS], const TV (*B)[kTS], int tx, int ty, TV (&acc)[16]) {
+// FP64 rank-64 tile product: acc[u][v] = sum_l A[l][4 tx + u] B[l][4 ty + v], l
+// ascending; thread (tx, ty) of 16 x 16. Four by four outputs per thread take four
+// 16-byte LDS reads for 16 FMAs (a row of 16 columns per thread took nine).
+__device__ __forceinline__ void tile_product(const double (*A)[kTS], const double (*B)[kTS], int tx, int ty,
+                                             double (&acc)[4][4]) {
 #pragma unroll
-    for (int p = 0; p < 16; ++p) acc[p] = 0;
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[u][v] = 0;
 #pragma unroll 4
     for (int l = 0; l < CB; ++l) {
-        const TV a = A[l][tx];
-        TV b[16];
-        read16<TV>(&B[l][16 * ty], b);
+        double a[4], b[4];
+        memcpy(a, &A[l][4 * tx], sizeof(a));
+        memcpy(b, &B[l][4 * ty], sizeof(b));
 #pragma unroll
-        for (int p = 0; p < 16; ++p) acc[p] += a * b[p];
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[u][v] += a[u] * b[v];
     }
 }
 
@@ -389,24 +293,12 @@ __device__ __forceinline__ void row_trail_mfma(float (&z)[CB], const float (*Lt)
     }
 }
 
-// The FP32 panel's trailing updates on the matrix cores, FP64's on the VALU.
-template <class TV, int SB>
-__device__ __forceinline__ void diag_trail(TV (&z)[CB], const TV (*Lt)[kTSB]) {
-    if constexpr (std::is_same<TV, float>::value) diag_trail_mfma<SB>(z);
-    else panel_trail<TV, SB>(z, Lt);
-}
-template <class TV, int SB>
-__device__ __forceinline__ void row_trail(TV (&z)[CB], const TV (*Lt)[kTSB], int lane) {
-    if constexpr (std::is_same<TV, float>::value) row_trail_mfma<SB>(z, Lt, lane);
-    else panel_trail<TV, SB>(z, Lt);
-}
-
 // Rank-64 update of step kp on block (ib, jb): A_ij -= L_{i,kp} L_{j,kp}^T
 // (256 threads; the staging tiles are S0 and S1).
 template <class TV>
 __device__ __forceinline__ void update_block(TV* __restrict__ M, int64_t lda, int kp, int ib, int jb, TV (*S0)[kTS],
                                              TV (*S1)[kTS]) {
-    const int t = threadIdx.x, tx = t % 64, ty = t / 64;
+    const int t = threadIdx.x;
     if constexpr (std::is_same<TV, float>::value) {
         // the target block is read together with the staging loads, so its
         // latency overlaps theirs instead of following the product
@@ -422,15 +314,107 @@ __device__ __forceinline__ void update_block(TV* __restrict__ M, int64_t lda, in
 #pragma unroll
         for (int v = 0; v < 16; ++v) dst[mfma_col(v, lane) * lda] = old[v] - acc[v];
     } else {
+        const int tx = t % 16, ty = t / 16;
+        TV* dst = M + (int64_t)ib * CB + 4 * tx + ((int64_t)jb * CB + 4 * ty) * lda;
+        TV old[4][4], acc[4][4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) old[u][v] = dst[u + v * lda];
         stage_block<TV>(M, lda, (int64_t)ib * CB, (int64_t)kp * CB, S0);
         stage_block<TV>(M, lda, (int64_t)jb * CB, (int64_t)kp * CB, S1);
         __syncthreads();
-        TV acc[16];
-        tile_product<TV>(S0, S1, tx, ty, acc);
-        TV* dst = M + (int64_t)ib * CB + tx + ((int64_t)jb * CB + 16 * ty) * lda;
+        tile_product(S0, S1, tx, ty, acc);
 #pragma unroll
-        for (int p = 0; p < 16; ++p) dst[p * lda] -= acc[p];
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) dst[u + v * lda] = old[u][v] - acc[u][v];
     }
+}
+
+// The FP64 panel in LDS: D the diagonal block, R the block row (or the identity), both
+// [row][column]. Stage s: wave 0 factors the 16 columns of sub-block s in registers
+// (readlane broadcasts), wave 1 solves the block row against sub-block s - 1; then all
+// four waves apply both rank-16 updates to the columns on the right, 4 x 4 entries per
+// thread, j ascending (each entry sees the operations of one rank-1 update per column
+// in column order). A row of the block in registers (64 doubles) would leave two waves
+// idle and spills; one pivot per barrier took 38 us a step, this takes 17 us.
+constexpr int kLS = 18;  // row stride of a published 16 x 16 diagonal sub-block
+
+__device__ __forceinline__ void panel64(double (*D)[kTS], double (*R)[kTS], double (*Ls)[16][kLS], double* invp, int w,
+                                        double* out, int64_t out_ld, int* __restrict__ fail) {
+    const int t = threadIdx.x, wave = t / 64, r = t % 64;
+    bool bad_any = false;
+#pragma unroll 1
+    for (int s = 0; s <= 4; ++s) {
+        const int q = s - 1;
+        if (wave == 0 && s < 4) {
+            double z[16], inv = 1.0;
+            memcpy(z, &D[r][16 * s], sizeof(z));
+#pragma unroll
+            for (int jj = 0; jj < 16; ++jj) {
+                const int j = 16 * s + jj;
+                const double p = lane_bcast(z[jj], j);
+                const bool bad = !(p > 0.0);
+                bad_any |= bad;
+                const double iv = bad ? 1.0 : pivot_rsqrt(p);
+                if (r == j) inv = iv;
+                const double l = (r > j) ? z[jj] * iv : (r == j ? p * iv : 0.0);
+                z[jj] = l;
+#pragma unroll
+                for (int m = jj + 1; m < 16; ++m) z[m] -= l * lane_bcast(l, 16 * s + m);
+            }
+            memcpy(&D[r][16 * s], z, sizeof(z));
+            if (r / 16 == s) {
+                invp[r] = inv;
+#pragma unroll
+                for (int jj = 0; jj < 16; ++jj) Ls[s & 1][jj][r % 16] = z[jj];
+            }
+        } else if (wave == 1 && s > 0) {
+            double z[16];
+            memcpy(z, &R[r][16 * q], sizeof(z));
+#pragma unroll
+            for (int jj = 0; jj < 16; ++jj) {
+                const double x = z[jj] * invp[16 * q + jj];
+                z[jj] = x;
+                out[r + (int64_t)(16 * q + jj) * out_ld] = x;
+#pragma unroll
+                for (int m = jj + 1; m < 16; ++m) z[m] -= x * Ls[q & 1][jj][m];
+            }
+            memcpy(&R[r][16 * q], z, sizeof(z));
+        }
+        if (s == 4) break;
+        __syncthreads();
+        const int cd = 4 * (3 - s), cr = s > 0 ? 4 * (4 - s) : 0;  // column groups right of s / of q
+        for (int tile = t; tile < 16 * (cd + cr); tile += 256) {
+            const int tx = tile % 16, g = tile / 16;
+            const bool diag = g < cd;
+            double (*A)[kTS] = diag ? D : R;
+            const int j0 = diag ? 16 * s : 16 * q, c0 = 16 * s + (diag ? 16 + 4 * g : 4 * (g - cd));
+            double acc[4][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) memcpy(acc[u], &A[tx + 16 * u][c0], sizeof(acc[u]));
+#pragma unroll 4
+            for (int j = 0; j < 16; j += 2) {
+                double a[4][2], b[4][2];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    memcpy(a[u], &A[tx + 16 * u][j0 + j], sizeof(a[u]));
+                    memcpy(b[u], &D[c0 + u][j0 + j], sizeof(b[u]));
+                }
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) acc[u][v] -= a[u][e] * b[v][e];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) memcpy(&A[tx + 16 * u][c0], acc[u], sizeof(acc[u]));
+        }
+        __syncthreads();
+    }
+    if (wave == 0 && bad_any && w == 0 && r == 0) fail[0] = 1;
 }
 
 // Step k of the factorization, one launch of 256-thread workgroups in two parts
@@ -442,23 +426,25 @@ __device__ __forceinline__ void update_block(TV* __restrict__ M, int64_t lda, in
 //    (k + 1 + w, k); w = T - k - 1 is the right-hand-side block row and
 //    w = T - k the identity. Then wave 0 factors the diagonal block and
 //    wave 1 solves X L_kk^T = B, writing L(k + 1 + w, k) into M, or
-//    Xinv_k = L_kk^-T (column-major 64 x 64) for the identity. FP32 works in
+//    Xinv_k = L_kk^-T (column-major 64 x 64) for the identity. Both work in
 //    16-column sub-blocks: wave 0 runs each sub-block's pivot chain on
 //    readlane broadcasts and publishes its columns through LDS, wave 1
-//    solves against them one sub-block behind, and both apply the rank-16
-//    update of the columns to the right as MFMA tiles. FP64 publishes one
-//    pivot column per barrier (two alternating LDS buffers);
+//    solves against them one sub-block behind, and the rank-16 update of the
+//    columns to the right follows (FP32 as MFMA tiles of the same two waves,
+//    FP64 see panel64);
 //  * the remaining workgroups apply the update of step k - 1 to the blocks
 //    (i, j) with k < j <= i <= T.
-// Four workgroups per CU (the FP32 MFMA accumulators stay in VGPRs, so the
-// update workgroups of a step run at four waves per SIMD).
+// Four workgroups per CU in FP32 (the MFMA accumulators stay in VGPRs, so the
+// update workgroups of a step run at four waves per SIMD), two in FP64, whose staging
+// tiles allow no more.
 template <class TV>
-__global__ void __launch_bounds__(256, 4) k_chol_step(int k, int T, int64_t lda, TV* __restrict__ M,
+__global__ void __launch_bounds__(256, sizeof(TV) == 8 ? 2 : 4) k_chol_step(int k, int T, int64_t lda, TV* __restrict__ M,
                                                    TV* __restrict__ Xinv, int* __restrict__ fail) {
     __shared__ __align__(16) TV S0[CB][kTS];
     __shared__ __align__(16) TV S1[CB][kTS];
-    __shared__ __align__(16) TV colS[2 * kColStride];
-    const int t = threadIdx.x, tx = t % 64, ty = t / 64;
+    __shared__ __align__(16) TV invp[CB];
+    __shared__ __align__(16) TV Ls[sizeof(TV) == 8 ? 2 : 1][16][kLS];  // FP64 only
+    const int t = threadIdx.x;
     const int NP = T - k + 1;
     const int kp = k - 1;
     if ((int)blockIdx.x >= NP) {
@@ -472,6 +458,42 @@ __global__ void __launch_bounds__(256, 4) k_chol_step(int k, int T, int64_t lda,
     const int role = wave < 2 ? wave : 2;
     const bool has_row = w < T - k;          // block row k + 1 + w of M (else the identity)
     const int64_t c0 = (int64_t)k * CB, i0 = (int64_t)(k + 1 + w) * CB;
+    if constexpr (std::is_same<TV, double>::value) {
+        const int ux = t % 16, uy = t / 16;
+        TV aD[4][4], aR[4][4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int64_t off = 4 * ux + u + (c0 + 4 * uy + v) * lda;
+                aD[u][v] = M[c0 + off];
+                aR[u][v] = has_row ? M[i0 + off] : (u + 4 * ux == v + 4 * uy ? TV(1) : TV(0));
+            }
+        if (k > 0) {
+            TV accD[4][4], accR[4][4];
+            stage_block<TV>(M, lda, c0, (int64_t)kp * CB, S0);
+            if (has_row) stage_block<TV>(M, lda, i0, (int64_t)kp * CB, S1);
+            __syncthreads();
+            tile_product(S0, S0, ux, uy, accD);
+            if (has_row) tile_product(S1, S0, ux, uy, accR);
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    aD[u][v] -= accD[u][v];
+                    if (has_row) aR[u][v] -= accR[u][v];
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            memcpy(&S0[4 * ux + u][4 * uy], aD[u], sizeof(aD[u]));
+            memcpy(&S1[4 * ux + u][4 * uy], aR[u], sizeof(aR[u]));
+        }
+        __syncthreads();
+        panel64(S0, S1, Ls, invp, w, has_row ? M + i0 + c0 * lda : Xinv + (int64_t)k * CB * CB, has_row ? lda : CB, fail);
+        return;
+    } else {
     TV z[CB];
     using VT = typename V16<TV>::type;
     constexpr int VN = V16<TV>::N;
@@ -479,45 +501,24 @@ __global__ void __launch_bounds__(256, 4) k_chol_step(int k, int T, int64_t lda,
         // FP32: the two target blocks are read together with the staging loads
         const int row = 32 * (wave >> 1) + (r & 31);
         float aD[16], aR[16];
-        if constexpr (std::is_same<TV, float>::value) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int64_t off = row + (c0 + 32 * (wave & 1) + mfma_col(v, r)) * lda;
-                aD[v] = M[c0 + off];
-                aR[v] = has_row ? M[i0 + off] : 0.f;
-            }
+        for (int v = 0; v < 16; ++v) {
+            const int64_t off = row + (c0 + 32 * (wave & 1) + mfma_col(v, r)) * lda;
+            aD[v] = M[c0 + off];
+            aR[v] = has_row ? M[i0 + off] : 0.f;
         }
         stage_block<TV>(M, lda, c0, (int64_t)kp * CB, S0);
         if (has_row) stage_block<TV>(M, lda, i0, (int64_t)kp * CB, S1);
         __syncthreads();
-        if constexpr (std::is_same<TV, float>::value) {
-            const f32x16 accD = tile_product_mfma(S0, S0, wave, r);
-            f32x16 accR;
-            if (has_row) accR = tile_product_mfma(S1, S0, wave, r);
-            __syncthreads();
+        const f32x16 accD = tile_product_mfma(S0, S0, wave, r);
+        f32x16 accR;
+        if (has_row) accR = tile_product_mfma(S1, S0, wave, r);
+        __syncthreads();
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int col = 32 * (wave & 1) + mfma_col(v, r);
-                S0[row][col] = aD[v] - accD[v];
-                if (has_row) S1[row][col] = aR[v] - accR[v];
-            }
-        } else {
-            TV accD[16], accR[16];
-            tile_product<TV>(S0, S0, tx, ty, accD);
-            if (has_row) tile_product<TV>(S1, S0, tx, ty, accR);
-            TV aD[16], aR[16];
-#pragma unroll
-            for (int p = 0; p < 16; ++p) {
-                const int64_t off = tx + (c0 + 16 * ty + p) * lda;
-                aD[p] = M[c0 + off];
-                aR[p] = has_row ? M[i0 + off] : TV(0);
-            }
-            __syncthreads();
-#pragma unroll
-            for (int p = 0; p < 16; ++p) {
-                S0[tx][16 * ty + p] = aD[p] - accD[p];
-                if (has_row) S1[tx][16 * ty + p] = aR[p] - accR[p];
-            }
+        for (int v = 0; v < 16; ++v) {
+            const int col = 32 * (wave & 1) + mfma_col(v, r);
+            S0[row][col] = aD[v] - accD[v];
+            if (has_row) S1[row][col] = aR[v] - accR[v];
         }
         __syncthreads();
         if (role == 0) {
@@ -549,57 +550,42 @@ __global__ void __launch_bounds__(256, 4) k_chol_step(int k, int T, int64_t lda,
         out_ld = has_row ? lda : CB;
     }
     bool bad_any = false;
-    if constexpr (std::is_same<TV, double>::value) {
-        // FP64: one pivot per barrier (the sub-block form below needs twice the
-        // FP32 registers for its broadcast operands and spills)
-        for (int e = t; e < 2 * kColStride; e += 256) colS[e] = TV(0);
-        __syncthreads();
-        TV coef = TV(0);
-        if (role == 0) coef = panel_pivot<TV>(0, z[0], colS, r, bad_any);
-        int j = 0;
-        panel_quarter<TV, 63>(j, z, colS, role, r, bad_any, coef, out, out_ld);
-        panel_quarter<TV, 47>(j, z, colS, role, r, bad_any, coef, out, out_ld);
-        panel_quarter<TV, 31>(j, z, colS, role, r, bad_any, coef, out, out_ld);
-        panel_quarter<TV, 15>(j, z, colS, role, r, bad_any, coef, out, out_ld);
-        if (role == 0 && bad_any && w == 0) fail[0] = 1;
-        return;
-    }
     __syncthreads();  // every wave holds its rows: S0 now carries the published L columns
     TV (*Lt)[kTSB] = reinterpret_cast<TV (*)[kTSB]>(&S0[0][0]);
-    TV* invp = colS;
     TV inv = TV(1);
     // the diagonal wave runs one sub-block ahead of the block-row wave
     if (role == 0) { diag_chain<TV, 0>(z, r, bad_any, inv); diag_publish<TV, 0>(z, r, inv, Lt, invp); }
     __syncthreads();
     if (role == 0) {
-        diag_trail<TV, 0>(z, Lt);
+        diag_trail_mfma<0>(z);
         diag_chain<TV, 1>(z, r, bad_any, inv);
         diag_publish<TV, 1>(z, r, inv, Lt, invp);
     } else if (role == 1) {
         row_solve<TV, 0>(z, Lt, invp, r, out, out_ld);
-        row_trail<TV, 0>(z, Lt, r);
+        row_trail_mfma<0>(z, Lt, r);
     }
     __syncthreads();
     if (role == 0) {
-        diag_trail<TV, 1>(z, Lt);
+        diag_trail_mfma<1>(z);
         diag_chain<TV, 2>(z, r, bad_any, inv);
         diag_publish<TV, 2>(z, r, inv, Lt, invp);
     } else if (role == 1) {
         row_solve<TV, 1>(z, Lt, invp, r, out, out_ld);
-        row_trail<TV, 1>(z, Lt, r);
+        row_trail_mfma<1>(z, Lt, r);
     }
     __syncthreads();
     if (role == 0) {
-        diag_trail<TV, 2>(z, Lt);
+        diag_trail_mfma<2>(z);
         diag_chain<TV, 3>(z, r, bad_any, inv);
         diag_publish<TV, 3>(z, r, inv, Lt, invp);
     } else if (role == 1) {
         row_solve<TV, 2>(z, Lt, invp, r, out, out_ld);
-        row_trail<TV, 2>(z, Lt, r);
+        row_trail_mfma<2>(z, Lt, r);
     }
     __syncthreads();
     if (role == 1) row_solve<TV, 3>(z, Lt, invp, r, out, out_ld);
     if (role == 0 && bad_any && w == 0) fail[0] = 1;
+    }
 }
 
 // y = row np of the layout (L^-1 rhs after the factorization).
