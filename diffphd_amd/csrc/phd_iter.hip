@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(NT) k_iter_residual(IterResidual a, TV* __rest
         const int c = a.vcand[v];
         if (c >= 0) r += a.F[3 * c + d];
     }
-    w[(int64_t)d * ldw + a.ipos[v]] = (TV)r;
+    w[a.ipos ? (int64_t)d * ldw + a.ipos[v] : i] = (TV)r;
 }
 
 // x <- 0 where it is not finite; block sums of x.x

@@ -147,7 +147,8 @@ struct IterResidual {
     double *pd_rhs = nullptr, *x_prev = nullptr;
 };
 // fwd: rhs is q~ and pd_rhs, c_dir are used; else b = rhs + the contributions.
-// w[d * ldw + ipos[v]] = the residual (the S product's input), x_prev = x.
+// w[d * ldw + ipos[v]] = the residual (the S product's input), or w[3 v + d] when
+// ipos is null; x_prev = x.
 template <class TV>
 void launch_iter_residual(hipStream_t s, const IterResidual& a, bool fwd, TV* w, int ldw);
 // x <- 0 where not finite; part[0 .. iter_rows(n)) = block sums of x.x
@@ -160,6 +161,20 @@ void launch_iter_push(hipStream_t s, int n, const AAHist& h, double* x, const do
 void launch_iter_combine(hipStream_t s, int n, bool fwd, const AAHist& h, const double* part, const double* gram_in,
                          double* gram_out, const double* x_prev, double* x, const unsigned char* fix, const double* fixval,
                          const double* pd_rhs, double* pd_prev, double* out);
+
+// ---- explicit inverse of small systems (phd_small.hip) -------------------------
+// out (n x ld, zero-filled by the caller past column n) = S^T S in vertex order;
+// items[item_ptr[t] .. item_ptr[t + 1]): the rows of S that cross column tile t
+template <class TV>
+void launch_dense_inverse(hipStream_t s, int n, int ld, const int* items, const int* item_ptr, const int* fd,
+                          const int64_t* base, const double* V, const int* perm, TV* out);
+// out (n x ldk) = the candidate columns of inv (n x ld), zeros past column K
+template <class TV>
+void launch_dense_columns(hipStream_t s, int n, int ld, int K, int ldk, const int* cand, const TV* inv, TV* out);
+// out = add + M x on the three axes (see k_dense_apply)
+template <class TV>
+void launch_dense_apply(hipStream_t s, int n, int ncol, int ld, const TV* M, const double* x, const double* add,
+                        const unsigned char* dmask, const double* dval, const int* vcand, double* uC, double* out);
 
 // ---- contact -----------------------------------------------------------------
 // normals / tangents at the frame-start positions (GetLocalFrame)

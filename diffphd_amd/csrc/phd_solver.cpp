@@ -1122,6 +1122,8 @@ void Body::setup(double dt, int threads) {
         Ap_[v + 1] = (int)Ai_.size();
         std::vector<std::pair<int, double>>().swap(r);
     }
+    d_inv64_.release(); d_invC64_.release();  // formed on first use
+    d_inv32_.release(); d_invC32_.release();
     // factor (host FP64) and expansion of S = L^-1 (device FP64, FP32 copy)
     factor_.build(nv_, Ap_, Ai_, Ax_, X_, threads);
     plan_.build(factor_, unit_items_, chunk_w_);
@@ -1836,6 +1838,11 @@ void Body::apply_ainv(double dt, const double* b, double* x, int precision, int 
 
 // x = A^-1 r with the FP64 factor on device vectors (the baseline's global solve).
 void Body::ainv64(const double* r, double* x) {
+    if (nv_ <= kDenseMaxVertices) {
+        ensure_dense(0);
+        launch_dense_apply<double>(stream_, nv_, nv_, inv_ld_, d_inv64_.p, r, nullptr, nullptr, nullptr, nullptr, nullptr, x);
+        return;
+    }
     spmv_S<double>(r, w64_, y64_, part64_, V64_.p);
     spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, x);
 }
@@ -2023,6 +2030,59 @@ void Body::iter_residual(bool fwd, const double* rhs, double* x, double* xprev, 
     launch_iter_residual<TV>(stream_, a, fwd, w.p, spmv_ldw(nv_));
 }
 
+void Body::iter_residual_dense(bool fwd, const double* rhs, double* x, double* xprev, double inv_h2m, const double* F,
+                               double* r) {
+    launch_iter_residual<double>(stream_, iter_args(rhs, x, xprev, inv_h2m, F), fwd, r, 0);
+}
+
+// ---------------------------------------------------------------------------
+// Explicit inverse of a small body (phd_small.hip).
+// ---------------------------------------------------------------------------
+bool Body::dense_inverse(const std::map<std::string, double>& opt, int precision) {
+    if (nv_ > kDenseMaxVertices || opt_or(opt, "phd_dense_inverse", 1.0) == 0.0) return false;
+    ensure_dense(precision);
+    return true;
+}
+
+void Body::ensure_dense(int precision) {
+    if (precision == 1 ? d_inv32_.p != nullptr : d_inv64_.p != nullptr) return;
+    const int T = (nv_ + 63) / 64;
+    std::vector<int> ptr(T + 1);
+    for (int t = 0; t < T; ++t) ptr[t] = plan_.cu_i0[plan_.tile_unit_ptr[t]];
+    ptr[T] = (int)plan_.items.size();
+    DevBuf<int> dptr;
+    dptr.upload(ptr);
+    inv_ld_ = (nv_ + 3) / 4 * 4;
+    inv_ldk_ = (K_ + 3) / 4 * 4;
+    auto form = [&](auto& inv, auto& invC) {
+        using TV = typename std::remove_reference<decltype(*inv.p)>::type;
+        inv.alloc((size_t)nv_ * inv_ld_);
+        hip_check(hipMemsetAsync(inv.p, 0, inv.n * sizeof(TV), stream_), "inverse padding");
+        launch_dense_inverse<TV>(stream_, nv_, inv_ld_, d_items_.p, dptr.p, d_fd_.p, d_base_.p, V64_.p, d_perm_.p, inv.p);
+        if (K_ > 0) {
+            invC.alloc((size_t)nv_ * inv_ldk_);
+            launch_dense_columns<TV>(stream_, nv_, inv_ld_, K_, inv_ldk_, d_cand_.p, inv.p, invC.p);
+        }
+        hip_check(hipStreamSynchronize(stream_), "explicit inverse");
+    };
+    if (precision == 1) form(d_inv32_, d_invC32_);
+    else form(d_inv64_, d_invC64_);
+}
+
+void Body::dense_solve(int precision, const double* r, const double* add, const double* dval, double* uC, double* x) {
+    if (precision == 1)
+        launch_dense_apply<float>(stream_, nv_, nv_, inv_ld_, d_inv32_.p, r, add, d_dmask_.p, dval, d_vcand_.p, uC, x);
+    else
+        launch_dense_apply<double>(stream_, nv_, nv_, inv_ld_, d_inv64_.p, r, add, d_dmask_.p, dval, d_vcand_.p, uC, x);
+}
+
+void Body::dense_impulse(int precision, const double* f, const double* dval, double* x) {
+    if (precision == 1)
+        launch_dense_apply<float>(stream_, nv_, K_, inv_ldk_, d_invC32_.p, f, x, d_dmask_.p, dval, nullptr, nullptr, x);
+    else
+        launch_dense_apply<double>(stream_, nv_, K_, inv_ldk_, d_invC64_.p, f, x, d_dmask_.p, dval, nullptr, nullptr, x);
+}
+
 // ---------------------------------------------------------------------------
 // Forward step.
 // ---------------------------------------------------------------------------
@@ -2130,6 +2190,7 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
     DevAnderson aa;
     aa.init(aa_window, n3, d_hist_q_, d_hist_g_);
     aa.replay = rp;
+    const bool dense = K == 0 && dense_inverse(opt, precision);
     hip_check(hipMemsetAsync(d_pdrhs_prev_.p, 0, sizeof(double) * n3, stream_), "prev pd_rhs");
     bool dense64 = precision == 0;
     bool converged = false;
@@ -2150,7 +2211,10 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
         {
             PhaseTimer ts(this, kFwdSolve);
             const double* F = K > 0 ? d_F_.p : nullptr;
-            if (precision == 1) {
+            if (dense) {
+                iter_residual_dense(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, d_r_.p);
+                dense_solve(precision, d_r_.p, d_qprev_.p, d_dval_full_.p, nullptr, d_q_.p);
+            } else if (precision == 1) {
                 iter_residual<float>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w32_);
                 spmv_rows<float>(w32_, y32_, part32_, V32_.p);
             } else {
@@ -2244,7 +2308,8 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
         }
         {
             PhaseTimer ts(this, kFwdSolve);
-            if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_qprev_.p, d_dval_full_.p, d_q_.p);
+            if (dense) { /* the explicit inverse left x in d_q_ */ }
+            else if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_qprev_.p, d_dval_full_.p, d_q_.p);
             else spmv_ST<double>(y64_, xpart64_, V64_.p, d_qprev_.p, d_dval_full_.p, d_q_.p);
             partial_dirichlet(d_q_.p, d_qprev_.p, d_dval_full_.p);
         }
@@ -2452,6 +2517,7 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
     const int aa_window = (int)opt_or(opt, "aa_window", 5);
     check(aa_window >= 0 && aa_window <= 6, "aa_window must be in [0, 6].");
     const double clip = opt_or(opt, "alg_phd_bwd_clip_norm", 1e6);
+    const bool dense = dense_inverse(opt, precision);
     DevBuf<double> d_rhs, d_s, d_sprev, d_zero;
     d_rhs.upload(rhs_qbar);
     d_s.alloc(n3);
@@ -2482,7 +2548,10 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
         for (int i = 0; i < max_it; ++i) {
             // s_prev = s; r = rhs + K s - A s
             kpd_elements(d_s.p, precision);
-            if (precision == 1) {
+            if (dense) {
+                iter_residual_dense(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, d_r_.p);
+                dense_solve(precision, d_r_.p, d_sprev.p, nullptr, nb > 0 ? d_uC_.p : nullptr, d_s.p);
+            } else if (precision == 1) {
                 iter_residual<float>(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, w32_);
                 spmv_rows<float>(w32_, y32_, part32_, V32_.p);
             } else {
@@ -2495,16 +2564,21 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
                 // copy in mixed mode), expand back to candidate impulses and scatter through
                 // S_C. The constraint residual J s rides along, so with an FP32 factor and
                 // G^-1 the iterates converge onto J s = 0 instead of drifting off it.
-                if (precision == 1) contact_gather<float>(y32_, d_uC_.p); else contact_gather<double>(y64_, d_uC_.p);
+                if (dense) { /* dense_solve wrote uC */ }
+                else if (precision == 1) contact_gather<float>(y32_, d_uC_.p);
+                else contact_gather<double>(y64_, d_uC_.p);
                 PhaseTimer tbs(this, kBwdBasisSolve);
                 launch_gather_nodes(stream_, K_, d_cand_.p, d_sprev.p, d_tmpK3_.p);
                 launch_basis_project(stream_, nb, d_bcidx.p, d_dirs.p, d_uC_.p, d_tmpK3_.p, d_rhsK_.p);
                 if (precision == 1) launch_gemv_sym<float>(stream_, nb, gld, d_Gs32.p, d_rhsK_.p, d_Gx.p);
                 else launch_gemv_sym<double>(stream_, nb, gld, d_Gs64.p, d_rhsK_.p, d_Gx.p);
                 launch_basis_expand(stream_, K_, d_bcptr.p, d_bclist.p, d_dirs.p, d_Gx.p, d_dF_.p);
-                if (precision == 1) contact_scatter<float>(d_dF_.p, y32_); else contact_scatter<double>(d_dF_.p, y64_);
+                if (dense) dense_impulse(precision, d_dF_.p, nullptr, d_s.p);
+                else if (precision == 1) contact_scatter<float>(d_dF_.p, y32_);
+                else contact_scatter<double>(d_dF_.p, y64_);
             }
-            if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_sprev.p, d_zero.p, d_s.p);
+            if (dense) { /* the explicit inverse left s in d_s */ }
+            else if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_sprev.p, d_zero.p, d_s.p);
             else spmv_ST<double>(y64_, xpart64_, V64_.p, d_sprev.p, d_zero.p, d_s.p);
             partial_dirichlet(d_s.p, d_sprev.p, nullptr);
             // safe_clip (backward_gpu.cpp:809-816) before and after the Anderson

@@ -428,6 +428,9 @@ private:
     DevBuf<double> d_dot_partial_, d_dot_out_;
     DevBuf<double> d_iter_part_, d_iter_norm_, d_aa_gram_[2];
     DevBuf<int> d_iperm_, d_vcand_;
+    int inv_ld_ = 0, inv_ldk_ = 0;
+    DevBuf<double> d_inv64_, d_invC64_;
+    DevBuf<float> d_inv32_, d_invC32_;
     DevBuf<unsigned char> d_fix_;  // Dirichlet DOFs (empty without any)
     DevBuf<float> w32_, y32_, part32_, xpart32_;
     DevBuf<double> w64_, y64_, part64_, xpart64_;
@@ -501,6 +504,20 @@ private:
     IterResidual iter_args(const double* rhs, double* x, double* xprev, double inv_h2m, const double* F);
     template <class TV>
     void iter_residual(bool fwd, const double* rhs, double* x, double* xprev, double inv_h2m, const double* F, DevBuf<TV>& w);
+    // the same with w in vertex order (AoS, FP64), for the explicit inverse
+    void iter_residual_dense(bool fwd, const double* rhs, double* x, double* xprev, double inv_h2m, const double* F, double* r);
+    // Explicit A^-1 of a small body (FP64 or an FP32 copy), formed on first use
+    // per precision. dense_inverse: whether a step takes it (option
+    // phd_dense_inverse = 0 keeps the products with S): the adjoint of every small
+    // body, the forward of one without a frictional boundary (with one, the
+    // iteration amplifies the round-off between the two forms).
+    static constexpr int kDenseMaxVertices = 4096;
+    bool dense_inverse(const std::map<std::string, double>& opt, int precision);
+    void ensure_dense(int precision);
+    // x = x_prev + A^-1 r (uC: A^-1 r at the candidates, may be null), and
+    // x += (A^-1)_C f; dval as in launch_dense_apply
+    void dense_solve(int precision, const double* r, const double* add, const double* dval, double* uC, double* x);
+    void dense_impulse(int precision, const double* f, const double* dval, double* x);
     template <class TV>
     void spmv_rows(DevBuf<TV>& w, DevBuf<TV>& y, DevBuf<TV>& part, const TV* V);
     bool solve_contact_system(int n, int precision, const int* J, bool plain_w = false);
