@@ -30,8 +30,8 @@ def _compare(spec, opt, tol):
 
 
 # 30 capped iterations from rest: both forms run the same iterations, which carry
-# round-off of 1e-16 (FP64) or 1e-7 times a shrinking residual (mixed) each; the
-# adjoint's steps likewise. 12 to 4,352 vertices: below one 64-row tile, one row past
+# round-off of 1e-16 (FP64) or 6e-8 times the step (mixed) each, and the unconverged
+# Anderson iteration multiplies it (by up to 1e2 here); the adjoint's steps likewise. 12 to 4,352 vertices: below one 64-row tile, one row past
 # it (65 = 13 x 5 x 1 vertices), the switch to four rows per workgroup, and 4,096 / 4,352
 # around the largest body with an inverse.
 @pytest.mark.parametrize("cells", [(2, 1, 1), (3, 3, 3), (12, 4, 0), (7, 6, 5), (10, 9, 8), (11, 10, 8), (15, 15, 15),
@@ -44,14 +44,14 @@ def test_hex_bodies(cells, precision):
     for dof, _ in spec["dirichlet"]:
         spec["v0"][dof] = 0.0
     opt = dict(spec["options"], max_pd_iter=30, rel_tol=0.0, abs_tol=0.0, phd_precision=precision)
-    _compare(spec, opt, 1e-9 if precision == 0 else 1e-5)
+    _compare(spec, opt, 1e-9 if precision == 0 else 1e-4)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
 def test_per_dof_dirichlet(precision):
     spec = slider()
     opt = dict(spec["options"], max_pd_iter=30, rel_tol=0.0, abs_tol=0.0, phd_precision=precision)
-    _compare(spec, opt, 1e-9 if precision == 0 else 1e-5)
+    _compare(spec, opt, 1e-9 if precision == 0 else 1e-4)
 
 
 @pytest.mark.parametrize("precision", [0, 1])
