@@ -70,27 +70,33 @@ bool propose_new_set(const std::set<int>& a, const std::set<int>& b, std::set<in
 }
 }  // namespace
 
-// ComputePdEnergy + ActuationEnergy: per-element energies summed on the host in
-// element order.
-double Body::baseline_energy(const double* q) {
+// ComputePdEnergy + ActuationEnergy at q: per-element energies summed on the host in
+// element order (the element forces stay in d_elem_ for baseline_force). rr (may be
+// null) = res . res, brought down with them.
+double Body::baseline_energy(const double* q, const double* res, double* rr) {
     d_bl_energy_.alloc(ne_);
+    pin_energy_.alloc((size_t)ne_ + 1);
     if (d_elem_.n < (size_t)ne_ * edim_ * 3) d_elem_.alloc((size_t)ne_ * edim_ * 3);
     launch_pd_energy_force(stream_, mat_, has_cor_ ? d_kc_.p : nullptr, has_vol_ ? d_kv_.p : nullptr, q, d_bl_energy_.p,
                            d_elem_.p);
+    hip_check(hipMemcpyAsync(pin_energy_.p, d_bl_energy_.p, sizeof(double) * ne_, hipMemcpyDeviceToHost, stream_), "energies");
+    if (rr) {
+        DotArgs a;
+        a.m = 1;
+        a.a[0] = a.b[0] = res;
+        launch_dots(stream_, dofs_, a, d_dot_partial_.p, d_dot_out_.p);
+        hip_check(hipMemcpyAsync(pin_energy_.p + ne_, d_dot_out_.p, sizeof(double), hipMemcpyDeviceToHost, stream_), "dots");
+    }
     hip_check(hipStreamSynchronize(stream_), "baseline energy");
-    std::vector<double> e(ne_);
-    d_bl_energy_.download(e.data(), ne_);
+    if (rr) *rr = pin_energy_.p[ne_];
     double t = 0;
-    for (double x : e) t += x;
+    for (int e = 0; e < ne_; ++e) t += pin_energy_.p[e];
     return t;
 }
 
-// PdEnergyForce + ActuationForce at q into f (3N, device).
-void Body::baseline_force(const double* q, double* f) {
-    d_bl_energy_.alloc(ne_);
-    if (d_elem_.n < (size_t)ne_ * edim_ * 3) d_elem_.alloc((size_t)ne_ * edim_ * 3);
-    launch_pd_energy_force(stream_, mat_, has_cor_ ? d_kc_.p : nullptr, has_vol_ ? d_kv_.p : nullptr, q, d_bl_energy_.p,
-                           d_elem_.p);
+// PdEnergyForce + ActuationForce into f (3N, device), at the positions of the last
+// baseline_energy call.
+void Body::baseline_force(double* f) {
     launch_gather_vertex(stream_, nv_, d_inc_ptr_.p, d_inc_idx_.p, d_elem_.p, f);
 }
 
@@ -168,6 +174,39 @@ void Body::pd_lhs_solve(const double* r, double* x, const std::vector<int>& froz
     launch_copy_nodes(stream_, nc, d_bl_nodes_.p, r, x);
 }
 
+// The two-loop recursion around PdLhsSolve.
+void Body::lbfgs_direction(const std::deque<int>& sh, const std::deque<int>& yh, const double* g, double* tmp, double* dir,
+                           const std::vector<int>& frozen) {
+    const int m = (int)sh.size();
+    if (m <= kLbfgsMax && dofs_ <= kLbfgsEntries) {
+        LbfgsHist h;
+        h.m = m;
+        for (int k = 0; k < m; ++k) { h.S[k] = d_bl_[sh[k]]->p; h.Y[k] = d_bl_[yh[k]]->p; }
+        d_bl_coef_.alloc(2 * kLbfgsMax);
+        launch_lbfgs_first(stream_, dofs_, h, g, tmp, d_bl_coef_.p);
+        pd_lhs_solve(tmp, dir, frozen);
+        launch_lbfgs_second(stream_, dofs_, h, d_bl_coef_.p, dir);
+        return;
+    }
+    launch_axpbypcz(stream_, dofs_, 1.0, g, 0.0, nullptr, 0.0, nullptr, tmp);
+    std::vector<double> rho(m), alpha(m);
+    for (int k = m - 1; k >= 0; --k) {
+        const double* sk = d_bl_[sh[k]]->p;
+        const double* yk = d_bl_[yh[k]]->p;
+        const auto d = dots({{yk, sk}, {sk, tmp}});
+        rho[k] = 1 / d[0];
+        alpha[k] = rho[k] * d[1];
+        launch_axpbypcz(stream_, dofs_, 1.0, tmp, -alpha[k], yk, 0.0, nullptr, tmp);
+    }
+    pd_lhs_solve(tmp, dir, frozen);
+    for (int k = 0; k < m; ++k) {
+        const double* sk = d_bl_[sh[k]]->p;
+        const double* yk = d_bl_[yh[k]]->p;
+        const double beta = rho[k] * dots({{yk, dir}})[0];
+        launch_axpbypcz(stream_, dofs_, 1.0, dir, alpha[k] - beta, sk, 0.0, nullptr, dir);
+    }
+}
+
 // PdNonlinearSolve (forward.cpp:294-526). Returns the iterations used; throws
 // when max_pd_iter is reached, as the reference does.
 int Body::pd_nonlinear_solve(const double* q_init, double inv_h2m, const double* rhs, const std::vector<int>& frozen,
@@ -202,19 +241,21 @@ int Body::pd_nonlinear_solve(const double* q_init, double inv_h2m, const double*
     const int nfix = (int)fix.size();
     d_bl_fix_.upload(fix);
     d_bl_fixv_.upload(fixv);
-    auto objective = [&](const double* qc, double e) {
+    auto objective = [&](const double* qc) {
         launch_axpbypcz(stream_, n3, 1.0, qc, -1.0, rhs, 0.0, nullptr, tmp);
-        return 0.5 * inv_h2m * dots({{tmp, tmp}})[0] + e;
+        double rr;
+        const double e = baseline_energy(qc, tmp, &rr);
+        return 0.5 * inv_h2m * rr + e;
     };
-    auto gradient = [&](const double* qc) {  // grad = (inv_h2m (q - rhs) - f) on the free DOFs
-        baseline_force(qc, force);
+    // grad = (inv_h2m (q - rhs) - f) on the free DOFs, at the last objective's q
+    auto gradient = [&](const double* qc) {
+        baseline_force(force);
         launch_axpbypcz(stream_, n3, inv_h2m, qc, -inv_h2m, rhs, -1.0, force, grad);
         launch_zero_dirichlet(stream_, nfix, d_bl_fix_.p, grad);
     };
     hip_check(hipMemcpyAsync(q_sol, q_init, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "q_init");
     launch_set_dirichlet(stream_, nfix, d_bl_fix_.p, d_bl_fixv_.p, q_sol);
-    double energy = baseline_energy(q_sol);
-    double obj = objective(q_sol, energy);
+    double obj = objective(q_sol);
     gradient(q_sol);
     launch_axpbypcz(stream_, n3, inv_h2m, rhs, 0.0, nullptr, 0.0, nullptr, tmp);
     launch_zero_dirichlet(stream_, nfix, d_bl_fix_.p, tmp);
@@ -248,25 +289,7 @@ int Body::pd_nonlinear_solve(const double* q_init, double inv_h2m, const double*
                     sh.pop_front();
                     yh.pop_front();
                 }
-                // two-loop recursion, newest pair first
-                launch_axpbypcz(stream_, n3, 1.0, grad, 0.0, nullptr, 0.0, nullptr, tmp);
-                const int m = (int)sh.size();
-                std::vector<double> rho(m), alpha(m);
-                for (int k = m - 1; k >= 0; --k) {
-                    const double* sk = d_bl_[sh[k]]->p;
-                    const double* yk = d_bl_[yh[k]]->p;
-                    const auto d = dots({{yk, sk}, {sk, tmp}});
-                    rho[k] = 1 / d[0];
-                    alpha[k] = rho[k] * d[1];
-                    launch_axpbypcz(stream_, n3, 1.0, tmp, -alpha[k], yk, 0.0, nullptr, tmp);
-                }
-                pd_lhs_solve(tmp, dir, frozen);
-                for (int k = 0; k < m; ++k) {
-                    const double* sk = d_bl_[sh[k]]->p;
-                    const double* yk = d_bl_[yh[k]]->p;
-                    const double beta = rho[k] * dots({{yk, dir}})[0];
-                    launch_axpbypcz(stream_, n3, 1.0, dir, alpha[k] - beta, sk, 0.0, nullptr, dir);
-                }
+                lbfgs_direction(sh, yh, grad, tmp, dir, frozen);
             }
             hip_check(hipMemcpyAsync(xlast, q_sol, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "x_last");
             hip_check(hipMemcpyAsync(glast, grad, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "g_last");
@@ -279,18 +302,16 @@ int Body::pd_nonlinear_solve(const double* q_init, double inv_h2m, const double*
             // backtracking line search: obj(q - t d) < obj - 1e-4 t g.d (+ eps)
             double step = 1;
             launch_axpbypcz(stream_, n3, 1.0, q_sol, -step, dir, 0.0, nullptr, qn);
-            double en = baseline_energy(qn), on = objective(qn, en);
+            double on = objective(qn);
             for (int j = 0; j < max_ls; ++j) {
                 const double cond = obj - 1e-4 * step * gd;
                 if (!std::isnan(on) && on < cond + DBL_EPSILON) break;
                 step /= 2;
                 launch_axpbypcz(stream_, n3, 1.0, q_sol, -step, dir, 0.0, nullptr, qn);
-                en = baseline_energy(qn);
-                on = objective(qn, en);
+                on = objective(qn);
                 ++last_baseline.ls_steps;
             }
             hip_check(hipMemcpyAsync(q_sol, qn, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "accept");
-            energy = en;
             obj = on;
         } else {
             // local step with the augmented conditions' constant part, then the global step
@@ -301,6 +322,7 @@ int Body::pd_nonlinear_solve(const double* q_init, double inv_h2m, const double*
             launch_zero_dirichlet(stream_, nfix, d_bl_fix_.p, tmp);
             pd_lhs_solve(tmp, q_sol, frozen);
             launch_set_dirichlet(stream_, nfix, d_bl_fix_.p, d_bl_fixv_.p, q_sol);
+            baseline_energy(q_sol, nullptr, nullptr);
         }
         gradient(q_sol);
         if (std::sqrt(dots({{grad, grad}})[0]) <= rel_tol * rhs_norm + abs_tol) return it + 1;
@@ -365,7 +387,8 @@ void Body::forward_baseline(const std::string& method, const double* q, const do
         std::vector<double> vals;
         frozen_of(active, fr, vals);
         last_baseline.pd_iters += pd_nonlinear_solve(dq0.p, inv_h2m, d_qtilde_.p, fr, vals, opt, dqs.p);
-        baseline_force(dqs.p, dfs.p);
+        baseline_energy(dqs.p, nullptr, nullptr);
+        baseline_force(dfs.p);
         hip_check(hipStreamSynchronize(stream_), "baseline");
         dqs.download(qs.data(), n3);
         dfs.download(fs.data(), n3);
@@ -540,24 +563,7 @@ void Body::backward_baseline(const double* q, const double* v, const double* f_e
                     yh.pop_front();
                 }
                 double* qv = xn;  // scratch for the two-loop vector
-                launch_axpbypcz(stream_, n3, 1.0, grad, 0.0, nullptr, 0.0, nullptr, qv);
-                const int m = (int)sh.size();
-                std::vector<double> rho(m), alpha(m);
-                for (int k = m - 1; k >= 0; --k) {
-                    const double* sk = d_bl_[sh[k]]->p;
-                    const double* yk = d_bl_[yh[k]]->p;
-                    const auto d = dots({{yk, sk}, {sk, qv}});
-                    rho[k] = 1 / d[0];
-                    alpha[k] = rho[k] * d[1];
-                    launch_axpbypcz(stream_, n3, 1.0, qv, -alpha[k], yk, 0.0, nullptr, qv);
-                }
-                pd_lhs_solve(qv, dir, frozen);
-                for (int k = 0; k < m; ++k) {
-                    const double* sk = d_bl_[sh[k]]->p;
-                    const double* yk = d_bl_[yh[k]]->p;
-                    const double beta = rho[k] * dots({{yk, dir}})[0];
-                    launch_axpbypcz(stream_, n3, 1.0, dir, alpha[k] - beta, sk, 0.0, nullptr, dir);
-                }
+                lbfgs_direction(sh, yh, grad, qv, dir, frozen);
             }
             hip_check(hipMemcpyAsync(xl, x, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "x_last");
             hip_check(hipMemcpyAsync(gl, grad, sizeof(double) * n3, hipMemcpyDeviceToDevice, stream_), "g_last");

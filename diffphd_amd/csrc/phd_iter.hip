@@ -310,6 +310,58 @@ __global__ void __launch_bounds__(NT) k_iter_combine(int n, AAHist h, const doub
     }
 }
 
+// -----------------------------------------------------------------------------
+// The two loops of L-BFGS (h: pairs oldest first) in one workgroup each: every step
+// needs the previous one's dot product, which as launches with a host round trip each
+// took about 20 us; here it is a barrier. A thread owns its entries throughout.
+// -----------------------------------------------------------------------------
+constexpr int NL = 1024;
+
+// sum over the workgroup of two values; sh alternates between two buffers, so one
+// barrier per call is enough
+__device__ inline void block_sum2(double& a, double& b, double (*sh)[2]) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if (threadIdx.x % WAVE == 0) { sh[threadIdx.x / WAVE][0] = a; sh[threadIdx.x / WAVE][1] = b; }
+    __syncthreads();
+    a = b = 0;
+#pragma unroll
+    for (int w = 0; w < NL / WAVE; ++w) { a += sh[w][0]; b += sh[w][1]; }
+}
+
+// q = g, then from the newest pair to the oldest alpha_k = rho_k s_k . q and
+// q -= alpha_k y_k; coef: alpha, then rho (kLbfgsMax each)
+__global__ void __launch_bounds__(NL) k_lbfgs_first(int n, LbfgsHist h, const double* __restrict__ g, double* __restrict__ q,
+                                                    double* __restrict__ coef) {
+    __shared__ double sh[2][NL / WAVE][2];
+    for (int k = h.m - 1; k >= 0; --k) {
+        const double *s = h.S[k], *y = h.Y[k];
+        double ys = 0, sq = 0;
+        for (int i = threadIdx.x; i < n; i += NL) {
+            ys += y[i] * s[i];
+            sq += s[i] * (k == h.m - 1 ? g[i] : q[i]);
+        }
+        block_sum2(ys, sq, sh[k & 1]);
+        const double rho = 1 / ys, alpha = rho * sq;
+        for (int i = threadIdx.x; i < n; i += NL) q[i] = (k == h.m - 1 ? g[i] : q[i]) - alpha * y[i];
+        if (threadIdx.x == 0) { coef[k] = alpha; coef[kLbfgsMax + k] = rho; }
+    }
+}
+
+// from the oldest pair to the newest: d += (alpha_k - rho_k y_k . d) s_k
+__global__ void __launch_bounds__(NL) k_lbfgs_second(int n, LbfgsHist h, const double* __restrict__ coef,
+                                                     double* __restrict__ d) {
+    __shared__ double sh[2][NL / WAVE][2];
+    for (int k = 0; k < h.m; ++k) {
+        const double *s = h.S[k], *y = h.Y[k];
+        double yd = 0, unused = 0;
+        for (int i = threadIdx.x; i < n; i += NL) yd += y[i] * d[i];
+        block_sum2(yd, unused, sh[k & 1]);
+        const double c = coef[k] - coef[kLbfgsMax + k] * yd;
+        for (int i = threadIdx.x; i < n; i += NL) d[i] += c * s[i];
+    }
+}
+
 }  // namespace
 
 int iter_rows(int n) { return std::max(1, std::min(kIterRows, (n + NT - 1) / NT)); }
@@ -322,6 +374,13 @@ void launch_iter_residual(hipStream_t s, const IterResidual& a, bool fwd, TV* w,
 }
 template void launch_iter_residual<float>(hipStream_t, const IterResidual&, bool, float*, int);
 template void launch_iter_residual<double>(hipStream_t, const IterResidual&, bool, double*, int);
+
+void launch_lbfgs_first(hipStream_t s, int n, const LbfgsHist& h, const double* g, double* q, double* coef) {
+    hipLaunchKernelGGL(k_lbfgs_first, dim3(1), dim3(NL), 0, s, n, h, g, q, coef);
+}
+void launch_lbfgs_second(hipStream_t s, int n, const LbfgsHist& h, const double* coef, double* d) {
+    hipLaunchKernelGGL(k_lbfgs_second, dim3(1), dim3(NL), 0, s, n, h, coef, d);
+}
 
 void launch_iter_norm(hipStream_t s, int n, double* x, double* part) {
     hipLaunchKernelGGL(k_iter_norm, dim3(iter_rows(n)), dim3(NT), 0, s, n, x, part);

@@ -163,6 +163,20 @@ void launch_iter_combine(hipStream_t s, int n, bool fwd, const AAHist& h, const 
                          const double* pd_rhs, double* pd_prev, double* out);
 
 // ---- explicit inverse of small systems (phd_small.hip) -------------------------
+// L-BFGS direction of the baseline in one workgroup per loop, for vectors of up to
+// kLbfgsEntries and kLbfgsMax pairs (oldest first): beyond about 32,000 entries one
+// CU's reads of the pairs cost what the launches and round trips of many blocks do.
+// coef: 2 kLbfgsMax doubles carried from the first loop to the second.
+constexpr int kLbfgsMax = 32;
+constexpr int kLbfgsEntries = 32768;
+struct LbfgsHist {
+    int m = 0;
+    const double* S[kLbfgsMax] = {};
+    const double* Y[kLbfgsMax] = {};
+};
+void launch_lbfgs_first(hipStream_t s, int n, const LbfgsHist& h, const double* g, double* q, double* coef);
+void launch_lbfgs_second(hipStream_t s, int n, const LbfgsHist& h, const double* coef, double* d);
+
 // out (n x ld, zero-filled by the caller past column n) = S^T S in vertex order;
 // items[item_ptr[t] .. item_ptr[t + 1]): the rows of S that cross column tile t
 template <class TV>

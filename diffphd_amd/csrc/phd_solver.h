@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <array>
+#include <deque>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -56,6 +57,24 @@ struct DevBuf {
         std::vector<T> h(n);
         download(h.data(), n);
         return h;
+    }
+};
+
+// pinned host memory (doubles)
+struct PinBuf {
+    double* p = nullptr;
+    size_t n = 0;
+    PinBuf() = default;
+    PinBuf(const PinBuf&) = delete;
+    PinBuf& operator=(const PinBuf&) = delete;
+    ~PinBuf() { if (p) (void)hipHostFree(p); }
+    void alloc(size_t count) {
+        if (count <= n) return;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        n = 0;
+        hip_check(hipHostMalloc((void**)&p, count * sizeof(double), hipHostMallocDefault), "hipHostMalloc");
+        n = count;
     }
 };
 
@@ -526,15 +545,20 @@ private:
                       const std::vector<int>* replay_active, ReplayFrame* replay_out);
     DevBuf<unsigned char> d_enabled_;  // the replay's contacts among the candidates
     // baseline forward (phd_baseline.cpp)
-    double baseline_energy(const double* q);
-    void baseline_force(const double* q, double* f);
+    double baseline_energy(const double* q, const double* res, double* rr);
+    void baseline_force(double* f);
+    // dir = the L-BFGS direction of gradient g (pairs sh, yh: indices into d_bl_,
+    // oldest first); tmp: scratch
+    void lbfgs_direction(const std::deque<int>& sh, const std::deque<int>& yh, const double* g, double* tmp, double* dir,
+                         const std::vector<int>& frozen);
     void ainv64(const double* r, double* x);
     void pd_lhs_solve(const double* r, double* x, const std::vector<int>& frozen);
     int pd_nonlinear_solve(const double* q_init, double inv_h2m, const double* rhs, const std::vector<int>& frozen,
                            const std::vector<double>& frozen_vals, const std::map<std::string, double>& opt,
                            double* q_sol);
     std::map<int, int> zcol_;                  // frozen node -> column of d_Z_ (A^-1 e_node)
-    DevBuf<double> d_Z_, d_bl_energy_, d_bl_mu_;
+    DevBuf<double> d_Z_, d_bl_energy_, d_bl_mu_, d_bl_coef_;
+    PinBuf pin_energy_;
     DevBuf<int> d_bl_zcol_, d_bl_nodes_, d_bl_fix_;
     DevBuf<double> d_bl_fixv_;
     std::vector<int> g_frozen_;                // frozen set of the factored G below
