@@ -52,7 +52,9 @@ public:
 
 private:
     void pack(hipStream_t s);
-    void grad_pass(hipStream_t s, int nrows, const float* feat, const float* target, const int* idx, float loss_scale);
+    // loss_part: one partial loss per 16 rows
+    void grad_pass(hipStream_t s, int nrows, const float* feat, const float* target, const int* idx, float loss_scale,
+                   float* loss_part);
     bool ready_ = false;
     int step_ = 0;
     DevBuf<float> master_, m_, v_, grad_, partial_, loss_part_;
