@@ -129,25 +129,34 @@ __device__ __forceinline__ void row_solve(TV (&z)[CB], const TV (*Lt)[kTSB], con
     }
 }
 
-// S[l][row] = M(r0 + row, c0 + l) for the 64 x 64 block at (r0, c0); 256
-// threads, all loads in flight before the LDS stores.
 constexpr int kTS = CB + 4;  // LDS tile row stride (16-byte aligned rows)
+
+// The 64 x 64 block at (r0, c0) into registers (256 threads, all loads in flight), and
+// from there into LDS as S[l][row] = M(r0 + row, c0 + l).
+template <class TV>
+__device__ __forceinline__ void load_block(const TV* __restrict__ M, int64_t lda, int64_t r0, int64_t c0,
+                                           TV (&v)[CB * CB / 256]) {
+#pragma unroll
+    for (int u = 0; u < CB * CB / 256; ++u) {
+        const int e = (int)threadIdx.x + 256 * u;
+        v[u] = M[r0 + e % CB + (c0 + e / CB) * lda];
+    }
+}
+template <class TV>
+__device__ __forceinline__ void store_block(const TV (&v)[CB * CB / 256], TV (*S)[kTS]) {
+#pragma unroll
+    for (int u = 0; u < CB * CB / 256; ++u) {
+        const int e = (int)threadIdx.x + 256 * u;
+        S[e / CB][e % CB] = v[u];
+    }
+}
 
 template <class TV>
 __device__ __forceinline__ void stage_block(const TV* __restrict__ M, int64_t lda, int64_t r0, int64_t c0,
                                             TV (*S)[kTS]) {
-    const int t = threadIdx.x;
     TV v[CB * CB / 256];
-#pragma unroll
-    for (int u = 0; u < CB * CB / 256; ++u) {
-        const int e = t + 256 * u;
-        v[u] = M[r0 + e % CB + (c0 + e / CB) * lda];
-    }
-#pragma unroll
-    for (int u = 0; u < CB * CB / 256; ++u) {
-        const int e = t + 256 * u;
-        S[e / CB][e % CB] = v[u];
-    }
+    load_block<TV>(M, lda, r0, c0, v);
+    store_block<TV>(v, S);
 }
 
 // FP64 rank-64 tile product: acc[u][v] = sum_l A[l][4 tx + u] B[l][4 ty + v], l
@@ -293,43 +302,95 @@ __device__ __forceinline__ void row_trail_mfma(float (&z)[CB], const float (*Lt)
     }
 }
 
-// Rank-64 update of step kp on block (ib, jb): A_ij -= L_{i,kp} L_{j,kp}^T
-// (256 threads; the staging tiles are S0 and S1).
+// Updates of steps kp0 .. kp1 - 1 on block (ib, jb), in step order: A_ij -= L_{i,kp}
+// L_{j,kp}^T (256 threads; the staging tiles are S0 and S1). The block is read and
+// written once for all of them. FP64, with two workgroups per CU, loads the next
+// step's operands during the product; FP32 has four to overlap and no registers left.
 template <class TV>
-__device__ __forceinline__ void update_block(TV* __restrict__ M, int64_t lda, int kp, int ib, int jb, TV (*S0)[kTS],
+__device__ __forceinline__ void update_block(TV* __restrict__ M, int64_t lda, int kp0, int kp1, int ib, int jb, TV (*S0)[kTS],
                                              TV (*S1)[kTS]) {
     const int t = threadIdx.x;
+    const int64_t ri = (int64_t)ib * CB, rj = (int64_t)jb * CB;
     if constexpr (std::is_same<TV, float>::value) {
-        // the target block is read together with the staging loads, so its
-        // latency overlaps theirs instead of following the product
         const int lane = t % 64, wave = t / 64;
-        float* dst = M + (int64_t)ib * CB + 32 * (wave >> 1) + (lane & 31) + ((int64_t)jb * CB + 32 * (wave & 1)) * lda;
-        float old[16];
+        float* dst = M + ri + 32 * (wave >> 1) + (lane & 31) + (rj + 32 * (wave & 1)) * lda;
+        float val[16];
 #pragma unroll
-        for (int v = 0; v < 16; ++v) old[v] = dst[mfma_col(v, lane) * lda];
-        stage_block<TV>(M, lda, (int64_t)ib * CB, (int64_t)kp * CB, S0);
-        stage_block<TV>(M, lda, (int64_t)jb * CB, (int64_t)kp * CB, S1);
-        __syncthreads();
-        const f32x16 acc = tile_product_mfma(S0, S1, wave, lane);
+        for (int v = 0; v < 16; ++v) val[v] = dst[mfma_col(v, lane) * lda];
+#pragma unroll 1
+        for (int kp = kp0; kp < kp1; ++kp) {
+            stage_block<TV>(M, lda, ri, (int64_t)kp * CB, S0);
+            stage_block<TV>(M, lda, rj, (int64_t)kp * CB, S1);
+            __syncthreads();
+            const f32x16 acc = tile_product_mfma(S0, S1, wave, lane);
 #pragma unroll
-        for (int v = 0; v < 16; ++v) dst[mfma_col(v, lane) * lda] = old[v] - acc[v];
+            for (int v = 0; v < 16; ++v) val[v] -= acc[v];
+            if (kp + 1 < kp1) __syncthreads();
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) dst[mfma_col(v, lane) * lda] = val[v];
     } else {
         const int tx = t % 16, ty = t / 16;
-        TV* dst = M + (int64_t)ib * CB + 4 * tx + ((int64_t)jb * CB + 4 * ty) * lda;
-        TV old[4][4], acc[4][4];
+        TV a[CB * CB / 256], b[CB * CB / 256];
+        load_block<TV>(M, lda, ri, (int64_t)kp0 * CB, a);
+        load_block<TV>(M, lda, rj, (int64_t)kp0 * CB, b);
+        TV* dst = M + ri + 4 * tx + (rj + 4 * ty) * lda;
+        TV val[4][4], acc[4][4];
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) old[u][v] = dst[u + v * lda];
-        stage_block<TV>(M, lda, (int64_t)ib * CB, (int64_t)kp * CB, S0);
-        stage_block<TV>(M, lda, (int64_t)jb * CB, (int64_t)kp * CB, S1);
-        __syncthreads();
-        tile_product(S0, S1, tx, ty, acc);
+            for (int u = 0; u < 4; ++u) val[u][v] = dst[u + v * lda];
+#pragma unroll 1
+        for (int kp = kp0; kp < kp1; ++kp) {
+            store_block<TV>(a, S0);
+            store_block<TV>(b, S1);
+            __syncthreads();
+            if (kp + 1 < kp1) {
+                load_block<TV>(M, lda, ri, (int64_t)(kp + 1) * CB, a);
+                load_block<TV>(M, lda, rj, (int64_t)(kp + 1) * CB, b);
+            }
+            tile_product(S0, S1, tx, ty, acc);
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) val[u][v] -= acc[u][v];
+            if (kp + 1 < kp1) __syncthreads();
+        }
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) dst[u + v * lda] = old[u][v] - acc[u][v];
+            for (int u = 0; u < 4; ++u) dst[u + v * lda] = val[u][v];
     }
+}
+
+// Trailing updates of one launch. Every block (i, j) takes the steps 0 .. j - 2 in
+// order before the panel of column j (which applies step j - 1 itself). They come in
+// groups of kGroup steps, so that a trailing block is read and written once per group
+// and not once per step (which bound the launches with many blocks: 45 us against the
+// panel's 14 at 95 block columns in FP32). Launch k = g + r, g the group's first step:
+//  * due now: r = 0: the previous group's steps on the columns g + 1 .. g + kGroup;
+//    r > 0: the steps g .. k - 1 on column k + 1;
+//  * due before launch g + kGroup: the previous group's steps on the columns beyond,
+//    the r-th of kGroup equal shares.
+constexpr int kGroup = 4;
+
+struct TrailPart {
+    int ndue, nlazy, lazy0;  // blocks due now, blocks of this launch's share and the first of them
+};
+__host__ __device__ inline int column_blocks(int T, int j0, int j1) {  // blocks (i, j), j0 <= j < j1, j <= i <= T
+    return j1 <= j0 ? 0 : (j1 - j0) * (T + 1) - (j0 + j1 - 1) * (j1 - j0) / 2;
+}
+__host__ __device__ inline TrailPart trail_part(int k, int T) {
+    const int r = k % kGroup, g = k - r;
+    TrailPart p{0, 0, 0};
+    if (r > 0) p.ndue = k + 1 < T ? column_blocks(T, k + 1, k + 2) : 0;
+    else if (k > 0) p.ndue = column_blocks(T, k + 1, k + 1 + kGroup < T ? k + 1 + kGroup : T);
+    if (g > 0) {
+        const int n = column_blocks(T, g + kGroup + 1, T);
+        p.lazy0 = (int)((int64_t)n * r / kGroup);
+        p.nlazy = (int)((int64_t)n * (r + 1) / kGroup) - p.lazy0;
+    }
+    return p;
 }
 
 // The FP64 panel in LDS: D the diagonal block, R the block row (or the identity), both
@@ -418,8 +479,8 @@ __device__ __forceinline__ void panel64(double (*D)[kTS], double (*R)[kTS], doub
 }
 
 // Step k of the factorization, one launch of 256-thread workgroups in two parts
-// that touch disjoint blocks, so the panel of step k runs next to the trailing
-// update of step k - 1:
+// that touch disjoint blocks, so the panel of step k runs next to trailing updates
+// of earlier steps:
 //  * workgroups w < T - k + 1 (panel of block column k): the rank-64 update of
 //    step k - 1 is applied here, in LDS, to the two blocks the workgroup
 //    reads: the diagonal block (k, k) (every workgroup repeats it) and block
@@ -432,8 +493,8 @@ __device__ __forceinline__ void panel64(double (*D)[kTS], double (*R)[kTS], doub
 //    solves against them one sub-block behind, and the rank-16 update of the
 //    columns to the right follows (FP32 as MFMA tiles of the same two waves,
 //    FP64 see panel64);
-//  * the remaining workgroups apply the update of step k - 1 to the blocks
-//    (i, j) with k < j <= i <= T.
+//  * the remaining workgroups apply trailing updates (trail_part), none of them of
+//    step k or to column k.
 // Four workgroups per CU in FP32 (the MFMA accumulators stay in VGPRs, so the
 // update workgroups of a step run at four waves per SIMD), two in FP64, whose staging
 // tiles allow no more.
@@ -448,9 +509,18 @@ __global__ void __launch_bounds__(256, sizeof(TV) == 8 ? 2 : 4) k_chol_step(int 
     const int NP = T - k + 1;
     const int kp = k - 1;
     if ((int)blockIdx.x >= NP) {
-        int u = (int)blockIdx.x - NP, jb = k + 1, cnt = T - jb + 1;
-        while (u >= cnt) { u -= cnt; ++jb; cnt = T - jb + 1; }
-        update_block<TV>(M, lda, kp, jb + u, jb, S0, S1);
+        const TrailPart p = trail_part(k, T);
+        const int rr = k % kGroup, g = k - rr;
+        int u = (int)blockIdx.x - NP, jb, kp0 = g - kGroup, kp1 = g;
+        if (u < p.ndue) {
+            jb = k + 1;
+            if (rr > 0) { kp0 = g; kp1 = k; }
+        } else {
+            u += p.lazy0 - p.ndue;
+            jb = g + kGroup + 1;
+        }
+        for (int cnt = T - jb + 1; u >= cnt; cnt = T - jb + 1) { u -= cnt; ++jb; }
+        update_block<TV>(M, lda, kp0, kp1, jb + u, jb, S0, S1);
         return;
     }
     const int w = blockIdx.x;
@@ -686,9 +756,8 @@ void launch_chol_solve(hipStream_t s, int n, TV* M, TV* work, TV* x, int* fail) 
     TV* y = work;
     TV* Xinv = work + np;
     for (int k = 0; k < T; ++k) {
-        // update blocks of step k - 1 left to the second part: columns k + 1 .. T - 1, rows j .. T
-        const int nu = k == 0 ? 0 : (T - k) * (T - k + 1) / 2 - 1;
-        hipLaunchKernelGGL(k_chol_step<TV>, dim3(T - k + 1 + nu), dim3(256), 0, s, k, T, lda, M, Xinv, fail);
+        const TrailPart p = trail_part(k, T);
+        hipLaunchKernelGGL(k_chol_step<TV>, dim3(T - k + 1 + p.ndue + p.nlazy), dim3(256), 0, s, k, T, lda, M, Xinv, fail);
     }
     hipLaunchKernelGGL(k_chol_gety<TV>, dim3((np + 255) / 256), dim3(256), 0, s, np, lda, (const TV*)M, y);
     for (int b0 = kBsGroup * ((T - 1) / kBsGroup); b0 >= 0; b0 -= kBsGroup)
