@@ -313,13 +313,37 @@ void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w) {
         }
         tile_unit_ptr[t + 1] = (int)cu_tile.size();
     }
+    int fine_items = unit_items;
+    auto count = [&](int h) {
+        size_t c = 0;
+        for (int t = 0; t < ntiles; ++t)
+            c += (cu_i1[tile_unit_ptr[t + 1] - 1] - cu_i0[tile_unit_ptr[t]] + h - 1) / h;
+        return c;
+    };
+    while (fine_items > 64 && count(fine_items) < 4096) fine_items /= 2;
+    fu_tile.clear(); fu_i0.clear(); fu_i1.clear(); tile_fine_ptr.clear();
+    if (fine_items < unit_items) {
+        tile_fine_ptr.assign(ntiles + 1, 0);
+        for (int t = 0; t < ntiles; ++t) {
+            const int i0 = cu_i0[tile_unit_ptr[t]], i1 = cu_i1[tile_unit_ptr[t + 1] - 1];
+            for (int a = i0; a < i1; a += fine_items) {
+                fu_tile.push_back(t);
+                fu_i0.push_back(a);
+                fu_i1.push_back(std::min(i1, a + fine_items));
+            }
+            tile_fine_ptr[t + 1] = (int)fu_tile.size();
+        }
+    }
     // S w by row groups x column chunks; per-(row, chunk) partial slots, contiguous per row
-    gu_group.clear(); gu_chunk.clear();
-    const int ngroups = (n + kRowGroup - 1) / kRowGroup;
-    for (int g = 0; g < ngroups; ++g) {
-        int lo = n, hi = -1;
-        for (int k = g * kRowGroup; k < std::min(n, (g + 1) * kRowGroup); ++k) { lo = std::min(lo, f.fd[k]); hi = std::max(hi, k); }
-        for (int c = lo / chunk_w; c <= hi / chunk_w; ++c) { gu_group.push_back(g); gu_chunk.push_back(c); }
+    for (row_group = 64;; row_group /= 4) {
+        gu_group.clear(); gu_chunk.clear();
+        const int ngroups = (n + row_group - 1) / row_group;
+        for (int g = 0; g < ngroups; ++g) {
+            int lo = n, hi = -1;
+            for (int k = g * row_group; k < std::min(n, (g + 1) * row_group); ++k) { lo = std::min(lo, f.fd[k]); hi = std::max(hi, k); }
+            for (int c = lo / chunk_w; c <= hi / chunk_w; ++c) { gu_group.push_back(g); gu_chunk.push_back(c); }
+        }
+        if (row_group == 4 || gu_group.size() >= (row_group == 64 ? 2048 : 256)) break;
     }
     rbase.assign(n + 1, 0);
     for (int k = 0; k < n; ++k) rbase[k + 1] = rbase[k] + (k / chunk_w - f.fd[k] / chunk_w + 1);
@@ -330,7 +354,7 @@ void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w) {
     std::vector<int64_t> work(nu, 0);
     for (size_t u = 0; u < nu; ++u) {
         const int g = gu_group[u], c0 = gu_chunk[u] * chunk_w, c1 = c0 + chunk_w - 1;
-        for (int k = g * kRowGroup; k < std::min(n, (g + 1) * kRowGroup); ++k)
+        for (int k = g * row_group; k < std::min(n, (g + 1) * row_group); ++k)
             work[u] += std::max(0, std::min(k, c1) - std::max(f.fd[k], c0) + 1);
     }
     std::vector<size_t> ord(nu);
@@ -393,7 +417,7 @@ void host_factor_check(int n, const std::vector<int>& Ap, const std::vector<int>
     for (size_t u = 0; u < plan.gu_group.size(); ++u) {
         const int g = plan.gu_group[u], ch = plan.gu_chunk[u];
         const int c0 = ch * plan.chunk_w, c1 = c0 + plan.chunk_w - 1;
-        for (int k = g * SpmvPlan::kRowGroup; k < std::min(n, (g + 1) * SpmvPlan::kRowGroup); ++k) {
+        for (int k = g * plan.row_group; k < std::min(n, (g + 1) * plan.row_group); ++k) {
             const int lo = std::max(f.fd[k], c0), hi = std::min(k, c1);
             if (lo > hi) continue;
             const int slot = plan.rbase[k] + ch - f.fd[k] / plan.chunk_w;
@@ -408,15 +432,27 @@ void host_factor_check(int n, const std::vector<int>& Ap, const std::vector<int>
             ypl[k] += pslot[s];
         }
     for (int j = 0; j < n; ++j) { double s = 0; for (int k = j; k < n; ++k) s += S(k, j) * yref[k]; xref[j] = s; }
-    for (size_t u = 0; u < plan.cu_tile.size(); ++u) {
-        const int t = plan.cu_tile[u];
-        for (int it = plan.cu_i0[u]; it < plan.cu_i1[u]; ++it) {
-            const int k = plan.items[it];
-            for (int l = 0; l < 64; ++l) {
-                const int j = 64 * t + l;
-                if (j < n && j >= f.fd[k] && j <= k) xpl[j] += V[f.base[k] + j] * yref[k];
+    auto cols = [&](const std::vector<int>& tile, const std::vector<int>& i0, const std::vector<int>& i1, std::vector<double>& x) {
+        for (size_t u = 0; u < tile.size(); ++u) {
+            const int t = tile[u];
+            for (int it = i0[u]; it < i1[u]; ++it) {
+                const int k = plan.items[it];
+                for (int l = 0; l < 64; ++l) {
+                    const int j = 64 * t + l;
+                    if (j < n && j >= f.fd[k] && j <= k) x[j] += V[f.base[k] + j] * yref[k];
+                }
             }
         }
+    };
+    cols(plan.cu_tile, plan.cu_i0, plan.cu_i1, xpl);
+    if (!plan.fu_tile.empty()) {
+        std::vector<double> xfl(n, 0.0);
+        cols(plan.fu_tile, plan.fu_i0, plan.fu_i1, xfl);
+        for (size_t t = 0; t + 1 < plan.tile_fine_ptr.size(); ++t)
+            for (int u = plan.tile_fine_ptr[t]; u < plan.tile_fine_ptr[t + 1]; ++u)
+                if (plan.fu_tile[u] != (int)t) viol += 1;
+        for (int j = 0; j < n; ++j)
+            if (std::fabs(xfl[j] - xref[j]) > std::fabs(xpl[j] - xref[j])) xpl[j] = xfl[j];
     }
     double e1 = 0, e2 = 0;
     for (int k = 0; k < n; ++k) { e1 = std::max(e1, std::fabs(ypl[k] - yref[k])); e2 = std::max(e2, std::fabs(xpl[k] - xref[k])); }

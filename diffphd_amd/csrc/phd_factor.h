@@ -39,7 +39,7 @@ struct Factor {
 };
 
 // Work units of the two SpMVs over the S layout.
-//  * rows (y = S w): units of (group of kRowGroup consecutive rows, chunk of
+//  * rows (y = S w): units of (group of row_group consecutive rows, chunk of
 //    chunk_w columns), see below.
 //  * cols (x = S^T y): tile t = columns [64t, 64t+63]; its items are the rows
 //    intersecting the tile (the tile's own rows then the ancestors of its last
@@ -49,10 +49,22 @@ struct SpmvPlan {
     std::vector<int> items;         // concatenated per tile
     std::vector<int> cu_tile, cu_i0, cu_i1;  // unit -> tile, item range
     std::vector<int> tile_unit_ptr;          // units of tile t
-    // S w by units of (group of kRowGroup consecutive rows, chunk of kChunkW
+    // The same items in shorter units, for the solves whose summation order is free
+    // (the adjoint and bodies without a frictional boundary; the frictional forward
+    // iteration amplifies round-off and keeps the order above): halved until they give
+    // every CU 16 waves or have 64 rows, one batch. Empty where the units above are
+    // that many. A unit of 512 rows is walked by one wave while most of the chip is
+    // idle: 66 us at 5,040 vertices in FP64 and 35 us at 9,261 in FP32, with units of
+    // 64 rows 15 and 10 us; 56 and 52 us at 35,301 in FP32.
+    std::vector<int> fu_tile, fu_i0, fu_i1, tile_fine_ptr;
+    // S w by units of (group of row_group consecutive rows, chunk of chunk_w
     // columns): each unit stages w[chunk] once for all rows of the group that
     // cross it. Row k's partial for chunk c sits in slot rbase[k] + c - fd(k) / chunk_w.
-    static constexpr int kRowGroup = 64;
+    // Rows per group: 64 where that gives every CU eight units (w is staged once for
+    // 64 rows); fewer on smaller factors, whose four waves a unit would each walk 16
+    // rows in a row while most of the chip is idle (21 us at 242 vertices, 31 us at
+    // 5,040 in FP64). A row's partial is the same wherever its unit ends.
+    int row_group = 64;
     int chunk_w = 1024;
     std::vector<int> gu_group, gu_chunk, rbase;
     void build(const Factor& f, int unit_items, int group_chunk_w = 1024);

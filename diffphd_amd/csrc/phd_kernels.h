@@ -59,12 +59,12 @@ void launch_expand_s(hipStream_t s, int n, int t_begin, int t_end, const int64_t
                      const int* parent, const int* depth, const int* fd, const int64_t* base, const unsigned char* chain,
                      double* ws, int64_t ws_stride, double* V64, float* V32);
 
-// S w by (64-row group, chunk_w-column chunk) units with w staged in LDS; the
+// S w by (row_group-row group, chunk_w-column chunk) units with w staged in LDS; the
 // per-(row, chunk) partials are then summed per row (plan: SpmvPlan::gu_*, rbase,
 // built for the same chunk_w, one of kSpmvChunks).
 constexpr int kSpmvChunks[3] = {512, 1024, 2048};
 template <class TV>
-void launch_spmv_rows_grp(hipStream_t s, int nunits, const int* gu_group, const int* gu_chunk, const int* fd,
+void launch_spmv_rows_grp(hipStream_t s, int nunits, int row_group, const int* gu_group, const int* gu_chunk, const int* fd,
                           const int64_t* base, const int* rbase, const TV* V, const TV* w, int n, TV* pslot, int chunk_w);
 template <class TV>
 void launch_spmv_rows_slots(hipStream_t s, int n, const int* rbase, const TV* pslot, TV* y);
@@ -72,9 +72,10 @@ template <class TV>
 void launch_spmv_cols(hipStream_t s, int nunits, const int* cu_tile, const int* cu_i0, const int* cu_i1, const int* items,
                       const int* fd, const int64_t* base, const TV* V, const TV* y, int n, TV* xpart);
 // out[3 perm[j] + d] = (add ? add[...] : 0) + sum of tile partials; vertices with dmask set keep dval.
+// fine: the partials of the fine units, which are many per tile.
 template <class TV>
 void launch_spmv_cols_fin(hipStream_t s, int n, const int* tile_unit_ptr, const TV* xpart, const int* perm,
-                          const double* add, const unsigned char* dmask, const double* dval, double* out);
+                          const double* add, const unsigned char* dmask, const double* dval, double* out, bool fine = false);
 // w[d * n + j] = r[3 perm[j] + d] (SoA, postorder), zero at dmask vertices.
 template <class TV>
 void launch_perm_in(hipStream_t s, int n, const int* perm, const double* r, const unsigned char* dmask, TV* w);
@@ -162,7 +163,6 @@ void launch_iter_combine(hipStream_t s, int n, bool fwd, const AAHist& h, const 
                          double* gram_out, const double* x_prev, double* x, const unsigned char* fix, const double* fixval,
                          const double* pd_rhs, double* pd_prev, double* out);
 
-// ---- explicit inverse of small systems (phd_small.hip) -------------------------
 // L-BFGS direction of the baseline in one workgroup per loop, for vectors of up to
 // kLbfgsEntries and kLbfgsMax pairs (oldest first): beyond about 32,000 entries one
 // CU's reads of the pairs cost what the launches and round trips of many blocks do.
@@ -177,6 +177,7 @@ struct LbfgsHist {
 void launch_lbfgs_first(hipStream_t s, int n, const LbfgsHist& h, const double* g, double* q, double* coef);
 void launch_lbfgs_second(hipStream_t s, int n, const LbfgsHist& h, const double* coef, double* d);
 
+// ---- explicit inverse of small systems (phd_small.hip) -------------------------
 // out (n x ld, zero-filled by the caller past column n) = S^T S in vertex order;
 // items[item_ptr[t] .. item_ptr[t + 1]): the rows of S that cross column tile t
 template <class TV>

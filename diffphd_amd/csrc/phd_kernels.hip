@@ -121,7 +121,7 @@ template <> struct Vec16<float> { using type = float4; static constexpr int N = 
 template <> struct Vec16<double> { using type = double2; static constexpr int N = 2; };
 
 // -----------------------------------------------------------------------------
-// y = S w by (group of 64 consecutive rows, chunk of CW columns) units: the
+// y = S w by (group of 4 rpw consecutive rows, chunk of CW columns) units: the
 // workgroup stages w on the chunk in LDS once, then its four waves stream the
 // rows of the group that cross the chunk (16-byte vectors, the whole chunk in
 // flight per row) against it. Row k's dot product on the chunk goes to its
@@ -129,7 +129,7 @@ template <> struct Vec16<double> { using type = double2; static constexpr int N 
 // one of kSpmvChunks (picked by the autotuner; the plan is built for it).
 // -----------------------------------------------------------------------------
 template <class TV, int CW>
-__global__ void __launch_bounds__(256) k_spmv_rows_grp(int nunits, const int* __restrict__ gu_group,
+__global__ void __launch_bounds__(256) k_spmv_rows_grp(int nunits, int rpw, const int* __restrict__ gu_group,
                                                        const int* __restrict__ gu_chunk, const int* __restrict__ fd,
                                                        const int64_t* __restrict__ base, const int* __restrict__ rbase,
                                                        const TV* __restrict__ V, const TV* __restrict__ w, int n,
@@ -161,17 +161,17 @@ __global__ void __launch_bounds__(256) k_spmv_rows_grp(int nunits, const int* __
         }
     __syncthreads();
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
-    // the metadata of this wave's 16 rows (64 g + wv + 4 l), one row per lane,
+    // the metadata of this wave's rpw (at most 16) rows 4 rpw g + wv + 4 l, one row per lane,
     // loaded together so that each row waits on one memory round trip
     int mf = 0, mrb = 0;
     int64_t mb = 0;
     {
-        const int kk = 64 * g + wv + 4 * lane;
-        if (lane < 16 && kk < n) { mf = fd[kk]; mb = base[kk]; mrb = rbase[kk]; }
+        const int kk = 4 * rpw * g + wv + 4 * lane;
+        if (lane < rpw && kk < n) { mf = fd[kk]; mb = base[kk]; mrb = rbase[kk]; }
     }
     // row l's values are loaded one row ahead of its FMAs and reduction
-    const int k0 = 64 * g + wv;
-    const int nr = k0 >= n ? 0 : min(16, (n - k0 + 3) / 4);
+    const int k0 = 4 * rpw * g + wv;
+    const int nr = k0 >= n ? 0 : min(rpw, (n - k0 + 3) / 4);
     auto bounds = [&](int l, int& f, int& lo, int& hi) {
         f = __builtin_amdgcn_readlane(mf, l);
         lo = max(f, c0);
@@ -268,10 +268,20 @@ __global__ void __launch_bounds__(256) k_spmv_rows_slots(int n, const int* __res
 // x = S^T y: one wavefront per (tile, item range) unit. A row of the tile is
 // 64 columns = 64 / VN lanes of 16-byte vectors, so one load instruction
 // covers VN rows (lane sub-group `sub`); four such loads are in flight. The
-// item metadata of 64 rows is loaded cooperatively (one row per lane) and
-// broadcast with cross-lane reads. The sub-group partial sums are reduced at
-// the end.
+// metadata of 64 rows (row, first column, base, y) is loaded one row per lane. FP32,
+// with four rows a load, broadcasts it with cross-lane reads. FP64 has half the rows
+// per load and nine cross-lane reads a row, which bound it (182 us where the 472 MB of
+// 29,469 vertices take 92 at 5.1 TB/s): it publishes the metadata in LDS, two or three
+// broadcast reads a row, and has the next group's loads in flight during the products
+// (92 us). The same in FP32 is no faster on large factors and 50 instead of 35 us at
+// 9,261 vertices. The sub-group partial sums are reduced at the end.
 // -----------------------------------------------------------------------------
+template <class TV> struct __align__(16) ColMeta {
+    int k, f;       // row (-1: none) and its first column
+    long long b;    // its base
+    TV y[4];        // y on the three axes
+};
+
 template <class TV>
 __global__ void __launch_bounds__(256) k_spmv_cols(int nunits, const int* __restrict__ cu_tile,
                                                    const int* __restrict__ cu_i0, const int* __restrict__ cu_i1,
@@ -282,9 +292,9 @@ __global__ void __launch_bounds__(256) k_spmv_cols(int nunits, const int* __rest
     constexpr int VN = Vec16<TV>::N;
     constexpr int LPR = WAVE / VN;  // lanes per row
     constexpr int U = 4;
-    const int u = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
+    const int u = blockIdx.x * 4 + threadIdx.x / WAVE;
     const int lane = threadIdx.x % WAVE;
-    if (u >= nunits) return;
+    if (u >= nunits) return;  // whole waves; no barrier below
     const int t = cu_tile[u];
     const int sub = lane / LPR, g = lane % LPR;
     const int jb = 64 * t + VN * g;
@@ -292,51 +302,120 @@ __global__ void __launch_bounds__(256) k_spmv_cols(int nunits, const int* __rest
     TV acc0[VN], acc1[VN], acc2[VN];
 #pragma unroll
     for (int e = 0; e < VN; ++e) acc0[e] = acc1[e] = acc2[e] = 0;
-    for (int it0 = i0; it0 < i1; it0 += WAVE) {
-        const int my = it0 + lane;
-        const int cnt = min(WAVE, i1 - it0);
-        int mk = -1, mf = 0x7fffffff;
-        int mblo = 0, mbhi = 0;
-        TV my0 = 0, my1 = 0, my2 = 0;
-        if (my < i1) {
-            mk = items[my];
-            mf = fd[mk];
-            const int64_t b = base[mk];
-            mblo = (int)(b & 0xffffffff);
-            mbhi = (int)(b >> 32);
-            my0 = y[mk];
-            my1 = y[n + mk];
-            my2 = y[2 * n + mk];
+    if constexpr (sizeof(TV) == 4) {
+        for (int it0 = i0; it0 < i1; it0 += WAVE) {
+            const int my = it0 + lane;
+            const int cnt = min(WAVE, i1 - it0);
+            int mk = -1, mf = 0x7fffffff;
+            int mblo = 0, mbhi = 0;
+            TV my0 = 0, my1 = 0, my2 = 0;
+            if (my < i1) {
+                mk = items[my];
+                mf = fd[mk];
+                const int64_t b = base[mk];
+                mblo = (int)(b & 0xffffffff);
+                mbhi = (int)(b >> 32);
+                my0 = y[mk];
+                my1 = y[n + mk];
+                my2 = y[2 * n + mk];
+            }
+            for (int q = 0; q < cnt; q += VN * U) {
+                TV v[U][VN];
+                TV ys0[U], ys1[U], ys2[U];
+                int kk[U], ff[U];
+#pragma unroll
+                for (int s = 0; s < U; ++s) {
+                    const int src = q + s * VN + sub;
+                    kk[s] = __shfl(mk, src, WAVE);
+                    ff[s] = __shfl(mf, src, WAVE);
+                    const int64_t bb = ((int64_t)__shfl(mbhi, src, WAVE) << 32) | (uint32_t)__shfl(mblo, src, WAVE);
+                    ys0[s] = __shfl(my0, src, WAVE);
+                    ys1[s] = __shfl(my1, src, WAVE);
+                    ys2[s] = __shfl(my2, src, WAVE);
+                    V16 tv;
+                    if (src < cnt) tv = *reinterpret_cast<const V16*>(V + bb + jb);
+                    else memset(&tv, 0, sizeof(tv));
+                    memcpy(v[s], &tv, sizeof(tv));
+                    if (src >= cnt) kk[s] = -1;
+                }
+#pragma unroll
+                for (int s = 0; s < U; ++s)
+#pragma unroll
+                    for (int e = 0; e < VN; ++e) {
+                        const int j = jb + e;
+                        const TV vv = (j >= ff[s] && j <= kk[s]) ? v[s][e] : TV(0);
+                        acc0[e] += vv * ys0[s];
+                        acc1[e] += vv * ys1[s];
+                        acc2[e] += vv * ys2[s];
+                    }
+            }
         }
-        for (int q = 0; q < cnt; q += VN * U) {
-            TV v[U][VN];
-            TV ys0[U], ys1[U], ys2[U];
-            int kk[U], ff[U];
+    } else {
+        constexpr int GPB = WAVE / (VN * U);  // groups per batch of 64 rows
+        __shared__ ColMeta<TV> sm[4][2][WAVE];
+        ColMeta<TV>(*const mine)[WAVE] = sm[threadIdx.x / WAVE];
+        auto fetch = [&](int it) {
+            ColMeta<TV> m{-1, 0x7fffffff, 0, {TV(0), TV(0), TV(0), TV(0)}};
+            if (it + lane < i1) {
+                m.k = items[it + lane];
+                m.f = fd[m.k];
+                m.b = base[m.k];
+                m.y[0] = y[m.k];
+                m.y[1] = y[n + m.k];
+                m.y[2] = y[2 * n + m.k];
+            }
+            return m;
+        };
+        auto publish = [&](const ColMeta<TV>& m, int buf) {
+            mine[buf][lane] = m;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        };
+        auto issue = [&](const ColMeta<TV>* m, int q, TV (&v)[U][VN]) {
 #pragma unroll
             for (int s = 0; s < U; ++s) {
-                const int src = q + s * VN + sub;
-                kk[s] = __shfl(mk, src, WAVE);
-                ff[s] = __shfl(mf, src, WAVE);
-                const int64_t bb = ((int64_t)__shfl(mbhi, src, WAVE) << 32) | (uint32_t)__shfl(mblo, src, WAVE);
-                ys0[s] = __shfl(my0, src, WAVE);
-                ys1[s] = __shfl(my1, src, WAVE);
-                ys2[s] = __shfl(my2, src, WAVE);
+                const ColMeta<TV>& r = m[(q * U + s) * VN + sub];
                 V16 tv;
-                if (src < cnt) tv = *reinterpret_cast<const V16*>(V + bb + jb);
+                if (r.k >= 0) tv = *reinterpret_cast<const V16*>(V + r.b + jb);
                 else memset(&tv, 0, sizeof(tv));
                 memcpy(v[s], &tv, sizeof(tv));
-                if (src >= cnt) kk[s] = -1;
             }
+        };
+        auto use = [&](const ColMeta<TV>* m, int q, const TV (&v)[U][VN]) {
 #pragma unroll
-            for (int s = 0; s < U; ++s)
+            for (int s = 0; s < U; ++s) {
+                const ColMeta<TV>& r = m[(q * U + s) * VN + sub];
 #pragma unroll
                 for (int e = 0; e < VN; ++e) {
                     const int j = jb + e;
-                    const TV vv = (j >= ff[s] && j <= kk[s]) ? v[s][e] : TV(0);
-                    acc0[e] += vv * ys0[s];
-                    acc1[e] += vv * ys1[s];
-                    acc2[e] += vv * ys2[s];
+                    const TV vv = (j >= r.f && j <= r.k) ? v[s][e] : TV(0);
+                    acc0[e] += vv * r.y[0];
+                    acc1[e] += vv * r.y[1];
+                    acc2[e] += vv * r.y[2];
                 }
+            }
+        };
+        TV va[U][VN], vb[U][VN];
+        publish(fetch(i0), 0);
+        ColMeta<TV> nxt = fetch(i0 + WAVE);
+        issue(mine[0], 0, va);
+        int buf = 0;
+#pragma unroll 1
+        for (int it = i0; it < i1; it += WAVE, buf ^= 1) {
+            publish(nxt, buf ^ 1);
+            nxt = fetch(it + 2 * WAVE);
+            // rolled, two groups a turn: unrolled, a whole batch's metadata is read first
+            // and takes 160 to 250 registers
+#pragma unroll 1
+            for (int q = 0; q < GPB; q += 2) {
+                issue(mine[buf], q + 1, vb);
+                use(mine[buf], q, va);
+                __builtin_amdgcn_sched_barrier(0);
+                const bool last = q + 2 == GPB;
+                issue(mine[last ? buf ^ 1 : buf], last ? 0 : q + 2, va);
+                use(mine[buf], q + 1, vb);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
     }
 #pragma unroll
@@ -358,21 +437,35 @@ __global__ void __launch_bounds__(256) k_spmv_cols(int nunits, const int* __rest
     }
 }
 
-template <class TV>
-__global__ void k_spmv_cols_fin(int n, const int* __restrict__ tile_unit_ptr, const TV* __restrict__ xpart,
-                                const int* __restrict__ perm, const double* __restrict__ add,
-                                const unsigned char* __restrict__ dmask, const double* __restrict__ dval,
-                                double* __restrict__ out) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const int t = j / WAVE, lane = j % WAVE;
+// Sum of a tile's unit partials, W waves per tile taking every W-th unit.
+template <class TV, int W>
+__global__ void __launch_bounds__(256) k_spmv_cols_fin(int n, const int* __restrict__ tile_unit_ptr,
+                                                       const TV* __restrict__ xpart, const int* __restrict__ perm,
+                                                       const double* __restrict__ add, const unsigned char* __restrict__ dmask,
+                                                       const double* __restrict__ dval, double* __restrict__ out) {
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
+    const int t = blockIdx.x * (4 / W) + wave / W;
+    const int j = t * WAVE + lane;
     double a0 = 0, a1 = 0, a2 = 0;
-    for (int u = tile_unit_ptr[t]; u < tile_unit_ptr[t + 1]; ++u) {
-        const TV* xp = xpart + (int64_t)u * 3 * WAVE;
-        a0 += (double)xp[lane];
-        a1 += (double)xp[WAVE + lane];
-        a2 += (double)xp[2 * WAVE + lane];
+    if (t * WAVE < n) {
+#pragma unroll 4
+        for (int u = tile_unit_ptr[t] + wave % W; u < tile_unit_ptr[t + 1]; u += W) {
+            const TV* xp = xpart + (int64_t)u * 3 * WAVE;
+            a0 += (double)xp[lane];
+            a1 += (double)xp[WAVE + lane];
+            a2 += (double)xp[2 * WAVE + lane];
+        }
     }
+    if constexpr (W > 1) {
+        __shared__ double sh[W - 1][3][WAVE];
+        static_assert(W == 4, "one tile per workgroup");
+        if (wave > 0) { sh[wave - 1][0][lane] = a0; sh[wave - 1][1][lane] = a1; sh[wave - 1][2][lane] = a2; }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < W - 1; ++w) { a0 += sh[w][0][lane]; a1 += sh[w][1][lane]; a2 += sh[w][2][lane]; }
+    }
+    if (j >= n) return;
     const int v = perm[j];
     if (dmask && dmask[v]) {
         out[3 * v] = dval[3 * v];
@@ -1632,20 +1725,20 @@ void launch_expand_s(hipStream_t s, int n, int t_begin, int t_end, const int64_t
 }
 
 template <class TV>
-void launch_spmv_rows_grp(hipStream_t s, int nunits, const int* gu_group, const int* gu_chunk, const int* fd,
+void launch_spmv_rows_grp(hipStream_t s, int nunits, int row_group, const int* gu_group, const int* gu_chunk, const int* fd,
                           const int64_t* base, const int* rbase, const TV* V, const TV* w, int n, TV* pslot, int chunk_w) {
     if (nunits == 0) return;
     switch (chunk_w) {
     case 512:
-        hipLaunchKernelGGL((k_spmv_rows_grp<TV, 512>), dim3(nunits), dim3(256), 0, s, nunits, gu_group, gu_chunk, fd, base,
+        hipLaunchKernelGGL((k_spmv_rows_grp<TV, 512>), dim3(nunits), dim3(256), 0, s, nunits, row_group / 4, gu_group, gu_chunk, fd, base,
                            rbase, V, w, n, pslot);
         break;
     case 1024:
-        hipLaunchKernelGGL((k_spmv_rows_grp<TV, 1024>), dim3(nunits), dim3(256), 0, s, nunits, gu_group, gu_chunk, fd, base,
+        hipLaunchKernelGGL((k_spmv_rows_grp<TV, 1024>), dim3(nunits), dim3(256), 0, s, nunits, row_group / 4, gu_group, gu_chunk, fd, base,
                            rbase, V, w, n, pslot);
         break;
     case 2048:
-        hipLaunchKernelGGL((k_spmv_rows_grp<TV, 2048>), dim3(nunits), dim3(256), 0, s, nunits, gu_group, gu_chunk, fd, base,
+        hipLaunchKernelGGL((k_spmv_rows_grp<TV, 2048>), dim3(nunits), dim3(256), 0, s, nunits, row_group / 4, gu_group, gu_chunk, fd, base,
                            rbase, V, w, n, pslot);
         break;
     default:
@@ -1665,9 +1758,13 @@ void launch_spmv_cols(hipStream_t s, int nunits, const int* cu_tile, const int* 
 }
 template <class TV>
 void launch_spmv_cols_fin(hipStream_t s, int n, const int* tile_unit_ptr, const TV* xpart, const int* perm,
-                          const double* add, const unsigned char* dmask, const double* dval, double* out) {
-    hipLaunchKernelGGL(k_spmv_cols_fin<TV>, dim3(blocks_for(n, 256)), dim3(256), 0, s, n, tile_unit_ptr, xpart, perm, add,
-                       dmask, dval, out);
+                          const double* add, const unsigned char* dmask, const double* dval, double* out, bool fine) {
+    if (fine)
+        hipLaunchKernelGGL((k_spmv_cols_fin<TV, 4>), dim3(blocks_for(n, WAVE)), dim3(256), 0, s, n, tile_unit_ptr, xpart, perm,
+                           add, dmask, dval, out);
+    else
+        hipLaunchKernelGGL((k_spmv_cols_fin<TV, 1>), dim3(blocks_for(n, 256)), dim3(256), 0, s, n, tile_unit_ptr, xpart, perm,
+                           add, dmask, dval, out);
 }
 template <class TV>
 void launch_perm_in(hipStream_t s, int n, const int* perm, const double* r, const unsigned char* dmask, TV* w) {
@@ -1675,13 +1772,13 @@ void launch_perm_in(hipStream_t s, int n, const int* perm, const double* r, cons
 }
 
 #define PHD_INST_TV(TV)                                                                                                  \
-    template void launch_spmv_rows_grp<TV>(hipStream_t, int, const int*, const int*, const int*, const int64_t*,       \
+    template void launch_spmv_rows_grp<TV>(hipStream_t, int, int, const int*, const int*, const int*, const int64_t*,       \
                                            const int*, const TV*, const TV*, int, TV*, int);                           \
     template void launch_spmv_rows_slots<TV>(hipStream_t, int, const int*, const TV*, TV*);                          \
     template void launch_spmv_cols<TV>(hipStream_t, int, const int*, const int*, const int*, const int*, const int*,    \
                                        const int64_t*, const TV*, const TV*, int, TV*);                                  \
     template void launch_spmv_cols_fin<TV>(hipStream_t, int, const int*, const TV*, const int*, const double*,          \
-                                           const unsigned char*, const double*, double*);                                \
+                                           const unsigned char*, const double*, double*, bool);                          \
     template void launch_perm_in<TV>(hipStream_t, int, const int*, const double*, const unsigned char*, TV*);           \
     template void launch_contact_gather<TV>(hipStream_t, const ContactPieces&, const int*, const TV*, const TV*, int,      \
                                             double*, double*);                                                         \

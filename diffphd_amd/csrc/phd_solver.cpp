@@ -1438,7 +1438,7 @@ void Body::build_partial_dirichlet() {
         hip_check(hipStreamSynchronize(stream_), "pdir");
         d_r_.upload(e);
         spmv_S<double>(d_r_.p, w64_, y64_, part64_, V64_.p);
-        spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, d_tmp_.p);
+        spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, d_tmp_.p, false);
         launch_pdir_columns(stream_, nv_, p0, na, d_tmp_.p, d_pZ_.p);
     }
     hip_check(hipStreamSynchronize(stream_), "pdir columns");
@@ -1518,8 +1518,15 @@ void Body::upload_plan() {
     d_cu_i0_.upload(plan_.cu_i0);
     d_cu_i1_.upload(plan_.cu_i1);
     d_tile_unit_ptr_.upload(plan_.tile_unit_ptr);
+    if (!plan_.fu_tile.empty()) {
+        d_fu_tile_.upload(plan_.fu_tile);
+        d_fu_i0_.upload(plan_.fu_i0);
+        d_fu_i1_.upload(plan_.fu_i1);
+        d_tile_fine_ptr_.upload(plan_.tile_fine_ptr);
+    }
     part32_.alloc(3 * (size_t)plan_.rbase[nv_] + 3); part64_.alloc(3 * (size_t)plan_.rbase[nv_] + 3);
-    xpart32_.alloc(192 * plan_.cu_tile.size() + 192); xpart64_.alloc(192 * plan_.cu_tile.size() + 192);
+    const size_t nu = std::max(plan_.cu_tile.size(), plan_.fu_tile.size());
+    xpart32_.alloc(192 * nu + 192); xpart64_.alloc(192 * nu + 192);
 }
 
 void Body::set_launch_shapes(int chunk_w, int unit_items, int local_block) {
@@ -1561,7 +1568,7 @@ Body::TuneResult Body::autotune(double dt, int threads, int reps) {
         plan_.build(factor_, unit_items_, kTuneChunks[i]);
         upload_plan();
         res.rows_ms[i] = time_ms([&] {
-            launch_spmv_rows_grp<float>(stream_, (int)plan_.gu_group.size(), d_gu_group_.p, d_gu_chunk_.p, d_fd_.p,
+            launch_spmv_rows_grp<float>(stream_, (int)plan_.gu_group.size(), plan_.row_group, d_gu_group_.p, d_gu_chunk_.p, d_fd_.p,
                                         d_base_.p, d_rbase_.p, V32_.p, w32_.p, nv_, part32_.p, kTuneChunks[i]);
             launch_spmv_rows_slots<float>(stream_, nv_, d_rbase_.p, part32_.p, y32_.p);
         });
@@ -1607,20 +1614,27 @@ template <class TV>
 void Body::spmv_rows(DevBuf<TV>& w, DevBuf<TV>& y, DevBuf<TV>& part, const TV* V) {
     hipEvent_t a = nullptr, b = nullptr;
     if (timing) { a = next_event(); b = next_event(); (void)hipEventRecord(a, stream_); }
-    launch_spmv_rows_grp<TV>(stream_, (int)plan_.gu_group.size(), d_gu_group_.p, d_gu_chunk_.p, d_fd_.p, d_base_.p,
+    launch_spmv_rows_grp<TV>(stream_, (int)plan_.gu_group.size(), plan_.row_group, d_gu_group_.p, d_gu_chunk_.p, d_fd_.p, d_base_.p,
                              d_rbase_.p, V, w.p, nv_, part.p, chunk_w_);
     if (timing) { (void)hipEventRecord(b, stream_); ev_rows_.push_back({a, b}); }
     launch_spmv_rows_slots<TV>(stream_, nv_, d_rbase_.p, part.p, y.p);
 }
 
 template <class TV>
-void Body::spmv_ST(DevBuf<TV>& y, DevBuf<TV>& xpart, const TV* V, const double* add, const double* dval, double* out) {
+void Body::spmv_ST(DevBuf<TV>& y, DevBuf<TV>& xpart, const TV* V, const double* add, const double* dval, double* out,
+                   bool fine) {
+    fine = fine && !plan_.fu_tile.empty();
     hipEvent_t a = nullptr, b = nullptr;
     if (timing) { a = next_event(); b = next_event(); (void)hipEventRecord(a, stream_); }
-    launch_spmv_cols<TV>(stream_, (int)plan_.cu_tile.size(), d_cu_tile_.p, d_cu_i0_.p, d_cu_i1_.p, d_items_.p, d_fd_.p,
-                         d_base_.p, V, y.p, nv_, xpart.p);
+    if (fine)
+        launch_spmv_cols<TV>(stream_, (int)plan_.fu_tile.size(), d_fu_tile_.p, d_fu_i0_.p, d_fu_i1_.p, d_items_.p, d_fd_.p,
+                             d_base_.p, V, y.p, nv_, xpart.p);
+    else
+        launch_spmv_cols<TV>(stream_, (int)plan_.cu_tile.size(), d_cu_tile_.p, d_cu_i0_.p, d_cu_i1_.p, d_items_.p, d_fd_.p,
+                             d_base_.p, V, y.p, nv_, xpart.p);
     if (timing) { (void)hipEventRecord(b, stream_); ev_cols_.push_back({a, b}); }
-    launch_spmv_cols_fin<TV>(stream_, nv_, d_tile_unit_ptr_.p, xpart.p, d_perm_.p, add, dval ? d_dmask_.p : nullptr, dval, out);
+    launch_spmv_cols_fin<TV>(stream_, nv_, fine ? d_tile_fine_ptr_.p : d_tile_unit_ptr_.p, xpart.p, d_perm_.p, add,
+                             dval ? d_dmask_.p : nullptr, dval, out, fine);
 }
 
 template <class TV>
@@ -1776,7 +1790,7 @@ void Body::warm_start(const double* v, double dt, double inv_h2m, bool learned) 
         local_rhs(x, inv_h2m);
         launch_residual(stream_, nv_, ell_w_, d_Aie_.p, d_Axe_.p, d_b_.p, x, d_dmask_.p, d_r_.p, d_pmask_.p);
         spmv_S<double>(d_r_.p, w64_, y64_, part64_, V64_.p);
-        spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, d_tmp_.p);
+        spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, d_tmp_.p, false);
         rn[g] = std::sqrt(dots({{d_tmp_.p, d_tmp_.p}})[0]);
     }
     const int pick = (std::isfinite(rn[1]) && rn[1] < rn[0]) ? 1 : 0;
@@ -1824,10 +1838,10 @@ void Body::apply_ainv(double dt, const double* b, double* x, int precision, int 
         if (it > 0) launch_residual(stream_, nv_, ell_w_, d_Aie_.p, d_Axe_.p, d_b_.p, d_q_.p, nullptr, d_r_.p, d_pmask_.p);
         if (precision == 1) {
             spmv_S<float>(d_r_.p, w32_, y32_, part32_, V32_.p);
-            spmv_ST<float>(y32_, xpart32_, V32_.p, d_q_.p, nullptr, d_q_.p);
+            spmv_ST<float>(y32_, xpart32_, V32_.p, d_q_.p, nullptr, d_q_.p, false);
         } else {
             spmv_S<double>(d_r_.p, w64_, y64_, part64_, V64_.p);
-            spmv_ST<double>(y64_, xpart64_, V64_.p, d_q_.p, nullptr, d_q_.p);
+            spmv_ST<double>(y64_, xpart64_, V64_.p, d_q_.p, nullptr, d_q_.p, false);
         }
         // per-DOF Dirichlet rows are identities: x_F = b_F, the increment is 0 there
         partial_dirichlet(d_q_.p, it == 0 ? nullptr : d_b_.p, d_b_.p);
@@ -1844,7 +1858,7 @@ void Body::ainv64(const double* r, double* x) {
         return;
     }
     spmv_S<double>(r, w64_, y64_, part64_, V64_.p);
-    spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, x);
+    spmv_ST<double>(y64_, xpart64_, V64_.p, nullptr, nullptr, x, true);
 }
 
 // Scratch bytes apply_ainv_noalloc needs: w (3 ldw), y (3n), row-chunk partials,
@@ -1879,7 +1893,7 @@ void Body::ainv_passes(const double* b_dev, double* x_dev, int refine, char* scr
             rhs = r;
         }
         launch_perm_in<TV>(stream_, nv_, d_perm_.p, rhs, nullptr, w);
-        launch_spmv_rows_grp<TV>(stream_, (int)plan_.gu_group.size(), d_gu_group_.p, d_gu_chunk_.p, d_fd_.p, d_base_.p,
+        launch_spmv_rows_grp<TV>(stream_, (int)plan_.gu_group.size(), plan_.row_group, d_gu_group_.p, d_gu_chunk_.p, d_fd_.p, d_base_.p,
                                  d_rbase_.p, V, w, nv_, part, chunk_w_);
         launch_spmv_rows_slots<TV>(stream_, nv_, d_rbase_.p, part, y);
         launch_spmv_cols<TV>(stream_, (int)plan_.cu_tile.size(), d_cu_tile_.p, d_cu_i0_.p, d_cu_i1_.p, d_items_.p,
@@ -2309,8 +2323,8 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
         {
             PhaseTimer ts(this, kFwdSolve);
             if (dense) { /* the explicit inverse left x in d_q_ */ }
-            else if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_qprev_.p, d_dval_full_.p, d_q_.p);
-            else spmv_ST<double>(y64_, xpart64_, V64_.p, d_qprev_.p, d_dval_full_.p, d_q_.p);
+            else if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_qprev_.p, d_dval_full_.p, d_q_.p, K_ == 0);
+            else spmv_ST<double>(y64_, xpart64_, V64_.p, d_qprev_.p, d_dval_full_.p, d_q_.p, K_ == 0);
             partial_dirichlet(d_q_.p, d_qprev_.p, d_dval_full_.p);
         }
         ++iters;
@@ -2578,8 +2592,8 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
                 else contact_scatter<double>(d_dF_.p, y64_);
             }
             if (dense) { /* the explicit inverse left s in d_s */ }
-            else if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_sprev.p, d_zero.p, d_s.p);
-            else spmv_ST<double>(y64_, xpart64_, V64_.p, d_sprev.p, d_zero.p, d_s.p);
+            else if (precision == 1) spmv_ST<float>(y32_, xpart32_, V32_.p, d_sprev.p, d_zero.p, d_s.p, true);
+            else spmv_ST<double>(y64_, xpart64_, V64_.p, d_sprev.p, d_zero.p, d_s.p, true);
             partial_dirichlet(d_s.p, d_sprev.p, nullptr);
             // safe_clip (backward_gpu.cpp:809-816) before and after the Anderson
             // step: non-finite entries to 0, then |s| <= clip

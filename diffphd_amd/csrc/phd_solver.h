@@ -418,7 +418,8 @@ private:
     DevBuf<double> V64_;
     DevBuf<float> V32_;
     DevBuf<int64_t> d_base_;
-    DevBuf<int> d_fd_, d_perm_, d_items_, d_cu_tile_, d_cu_i0_, d_cu_i1_, d_tile_unit_ptr_, d_gu_group_, d_gu_chunk_,
+    DevBuf<int> d_fd_, d_perm_, d_items_, d_cu_tile_, d_cu_i0_, d_cu_i1_, d_tile_unit_ptr_, d_fu_tile_, d_fu_i0_, d_fu_i1_,
+        d_tile_fine_ptr_, d_gu_group_, d_gu_chunk_,
         d_rbase_;
     int ell_w_ = 0;            // A in ELL form: column / value of entry j of row v at j * nv + v
     DevBuf<int> d_Aie_;
@@ -503,7 +504,8 @@ private:
     template <class TV>
     void spmv_S(const double* r, DevBuf<TV>& w, DevBuf<TV>& y, DevBuf<TV>& part, const TV* V);
     template <class TV>
-    void spmv_ST(DevBuf<TV>& y, DevBuf<TV>& xpart, const TV* V, const double* add, const double* dval, double* out);
+    void spmv_ST(DevBuf<TV>& y, DevBuf<TV>& xpart, const TV* V, const double* add, const double* dval, double* out,
+                 bool fine);  // fine: the order of the sum is free (SpmvPlan::fu_*)
     template <class TV>
     void contact_gather(DevBuf<TV>& y, double* out);
     template <class TV>
