@@ -68,6 +68,7 @@ SIGNATURES = [
     ("phd_phase_times", ctypes.c_int, [_P, _dp, ctypes.c_int, ctypes.c_int]),
     ("phd_last_contact_multipliers", ctypes.c_int, [_P, _dp, _dp, _dp, ctypes.c_int]),
     ("phd_dense_spd_solve", ctypes.c_int, [ctypes.c_int, _dp, _dp, _dp, ctypes.c_int]),
+    ("phd_dense_spd_inverse", ctypes.c_int, [ctypes.c_int, _dp, _dp, ctypes.c_int]),
     ("phd_mlp_num_params", ctypes.c_int, []),
     ("phd_mlp_init", ctypes.c_int, [_P, ctypes.c_int]),
     ("phd_mlp_set_normalization", ctypes.c_int, [_P, _fp, _fp, ctypes.c_float]),

@@ -19,7 +19,7 @@ ARCH = os.environ.get("PHD_OFFLOAD_ARCH", "gfx950")
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wno-unused-command-line-argument", "-I" + os.path.join(HERE, "..", "include")]
-LIBS = ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-lpthread"]
+LIBS = ["-L/opt/rocm/lib", "-lrocblas", "-lpthread"]
 
 
 def _run(cmd):

@@ -370,6 +370,44 @@ int phd_dense_spd_solve(int n, const double* A, const double* b, double* x, int 
     }
 }
 
+int phd_dense_spd_inverse(int n, const double* A, double* X, int precision) {
+    try {
+        if (n <= 0) throw std::runtime_error("n must be positive");
+        const int np = phd::chol_padded(n);
+        const int64_t lda = phd::chol_inv_lda(n);
+        std::vector<double> L((size_t)lda * np, 0.0);
+        for (int c = 0; c < np; ++c) {
+            for (int r = c; r < np; ++r) L[r + (size_t)c * lda] = (r < n && c < n) ? A[r + (size_t)c * n] : (r == c ? 1.0 : 0.0);
+            L[np + c + (size_t)c * lda] = 1.0;
+        }
+        int fail = 0;
+        auto run = [&](auto tag) {
+            using TV = decltype(tag);
+            std::vector<TV> Lt(L.begin(), L.end()), xt((size_t)np * np);
+            phd::DevBuf<TV> dM, dX;
+            phd::DevBuf<int> df;
+            dM.upload(Lt);
+            dX.alloc((size_t)np * np);
+            df.alloc(1);
+            phd::launch_clear_flag(nullptr, df.p);
+            phd::launch_chol_inverse(nullptr, n, dM.p, dX.p, df.p);
+            phd::hip_check(hipDeviceSynchronize(), "dense inverse");
+            dX.download(xt.data(), xt.size());
+            df.download(&fail, 1);
+            for (int c = 0; c < np; ++c)
+                for (int r = 0; r < np; ++r) {
+                    if (r < n && c < n) X[r + (size_t)c * n] = (double)xt[r + (size_t)c * np];
+                    else if (!fail && xt[r + (size_t)c * np] != TV(0)) throw std::runtime_error("padding is not zero");
+                }
+        };
+        if (precision == 1) run(float{}); else run(double{});
+        return fail ? 1 : 0;
+    } catch (const std::exception& e) {
+        g_create_error = e.what();
+        return -1;
+    }
+}
+
 int phd_mlp_num_params(void) { return phd::MlpLayout::total; }
 
 int phd_mlp_init(phd_ctx ctx, int seed) {

@@ -39,6 +39,19 @@ void launch_chol_assemble(hipStream_t s, int nJ, const int* J, const TH* H, int 
 template <class TV>
 void launch_chol_solve(hipStream_t s, int n, TV* M, TV* work, TV* x, int* fail);
 
+// Inverse of a dense SPD matrix: G^-1 = Y Y^T with Y = L^-T, which the same
+// factorization forms from an identity below the matrix. Layout of M (column-major,
+// lda = chol_inv_lda(n) = 2 np, np columns): rows [0, np) the lower triangle of G,
+// identity on the padding; rows [np, 2 np) the identity. Gs (np x np, column-major)
+// gets the whole inverse, zero past n. *fail is set as by launch_chol_solve.
+inline int64_t chol_inv_lda(int n) { return 2 * (int64_t)chol_padded(n); }
+inline int64_t chol_inv_elems(int n) { return chol_inv_lda(n) * chol_padded(n); }
+template <class TV, class TS>
+void launch_chol_inverse(hipStream_t s, int n, TV* M, TS* Gs, int* fail);
+// Writes the basis Gram matrix G_ab = (d_a . d_b) H[cidx_a][cidx_b] into that layout.
+template <class TV>
+void launch_gram_assemble(hipStream_t s, int nb, const int* cidx, const double* dirs, const double* H, int K, TV* M);
+
 // Clears the failure flag with a kernel (safe inside captured graphs).
 void launch_clear_flag(hipStream_t s, int* flag);
 

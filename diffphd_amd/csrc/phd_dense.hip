@@ -19,9 +19,10 @@ __global__ void __launch_bounds__(256) k_chol_assemble(int nJ, int np, int64_t l
     const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= rows * np) return;
     const int r = (int)(idx % rows), c = (int)(idx / rows);
-    if (r < c) return;
     double v;
-    if (r >= np) {
+    if (r < c) {
+        v = 0.0;
+    } else if (r >= np) {
         v = (r == np && c < nJ) ? rhs[c] : 0.0;
     } else if (r >= nJ || c >= nJ) {
         v = (r == c) ? 1.0 : 0.0;
@@ -363,6 +364,11 @@ __device__ __forceinline__ void update_block(TV* __restrict__ M, int64_t lda, in
     }
 }
 
+// The rows below the matrix (block rows T, T + 1, ...) are either one right-hand-side
+// block row, or (INV) the identity, one block row per block column: L^-1 rhs and
+// Y = L^-T come out of the factorization there. Block row T + i of Y starts at
+// column i, so the updates of steps up to kp reach kp + 1 of its block rows.
+//
 // Trailing updates of one launch. Every block (i, j) takes the steps 0 .. j - 2 in
 // order before the panel of column j (which applies step j - 1 itself). They come in
 // groups of kGroup steps, so that a trailing block is read and written once per group
@@ -377,16 +383,18 @@ constexpr int kGroup = 4;
 struct TrailPart {
     int ndue, nlazy, lazy0;  // blocks due now, blocks of this launch's share and the first of them
 };
-__host__ __device__ inline int column_blocks(int T, int j0, int j1) {  // blocks (i, j), j0 <= j < j1, j <= i <= T
-    return j1 <= j0 ? 0 : (j1 - j0) * (T + 1) - (j0 + j1 - 1) * (j1 - j0) / 2;
+// blocks of the columns j0 <= j < j1: rows j .. T - 1 and `extra` rows below
+__host__ __device__ inline int column_blocks(int T, int extra, int j0, int j1) {
+    return j1 <= j0 ? 0 : (j1 - j0) * (T + extra) - (j0 + j1 - 1) * (j1 - j0) / 2;
 }
+template <bool INV>
 __host__ __device__ inline TrailPart trail_part(int k, int T) {
     const int r = k % kGroup, g = k - r;
     TrailPart p{0, 0, 0};
-    if (r > 0) p.ndue = k + 1 < T ? column_blocks(T, k + 1, k + 2) : 0;
-    else if (k > 0) p.ndue = column_blocks(T, k + 1, k + 1 + kGroup < T ? k + 1 + kGroup : T);
+    if (r > 0) p.ndue = k + 1 < T ? column_blocks(T, INV ? k : 1, k + 1, k + 2) : 0;
+    else if (k > 0) p.ndue = column_blocks(T, INV ? g : 1, k + 1, k + 1 + kGroup < T ? k + 1 + kGroup : T);
     if (g > 0) {
-        const int n = column_blocks(T, g + kGroup + 1, T);
+        const int n = column_blocks(T, INV ? g : 1, g + kGroup + 1, T);
         p.lazy0 = (int)((int64_t)n * r / kGroup);
         p.nlazy = (int)((int64_t)n * (r + 1) / kGroup) - p.lazy0;
     }
@@ -481,7 +489,7 @@ __device__ __forceinline__ void panel64(double (*D)[kTS], double (*R)[kTS], doub
 // Step k of the factorization, one launch of 256-thread workgroups in two parts
 // that touch disjoint blocks, so the panel of step k runs next to trailing updates
 // of earlier steps:
-//  * workgroups w < T - k + 1 (panel of block column k): the rank-64 update of
+//  * workgroups w < T - k + 1, INV w < T (panel of block column k): the rank-64 update of
 //    step k - 1 is applied here, in LDS, to the two blocks the workgroup
 //    reads: the diagonal block (k, k) (every workgroup repeats it) and block
 //    (k + 1 + w, k); w = T - k - 1 is the right-hand-side block row and
@@ -498,7 +506,7 @@ __device__ __forceinline__ void panel64(double (*D)[kTS], double (*R)[kTS], doub
 // Four workgroups per CU in FP32 (the MFMA accumulators stay in VGPRs, so the
 // update workgroups of a step run at four waves per SIMD), two in FP64, whose staging
 // tiles allow no more.
-template <class TV>
+template <class TV, bool INV>
 __global__ void __launch_bounds__(256, sizeof(TV) == 8 ? 2 : 4) k_chol_step(int k, int T, int64_t lda, TV* __restrict__ M,
                                                    TV* __restrict__ Xinv, int* __restrict__ fail) {
     __shared__ __align__(16) TV S0[CB][kTS];
@@ -506,10 +514,10 @@ __global__ void __launch_bounds__(256, sizeof(TV) == 8 ? 2 : 4) k_chol_step(int 
     __shared__ __align__(16) TV invp[CB];
     __shared__ __align__(16) TV Ls[sizeof(TV) == 8 ? 2 : 1][16][kLS];  // FP64 only
     const int t = threadIdx.x;
-    const int NP = T - k + 1;
+    const int NP = INV ? T : T - k + 1;
     const int kp = k - 1;
     if ((int)blockIdx.x >= NP) {
-        const TrailPart p = trail_part(k, T);
+        const TrailPart p = trail_part<INV>(k, T);
         const int rr = k % kGroup, g = k - rr;
         int u = (int)blockIdx.x - NP, jb, kp0 = g - kGroup, kp1 = g;
         if (u < p.ndue) {
@@ -519,14 +527,19 @@ __global__ void __launch_bounds__(256, sizeof(TV) == 8 ? 2 : 4) k_chol_step(int 
             u += p.lazy0 - p.ndue;
             jb = g + kGroup + 1;
         }
-        for (int cnt = T - jb + 1; u >= cnt; cnt = T - jb + 1) { u -= cnt; ++jb; }
+        const int extra = INV ? kp1 : 1;
+        for (int cnt = T - jb + extra; u >= cnt; cnt = T - jb + extra) { u -= cnt; ++jb; }
+        // a block row of Y takes no part in the steps before its first column
+        if (INV && jb + u >= T) kp0 = max(kp0, jb + u - T);
         update_block<TV>(M, lda, kp0, kp1, jb + u, jb, S0, S1);
         return;
     }
     const int w = blockIdx.x;
     const int wave = t / 64, r = t % 64;
     const int role = wave < 2 ? wave : 2;
-    const bool has_row = w < T - k;          // block row k + 1 + w of M (else the identity)
+    // block row k + 1 + w of M, which INV continues with the first k + 1 of Y; without
+    // INV the last workgroup has the identity instead
+    const bool has_row = INV || w < T - k;
     const int64_t c0 = (int64_t)k * CB, i0 = (int64_t)(k + 1 + w) * CB;
     if constexpr (std::is_same<TV, double>::value) {
         const int ux = t % 16, uy = t / 16;
@@ -756,14 +769,131 @@ void launch_chol_solve(hipStream_t s, int n, TV* M, TV* work, TV* x, int* fail) 
     TV* y = work;
     TV* Xinv = work + np;
     for (int k = 0; k < T; ++k) {
-        const TrailPart p = trail_part(k, T);
-        hipLaunchKernelGGL(k_chol_step<TV>, dim3(T - k + 1 + p.ndue + p.nlazy), dim3(256), 0, s, k, T, lda, M, Xinv, fail);
+        const TrailPart p = trail_part<false>(k, T);
+        hipLaunchKernelGGL((k_chol_step<TV, false>), dim3(T - k + 1 + p.ndue + p.nlazy), dim3(256), 0, s, k, T, lda, M, Xinv, fail);
     }
     hipLaunchKernelGGL(k_chol_gety<TV>, dim3((np + 255) / 256), dim3(256), 0, s, np, lda, (const TV*)M, y);
     for (int b0 = kBsGroup * ((T - 1) / kBsGroup); b0 >= 0; b0 -= kBsGroup)
         hipLaunchKernelGGL(k_chol_bsolve<TV>, dim3(b0 + 1), dim3(256), 0, s, b0, T, lda, (const TV*)M, (const TV*)Xinv, y,
                            x);
 }
+
+// Gs = Y Y^T (both triangles, zero past n) from the factor's rows [np, 2 np): block
+// (i, j), i >= j, is the sum over the block columns k >= i, one workgroup each. The
+// blocks of small i have the longest sums and come first. At 6,339 rows in FP32 the
+// factorization takes 3.4 ms and this product 1.0 (85 TFLOP/s), where the library's
+// factorization and inversion took 30.
+template <class TV, class TS>
+__global__ void __launch_bounds__(256, sizeof(TV) == 8 ? 2 : 4) k_chol_inverse_product(int n, int T, int64_t lda,
+                                                                                       const TV* __restrict__ M,
+                                                                                       TS* __restrict__ Gs) {
+    __shared__ __align__(16) TV S0[CB][kTS];
+    __shared__ __align__(16) TV S1[CB][kTS];
+    int ib = 0, jb = blockIdx.x;
+    // row of the packed lower triangle: ib (ib + 1) / 2 <= blockIdx.x
+    ib = (int)((sqrt(8.0 * jb + 1.0) - 1.0) * 0.5);
+    while ((int64_t)ib * (ib + 1) / 2 > jb) --ib;
+    while ((int64_t)(ib + 1) * (ib + 2) / 2 <= jb) ++ib;
+    jb -= (int)((int64_t)ib * (ib + 1) / 2);
+    const int t = threadIdx.x;
+    const int64_t yi = (int64_t)(T + ib) * CB, yj = (int64_t)(T + jb) * CB;
+    if constexpr (std::is_same<TV, float>::value) {
+        const int lane = t % 64, wave = t / 64;
+        float val[16];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) val[v] = 0.f;
+#pragma unroll 1
+        for (int kp = ib; kp < T; ++kp) {
+            stage_block<TV>(M, lda, yi, (int64_t)kp * CB, S0);
+            stage_block<TV>(M, lda, yj, (int64_t)kp * CB, S1);
+            __syncthreads();
+            const f32x16 acc = tile_product_mfma(S0, S1, wave, lane);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) val[v] += acc[v];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) S0[32 * (wave >> 1) + (lane & 31)][32 * (wave & 1) + mfma_col(v, lane)] = val[v];
+    } else {
+        const int tx = t % 16, ty = t / 16;
+        TV val[4][4], acc[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) val[u][v] = TV(0);
+#pragma unroll 1
+        for (int kp = ib; kp < T; ++kp) {
+            stage_block<TV>(M, lda, yi, (int64_t)kp * CB, S0);
+            stage_block<TV>(M, lda, yj, (int64_t)kp * CB, S1);
+            __syncthreads();
+            tile_product(S0, S1, tx, ty, acc);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) val[u][v] += acc[u][v];
+            __syncthreads();
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) S0[4 * tx + u][4 * ty + v] = val[u][v];
+    }
+    __syncthreads();
+    const int64_t ld = (int64_t)T * CB;
+    const int r = t % CB;
+    for (int c = t / CB; c < CB; c += 256 / CB) {
+        const int64_t ri = (int64_t)ib * CB, rj = (int64_t)jb * CB;
+        Gs[ri + r + (rj + c) * ld] = ri + r < n && rj + c < n ? (TS)S0[r][c] : TS(0);
+        if (ib != jb) Gs[rj + r + (ri + c) * ld] = rj + r < n && ri + c < n ? (TS)S0[c][r] : TS(0);
+    }
+}
+
+template <class TV, class TS>
+void launch_chol_inverse(hipStream_t s, int n, TV* M, TS* Gs, int* fail) {
+    const int T = chol_padded(n) / CB;
+    const int64_t lda = chol_inv_lda(n);
+    for (int k = 0; k < T; ++k) {
+        const TrailPart p = trail_part<true>(k, T);
+        hipLaunchKernelGGL((k_chol_step<TV, true>), dim3(T + p.ndue + p.nlazy), dim3(256), 0, s, k, T, lda, M, (TV*)nullptr,
+                           fail);
+    }
+    hipLaunchKernelGGL((k_chol_inverse_product<TV, TS>), dim3(T * (T + 1) / 2), dim3(256), 0, s, n, T, lda, M, Gs);
+}
+template void launch_chol_inverse<float, float>(hipStream_t, int, float*, float*, int*);
+template void launch_chol_inverse<double, float>(hipStream_t, int, double*, float*, int*);
+template void launch_chol_inverse<double, double>(hipStream_t, int, double*, double*, int*);
+
+// M_ab = (d_a . d_b) H[cidx_a][cidx_b] in the layout of launch_chol_inverse
+template <class TV>
+__global__ void __launch_bounds__(256) k_gram_assemble(int nb, int np, int64_t lda, const int* __restrict__ cidx,
+                                                       const double* __restrict__ dirs, const double* __restrict__ H, int K,
+                                                       TV* __restrict__ M) {
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= lda * np) return;
+    const int r = (int)(idx % lda), c = (int)(idx / lda);
+    double v;
+    if (r < c) {
+        v = 0.0;
+    } else if (r >= np) {
+        v = r - np == c ? 1.0 : 0.0;
+    } else if (r >= nb) {
+        v = r == c ? 1.0 : 0.0;
+    } else {
+        const double dd = dirs[3 * c] * dirs[3 * r] + dirs[3 * c + 1] * dirs[3 * r + 1] + dirs[3 * c + 2] * dirs[3 * r + 2];
+        v = dd * H[(int64_t)cidx[c] * K + cidx[r]];
+    }
+    M[idx] = (TV)v;
+}
+
+template <class TV>
+void launch_gram_assemble(hipStream_t s, int nb, const int* cidx, const double* dirs, const double* H, int K, TV* M) {
+    const int np = chol_padded(nb);
+    const int64_t lda = chol_inv_lda(nb), total = lda * np;
+    hipLaunchKernelGGL(k_gram_assemble<TV>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, nb, np, lda, cidx, dirs, H,
+                       K, M);
+}
+template void launch_gram_assemble<float>(hipStream_t, int, const int*, const double*, const double*, int, float*);
+template void launch_gram_assemble<double>(hipStream_t, int, const int*, const double*, const double*, int, double*);
 
 void launch_clear_flag(hipStream_t s, int* flag) { hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(64), 0, s, flag); }
 

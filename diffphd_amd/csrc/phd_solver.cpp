@@ -16,7 +16,6 @@
 #include "phd_mlp.h"
 
 #include <rocblas/rocblas.h>
-#include <rocsolver/rocsolver.h>
 
 #include <algorithm>
 #include <chrono>
@@ -2541,7 +2540,7 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
 
     // Constrained solve data (Woodbury basis); nb == 0 means the plain backbone.
     int nb = 0;
-    DevBuf<double> d_G, d_Gx, d_dirs, d_Gs64;
+    DevBuf<double> d_Gx, d_dirs, d_Gs64;
     DevBuf<float> d_Gs32;  // G^-1 as a full symmetric matrix (leading dimension gld)
     int64_t gld = 0;
     DevBuf<int> d_bcidx, d_bcptr, d_bclist;  // basis row -> candidate; candidate -> its basis rows
@@ -2751,49 +2750,27 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
                 // so the iterates still converge onto J s = 0); FP64 when the FP32
                 // factor breaks down or with phd_gram32 = 0.
                 bool g32 = precision == 1 && opt_or(opt, "phd_gram32", 1.0) != 0.0;
+                auto invert = [&](auto& M, auto& Gs) {
+                    M.alloc((size_t)chol_inv_elems(nb));
+                    Gs.alloc((size_t)(gld * gld));
+                    launch_gram_assemble(stream_, nb, d_bcidx.p, d_dirs.p, d_H_.p, K_, M.p);
+                    launch_clear_flag(stream_, d_info_.p);
+                    launch_chol_inverse(stream_, nb, M.p, Gs.p, d_info_.p);
+                    hip_check(hipMemcpyAsync(&info, d_info_.p, sizeof(int), hipMemcpyDeviceToHost, stream_), "info");
+                    hip_check(hipStreamSynchronize(stream_), "basis inverse");
+                    return info == 0;
+                };
                 if (g32) {
                     DevBuf<float> dGf;
-                    dGf.alloc((size_t)nb * nb);
-                    launch_assemble_g<float>(stream_, nb, d_bcidx.p, d_dirs.p, d_H_.p, K_, dGf.p);
-                    check(rocsolver_spotrf((rocblas_handle)blas_, rocblas_fill_lower, nb, dGf.p, nb, d_info_.p) ==
-                              rocblas_status_success, "spotrf (basis) failed");
-                    hip_check(hipMemcpyAsync(&info, d_info_.p, sizeof(int), hipMemcpyDeviceToHost, stream_), "info");
-                    hip_check(hipStreamSynchronize(stream_), "basis factor");
-                    if (info == 0) {
-                        check(rocsolver_spotri((rocblas_handle)blas_, rocblas_fill_lower, nb, dGf.p, nb, d_info_.p) ==
-                                  rocblas_status_success, "spotri (basis) failed");
-                        hip_check(hipMemcpyAsync(&info, d_info_.p, sizeof(int), hipMemcpyDeviceToHost, stream_), "info");
-                        hip_check(hipStreamSynchronize(stream_), "basis inverse");
-                    }
-                    if (info == 0) {
-                        d_Gs32.alloc((size_t)(gld * gld));
-                        launch_sym_full<float, float>(stream_, nb, gld, dGf.p, d_Gs32.p);
-                        hip_check(hipStreamSynchronize(stream_), "basis sym");
-                    } else {
+                    if (!invert(dGf, d_Gs32)) {
                         g32 = false;
                         ++last_bwd.gram_fp64_fallbacks;
                     }
                 }
                 if (!g32) {
-                    d_G.alloc((size_t)nb * nb);
-                    launch_assemble_g<double>(stream_, nb, d_bcidx.p, d_dirs.p, d_H_.p, K_, d_G.p);
-                    check(rocsolver_dpotrf((rocblas_handle)blas_, rocblas_fill_lower, nb, d_G.p, nb, d_info_.p) ==
-                              rocblas_status_success, "dpotrf (basis) failed");
-                    hip_check(hipMemcpyAsync(&info, d_info_.p, sizeof(int), hipMemcpyDeviceToHost, stream_), "info");
-                    hip_check(hipStreamSynchronize(stream_), "basis factor");
-                    check(info == 0, "Contact basis Gram matrix is not positive definite.");
-                    check(rocsolver_dpotri((rocblas_handle)blas_, rocblas_fill_lower, nb, d_G.p, nb, d_info_.p) ==
-                              rocblas_status_success, "dpotri (basis) failed");
-                    hip_check(hipMemcpyAsync(&info, d_info_.p, sizeof(int), hipMemcpyDeviceToHost, stream_), "info");
-                    hip_check(hipStreamSynchronize(stream_), "basis inverse");
-                    check(info == 0, "Contact basis Gram matrix is singular.");
-                    if (precision == 1) {
-                        d_Gs32.alloc((size_t)(gld * gld));
-                        launch_sym_full<double, float>(stream_, nb, gld, d_G.p, d_Gs32.p);
-                    } else {
-                        d_Gs64.alloc((size_t)(gld * gld));
-                        launch_sym_full<double, double>(stream_, nb, gld, d_G.p, d_Gs64.p);
-                    }
+                    DevBuf<double> dG;
+                    check(precision == 1 ? invert(dG, d_Gs32) : invert(dG, d_Gs64),
+                          "Contact basis Gram matrix is not positive definite.");
                 }
                 d_Gx.alloc(nb);
                 tbf.reset();

@@ -251,6 +251,11 @@ int phd_last_contact_multipliers(phd_ctx ctx, double* lambda, double* lt1, doubl
  * Test entry point; no counterpart in the reference. */
 int phd_dense_spd_solve(int n, const double* A, const double* b, double* x, int precision);
 
+/* Inverse X (n x n column-major, host) of a dense SPD matrix through the same
+ * factorization, as the adjoint forms it for its contact basis; arguments and
+ * result as above. Test entry point; no counterpart in the reference. */
+int phd_dense_spd_inverse(int n, const double* A, double* X, int precision);
+
 /* ---- Learned warm start of the PD iteration (no counterpart in the reference:
  * its initial iterate is q_t, deformable_projective_dynamics_forward_gpu.cpp:1069).
  * A per-vertex MLP 13 -> 128 -> 128 -> 128 -> 3 (GELU, BF16 weights on MFMA,
