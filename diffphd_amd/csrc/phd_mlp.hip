@@ -81,115 +81,200 @@ __device__ inline float col_sum(const f32x4& d) {  // sum over the 16 rows of co
     return s;
 }
 
-// One hidden layer forward: z = A W + b (A from LDS), H = gelu(z) into LDS.
+// 16 rows of features into an LDS tile, 4 columns per lane, zero past nrows
+__device__ inline void load_features(int v0, int nrows, const float* __restrict__ feat, const int* __restrict__ idx,
+                                     uint16_t* X0, int lane) {
+    const int row = lane / 4, c = 4 * (lane % 4);
+    const int gr = v0 + row;
+    float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (gr < nrows) f = *reinterpret_cast<const float4*>(feat + (size_t)(idx ? idx[gr] : gr) * kMlpInPad + c);
+    X0[row * LDX + c] = f2bf(f.x);
+    X0[row * LDX + c + 1] = f2bf(f.y);
+    X0[row * LDX + c + 2] = f2bf(f.z);
+    X0[row * LDX + c + 3] = f2bf(f.w);
+}
+
+// One hidden layer forward: gelu(A W + b), A from LDS, into LDS
 template <int K>
-__device__ inline void layer_fwd(const uint16_t* A, int lda, const uint16_t* Wf, const float* b, uint16_t* Hout,
-                                 f32x4 (&z)[H / 16], int lane) {
+__device__ inline void layer_fwd(const uint16_t* A, int lda, const uint16_t* Wf, const float* b, uint16_t* Hout, int lane) {
+    bf16x4 a[K / 16];
+#pragma unroll
+    for (int ks = 0; ks < K / 16; ++ks) a[ks] = lds_a(A, lda, 16 * ks, lane);
 #pragma unroll
     for (int nt = 0; nt < H / 16; ++nt) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < K / 16; ++ks) acc = mfma(lds_a(A, lda, 16 * ks, lane), gl_b(Wf, K, 16 * nt, 16 * ks, lane), acc);
+        for (int ks = 0; ks < K / 16; ++ks) acc = mfma(a[ks], gl_b(Wf, K, 16 * nt, 16 * ks, lane), acc);
         const float bb = b[16 * nt + (lane & 15)];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[r] += bb;
-        z[nt] = acc;
         f32x4 h;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) h[r] = gelu(acc[r]);
+        for (int r = 0; r < 4; ++r) h[r] = gelu(acc[r] + bb);
         store_d(Hout, LDH, 16 * nt, lane, h);
     }
 }
 
-// Backward through a hidden layer given dz (D layout, 8 tiles): writes dW, db
-// into P and returns dA = dz W^T (D layout) for the layer below (if wanted).
-template <bool WANT_DA>
-__device__ inline void layer_bwd(const uint16_t* Ain, int lda, int kin, const f32x4 (&dz)[H / 16], const uint16_t* Wb,
-                                 uint16_t* G, float* P, int offW, int offb, f32x4 (&dA)[H / 16], int lane) {
-#pragma unroll
-    for (int bt = 0; bt < H / 16; ++bt) {
-        const float s = col_sum(dz[bt]);
-        if (lane < 16) P[offb + 16 * bt + lane] = s;
-    }
-    for (int a = 0; a < kin / 16; ++a) {
-        const bf16x4 at = lds_at(Ain, lda, 16 * a, lane);
-#pragma unroll
-        for (int bt = 0; bt < H / 16; ++bt) {
-            const f32x4 acc = mfma(at, d_as_b(dz[bt]), f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int r = 0; r < 4; ++r) P[offW + (16 * a + 4 * (lane >> 4) + r) * H + 16 * bt + (lane & 15)] = acc[r];
-        }
-    }
-    if (!WANT_DA) return;
-#pragma unroll
-    for (int bt = 0; bt < H / 16; ++bt) store_d(G, LDH, 16 * bt, lane, dz[bt]);
-    wave_sync();
-#pragma unroll
-    for (int it = 0; it < H / 16; ++it) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < H / 16; ++ks) acc = mfma(lds_a(G, LDH, 16 * ks, lane), gl_b(Wb, H, 16 * it, 16 * ks, lane), acc);
-        dA[it] = acc;
-    }
-    wave_sync();
-}
-
-// Forward (TRAIN = false: outputs) or forward + backward (TRAIN = true: per-wave
-// gradient partials and loss) of 16 rows per wavefront. Row r of the pass is
-// row idx[r] of feat / target (idx == nullptr: identity).
-template <bool TRAIN>
-__global__ void __launch_bounds__(256) k_mlp_pass(int nrows, const float* __restrict__ feat, const float* __restrict__ target,
-                                                  const int* __restrict__ idx, const uint16_t* __restrict__ wf,
-                                                  const uint16_t* __restrict__ wb, const float* __restrict__ master,
-                                                  float* __restrict__ out, float* __restrict__ partial,
-                                                  float* __restrict__ loss_part, float loss_scale) {
+// Inference: 16 rows per wavefront through the four layers, the hidden rows in place (a
+// layer's rows are in registers before its outputs are written): 20 KB of LDS let four
+// workgroups share a CU, where three tiles per wave left room for two (177 us at
+// 139,425 rows, now 153).
+__global__ void __launch_bounds__(256, 4) k_mlp_forward(int nrows, const float* __restrict__ feat,
+                                                     const uint16_t* __restrict__ wf, const float* __restrict__ master,
+                                                     float* __restrict__ out) {
     __shared__ __align__(16) uint16_t sX[WPB][16 * LDX];
-    __shared__ __align__(16) uint16_t sH[WPB][3][16 * LDH];
-    __shared__ __align__(16) uint16_t sG[WPB][16 * LDH];
+    __shared__ __align__(16) uint16_t sH[WPB][16 * LDH];
     const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
-    const int w = blockIdx.x * WPB + wv;
-    const int v0 = 16 * w;
+    const int v0 = 16 * (blockIdx.x * WPB + wv);
     if (v0 >= nrows) return;
     uint16_t* X0 = sX[wv];
-    uint16_t* H1 = sH[wv][0];
-    uint16_t* H2 = sH[wv][1];
-    uint16_t* H3 = sH[wv][2];
-    uint16_t* G = sG[wv];
-    {  // features: 16 rows x 16 columns, 4 per lane
-        const int row = lane / 4, c = 4 * (lane % 4);
-        const int gr = v0 + row;
-        float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (gr < nrows) f = *reinterpret_cast<const float4*>(feat + (size_t)(idx ? idx[gr] : gr) * kMlpInPad + c);
-        X0[row * LDX + c] = f2bf(f.x);
-        X0[row * LDX + c + 1] = f2bf(f.y);
-        X0[row * LDX + c + 2] = f2bf(f.z);
-        X0[row * LDX + c + 3] = f2bf(f.w);
-    }
+    uint16_t* Hs = sH[wv];
+    load_features(v0, nrows, feat, nullptr, X0, lane);
     wave_sync();
-    f32x4 z1[H / 16], z2[H / 16], z3[H / 16];
-    layer_fwd<kMlpInPad>(X0, LDX, wf + WO1, master + MlpLayout::b1, H1, z1, lane);
+    layer_fwd<kMlpInPad>(X0, LDX, wf + WO1, master + MlpLayout::b1, Hs, lane);
     wave_sync();
-    layer_fwd<H>(H1, LDH, wf + WO2, master + MlpLayout::b2, H2, z2, lane);
+    layer_fwd<H>(Hs, LDH, wf + WO2, master + MlpLayout::b2, Hs, lane);
     wave_sync();
-    layer_fwd<H>(H2, LDH, wf + WO3, master + MlpLayout::b3, H3, z3, lane);
+    layer_fwd<H>(Hs, LDH, wf + WO3, master + MlpLayout::b3, Hs, lane);
     wave_sync();
     f32x4 o = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int ks = 0; ks < H / 16; ++ks) o = mfma(lds_a(H3, LDH, 16 * ks, lane), gl_b(wf + WO4, H, 0, 16 * ks, lane), o);
+    for (int ks = 0; ks < H / 16; ++ks) o = mfma(lds_a(Hs, LDH, 16 * ks, lane), gl_b(wf + WO4, H, 0, 16 * ks, lane), o);
     const int col = lane & 15;
     const float b4 = master[MlpLayout::b4 + col];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] += b4;
-    if (!TRAIN) {
+    for (int r = 0; r < 4; ++r) {
+        const int gr = v0 + 4 * (lane >> 4) + r;
+        if (col < kMlpOut && gr < nrows) out[(size_t)gr * kMlpOut + col] = o[r] + b4;
+    }
+}
+
+// Training pass: 16 rows per workgroup, whose four waves take two of the eight
+// 16-column tiles of every layer each, forward and backward. A batch has far fewer
+// tiles of 16 rows than the chip has SIMDs, so what counts is the length of one tile's
+// chain: with one wave per tile, 1,100 dependent tile products, their weight loads and
+// the activations in a row, a batch of 4,096 took 76 us; here 28 us. The weights of
+// all layers are loaded at the start, while the features arrive.
+constexpr int NTW = H / 16 / 4;  // tiles per wave and layer
+template <int K>
+struct Frags {  // a wave's columns of a weight matrix as B fragments
+    bf16x4 f[NTW][K / 16];
+    __device__ inline void load(const uint16_t* W, int wv, int lane) {
+#pragma unroll
+        for (int j = 0; j < NTW; ++j)
+#pragma unroll
+            for (int ks = 0; ks < K / 16; ++ks) f[j][ks] = gl_b(W, K, 16 * (NTW * wv + j), 16 * ks, lane);
+    }
+};
+
+template <int K>
+__device__ inline void tile_fwd(const uint16_t* A, int lda, const Frags<K>& W, const float* b, uint16_t* Hout,
+                                f32x4 (&z)[NTW], int wv, int lane) {
+    f32x4 acc[NTW];
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < K / 16; ++ks) {
+        const bf16x4 a = lds_a(A, lda, 16 * ks, lane);
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) acc[j] = mfma(a, W.f[j][ks], acc[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) {
+        const int nt = NTW * wv + j;
+        const float bb = b[16 * nt + (lane & 15)];
+        f32x4 h;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int gr = v0 + 4 * (lane >> 4) + r;
-            if (col < kMlpOut && gr < nrows) out[(size_t)gr * kMlpOut + col] = o[r];
+            z[j][r] = acc[j][r] + bb;
+            h[r] = gelu(z[j][r]);
         }
-        return;
+        store_d(Hout, LDH, 16 * nt, lane, h);
     }
-    // ---- backward: loss = loss_scale * sum (o - t)^2 over valid rows, 3 outputs
-    float* P = partial + (size_t)w * MlpLayout::total;
+}
+
+// dW (the wave's columns) and db of a hidden layer, from its input rows and dz
+template <int KIN>
+__device__ inline void tile_grad(const uint16_t* Ain, int lda, const f32x4 (&dz)[NTW], float* P, int offW, int offb, int wv,
+                                 int lane) {
+    bf16x4 d[NTW];
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) {
+        const float s = col_sum(dz[j]);
+        if (lane < 16) P[offb + 16 * (NTW * wv + j) + lane] = s;
+        d[j] = d_as_b(dz[j]);
+    }
+#pragma unroll
+    for (int a = 0; a < KIN / 16; ++a) {
+        const bf16x4 at = lds_at(Ain, lda, 16 * a, lane);
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) {
+            const f32x4 acc = mfma(at, d[j], f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                P[offW + (16 * a + 4 * (lane >> 4) + r) * H + 16 * (NTW * wv + j) + (lane & 15)] = acc[r];
+        }
+    }
+}
+
+// dz of the layer below, in place of its z: (dz W^T) gelu'(z), dz through G
+__device__ inline void tile_back(uint16_t* G, const f32x4 (&dz)[NTW], const Frags<H>& W, f32x4 (&z)[NTW], int wv, int lane) {
+    __syncthreads();  // G is free
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) store_d(G, LDH, 16 * (NTW * wv + j), lane, dz[j]);
+    __syncthreads();
+    f32x4 acc[NTW];
+#pragma unroll
+    for (int j = 0; j < NTW; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < H / 16; ++ks) {
+        const bf16x4 a = lds_a(G, LDH, 16 * ks, lane);
+#pragma unroll
+        for (int j = 0; j < NTW; ++j) acc[j] = mfma(a, W.f[j][ks], acc[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < NTW; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[j][r] = acc[j][r] * gelu_d(z[j][r]);
+}
+
+// Per-tile gradient partials and loss of 16 rows per workgroup. Row r of the pass is
+// row idx[r] of feat / target (idx == nullptr: identity).
+__global__ void __launch_bounds__(256, 1) k_mlp_train(int nrows, const float* __restrict__ feat,
+                                                      const float* __restrict__ target, const int* __restrict__ idx,
+                                                      const uint16_t* __restrict__ wf, const uint16_t* __restrict__ wb,
+                                                      const float* __restrict__ master, float* __restrict__ partial,
+                                                      float* __restrict__ loss_part, float loss_scale) {
+    __shared__ __align__(16) uint16_t X0[16 * LDX];
+    __shared__ __align__(16) uint16_t H1[16 * LDH], H2[16 * LDH], H3[16 * LDH], G[16 * LDH];
+    const int lane = threadIdx.x % 64, wv = threadIdx.x / 64;
+    const int v0 = 16 * blockIdx.x;
+    if (wv == 0) load_features(v0, nrows, feat, idx, X0, lane);
+    Frags<kMlpInPad> w1;
+    Frags<H> w2, w3, b3, b2;
+    bf16x4 w4[H / 16];
+    Frags<kMlpOutPad> b4w;
+    w1.load(wf + WO1, wv, lane);
+    w2.load(wf + WO2, wv, lane);
+    w3.load(wf + WO3, wv, lane);
+#pragma unroll
+    for (int ks = 0; ks < H / 16; ++ks) w4[ks] = gl_b(wf + WO4, H, 0, 16 * ks, lane);
+    b4w.load(wb + WO4, wv, lane);
+    b3.load(wb + WO3, wv, lane);
+    b2.load(wb + WO2, wv, lane);
+    __syncthreads();
+    f32x4 z1[NTW], z2[NTW], z3[NTW];
+    tile_fwd<kMlpInPad>(X0, LDX, w1, master + MlpLayout::b1, H1, z1, wv, lane);
+    __syncthreads();
+    tile_fwd<H>(H1, LDH, w2, master + MlpLayout::b2, H2, z2, wv, lane);
+    __syncthreads();
+    tile_fwd<H>(H2, LDH, w3, master + MlpLayout::b3, H3, z3, wv, lane);
+    __syncthreads();
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};  // the output tile, by every wave
+#pragma unroll
+    for (int ks = 0; ks < H / 16; ++ks) o = mfma(lds_a(H3, LDH, 16 * ks, lane), w4[ks], o);
+    const int col = lane & 15;
+    const float b4 = master[MlpLayout::b4 + col];
+    // loss = loss_scale * sum (o - t)^2 over valid rows, 3 outputs
+    float* P = partial + (size_t)blockIdx.x * MlpLayout::total;
     f32x4 d4;
     float lsum = 0.f;
 #pragma unroll
@@ -197,49 +282,41 @@ __global__ void __launch_bounds__(256) k_mlp_pass(int nrows, const float* __rest
         const int gr = v0 + 4 * (lane >> 4) + r;
         float d = 0.f;
         if (col < kMlpOut && gr < nrows) {
-            const float e = o[r] - target[(size_t)(idx ? idx[gr] : gr) * kMlpOut + col];
+            const float e = o[r] + b4 - target[(size_t)(idx ? idx[gr] : gr) * kMlpOut + col];
             lsum += e * e;
             d = 2.f * loss_scale * e;
         }
         d4[r] = d;
     }
+    if (wv == 0) {
 #pragma unroll
-    for (int off = 32; off >= 1; off /= 2) lsum += __shfl_xor(lsum, off, 64);
-    if (lane == 0) loss_part[w] = lsum * loss_scale;
-    // layer 4: db4, dW4 = H3^T d4, dH3 = d4 W4^T
-    {
+        for (int off = 32; off >= 1; off /= 2) lsum += __shfl_xor(lsum, off, 64);
+        if (lane == 0) loss_part[blockIdx.x] = lsum * loss_scale;
         const float s = col_sum(d4);
         if (lane < 16) P[MlpLayout::b4 + lane] = s;
-#pragma unroll
-        for (int a = 0; a < H / 16; ++a) {
-            const f32x4 acc = mfma(lds_at(H3, LDH, 16 * a, lane), d_as_b(d4), f32x4{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int r = 0; r < 4; ++r) P[MlpLayout::W4 + (16 * a + 4 * (lane >> 4) + r) * kMlpOutPad + col] = acc[r];
-        }
         store_d(G, LDH, 0, lane, d4);
-        wave_sync();
-        f32x4 dh[H / 16];
-#pragma unroll
-        for (int it = 0; it < H / 16; ++it)
-            dh[it] = mfma(lds_a(G, LDH, 0, lane), gl_b(wb + WO4, kMlpOutPad, 16 * it, 0, lane), f32x4{0.f, 0.f, 0.f, 0.f});
-        wave_sync();
-#pragma unroll
-        for (int it = 0; it < H / 16; ++it)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) z3[it][r] = dh[it][r] * gelu_d(z3[it][r]);  // z3 now holds dz3
     }
-    f32x4 dA[H / 16];
-    layer_bwd<true>(H2, LDH, H, z3, wb + WO3, G, P, MlpLayout::W3, MlpLayout::b3, dA, lane);
+    // layer 4: dW4 = H3^T d4, dz3 = (d4 W4^T) gelu'(z3)
 #pragma unroll
-    for (int it = 0; it < H / 16; ++it)
+    for (int j = 0; j < NTW; ++j) {
+        const int a = NTW * wv + j;
+        const f32x4 acc = mfma(lds_at(H3, LDH, 16 * a, lane), d_as_b(d4), f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z2[it][r] = dA[it][r] * gelu_d(z2[it][r]);
-    layer_bwd<true>(H1, LDH, H, z2, wb + WO2, G, P, MlpLayout::W2, MlpLayout::b2, dA, lane);
+        for (int r = 0; r < 4; ++r) P[MlpLayout::W4 + (16 * a + 4 * (lane >> 4) + r) * kMlpOutPad + col] = acc[r];
+    }
+    __syncthreads();
 #pragma unroll
-    for (int it = 0; it < H / 16; ++it)
+    for (int j = 0; j < NTW; ++j) {
+        const f32x4 dh = mfma(lds_a(G, LDH, 0, lane), b4w.f[j][0], f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-        for (int r = 0; r < 4; ++r) z1[it][r] = dA[it][r] * gelu_d(z1[it][r]);
-    layer_bwd<false>(X0, LDX, kMlpInPad, z1, nullptr, G, P, MlpLayout::W1, MlpLayout::b1, dA, lane);
+        for (int r = 0; r < 4; ++r) z3[j][r] = dh[r] * gelu_d(z3[j][r]);
+    }
+    // the gradients of a layer are written while the next dz is on its way
+    tile_back(G, z3, b3, z2, wv, lane);
+    tile_grad<H>(H2, LDH, z3, P, MlpLayout::W3, MlpLayout::b3, wv, lane);
+    tile_back(G, z2, b2, z1, wv, lane);
+    tile_grad<H>(H1, LDH, z2, P, MlpLayout::W2, MlpLayout::b2, wv, lane);
+    tile_grad<kMlpInPad>(X0, LDX, z1, P, MlpLayout::W1, MlpLayout::b1, wv, lane);
 }
 
 // Position of a weight parameter in the BF16 copies (forward wo + out nin + in,
@@ -408,16 +485,15 @@ void WarmStartNet::forward(hipStream_t s, int n, const float* feat, float* out) 
     check(ready_, "warm-start network not initialized");
     if (n <= 0) return;
     const int nw = (n + 15) / 16;
-    hipLaunchKernelGGL(k_mlp_pass<false>, dim3((nw + WPB - 1) / WPB), dim3(64 * WPB), 0, s, n, feat, nullptr, nullptr,
-                       wf_.p, wb_.p, master_.p, out, nullptr, nullptr, 0.f);
+    hipLaunchKernelGGL(k_mlp_forward, dim3((nw + WPB - 1) / WPB), dim3(64 * WPB), 0, s, n, feat, wf_.p, master_.p, out);
 }
 
 void WarmStartNet::grad_pass(hipStream_t s, int nrows, const float* feat, const float* target, const int* idx,
                              float loss_scale, float* loss_part) {
     const int nw = (nrows + 15) / 16;
     if (partial_.n < (size_t)nw * MlpLayout::total) partial_.alloc((size_t)nw * MlpLayout::total);
-    hipLaunchKernelGGL(k_mlp_pass<true>, dim3((nw + WPB - 1) / WPB), dim3(64 * WPB), 0, s, nrows, feat, target, idx, wf_.p,
-                       wb_.p, master_.p, nullptr, partial_.p, loss_part, loss_scale);
+    hipLaunchKernelGGL(k_mlp_train, dim3(nw), dim3(256), 0, s, nrows, feat, target, idx, wf_.p, wb_.p, master_.p, partial_.p,
+                       loss_part, loss_scale);
 }
 
 double WarmStartNet::loss_grad(hipStream_t s, int n, const float* feat, const float* target, float* grad) {
