@@ -117,6 +117,7 @@ Body::Body(int device) : device_(device) {
     hip_check(hipSetDevice(device_), "hipSetDevice");
     scratch_ = scratch_address(device_);
     hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "hipStreamCreate");
+    hip_check(hipEventCreateWithFlags(&ev_iter_, hipEventDisableTiming), "hipEventCreate");
     hip_check(hipHostMalloc((void**)&pin_small_, kPinSmallBytes + kIterOut * sizeof(double),
                             hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
     rocblas_handle h;
@@ -129,6 +130,7 @@ Body::~Body() {
     if (pin_small_) (void)hipHostFree(pin_small_);
     for (auto e : ev_pool_) (void)hipEventDestroy(e);
     if (blas_) rocblas_destroy_handle((rocblas_handle)blas_);
+    if (ev_iter_) (void)hipEventDestroy(ev_iter_);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -1964,7 +1966,12 @@ struct DevAnderson {
 // the regularized least squares and replaces xnew by
 // xprev + g - sum gamma_a (dQ_a + dG_a). The host waits once, for the sums of
 // the convergence test and the restart flag that ride along.
-bool Body::iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew, double clip, double* sums, double* gg) {
+// ahead (may be empty) queues the part of the next iteration that leaves xnew as it is:
+// the device works on it while the host reads this iteration's sums, decides and queues
+// the rest. Without it the queue ran empty once per iteration, 25 us until its next kernel
+// started (9,261 vertices, traced), now 6.
+bool Body::iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew, double clip, double* sums, double* gg,
+                   const std::function<void()>& ahead) {
     const int n3 = dofs_;
     AAHist h;
     h.push = aa.window > 0 ? 1 : 0;
@@ -1993,7 +2000,13 @@ bool Body::iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew,
     launch_iter_combine(stream_, n3, fwd, h, d_iter_part_.p, d_aa_gram_[aa.gram_at].p, d_aa_gram_[1 - aa.gram_at].p, xprev,
                         xnew, d_fix_.p, d_dval_full_.p, d_pdrhs_.p, d_pdrhs_prev_.p, pin_iter());
     if (h.m > 0) aa.gram_at = 1 - aa.gram_at;
-    hip_check(hipStreamSynchronize(stream_), "iteration");
+    if (ahead) {
+        hip_check(hipEventRecord(ev_iter_, stream_), "iteration");
+        ahead();
+        hip_check(hipEventSynchronize(ev_iter_), "iteration");
+    } else {
+        hip_check(hipStreamSynchronize(stream_), "iteration");
+    }
     const double* out = pin_iter();
     const int rows = iter_rows(n3);
     for (int k = 0; k < (fwd ? 4 : 1); ++k) {
@@ -2215,25 +2228,34 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
     const int* const listP = lists + K;
     const int* const listF = lists + 2 * (size_t)K;
     const int* const listG = lists + 3 * (size_t)K;
-    for (int iter = 0; iter < max_pd_iter; ++iter) {
+    // local step, residual of the global system with the previous contact impulses and its
+    // solve, up to where q is written; q_prev = q
+    auto front = [&] {
         {
             PhaseTimer tl(this, kFwdLocal);
             launch_local_step(stream_, mat_, d_q_.p, d_elem_.p, local_block_, local_fp32_, K_ == 0);
         }
-        // residual of the global system with the previous contact impulses; q_prev = q
-        {
+        PhaseTimer ts(this, kFwdSolve);
+        const double* F = K > 0 ? d_F_.p : nullptr;
+        if (dense) {
+            iter_residual_dense(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, d_r_.p);
+        } else if (precision == 1) {
+            iter_residual<float>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w32_);
+            spmv_rows<float>(w32_, y32_, part32_, V32_.p);
+        } else {
+            iter_residual<double>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w64_);
+            spmv_rows<double>(w64_, y64_, part64_, V64_.p);
+        }
+    };
+    // The last iteration's front is for nothing: queued ahead where S is read in less than
+    // the 25 us that a turn of the loop gains. A mesh's restitution reads q_prev afterwards.
+    const bool run_ahead = !mesh && timing_level < 2 && (dense || (int64_t)factor_.v_len * (precision == 1 ? 4 : 8) < (int64_t)128 << 20);
+    bool queued = false;
+    for (int iter = 0; iter < max_pd_iter; ++iter) {
+        if (!queued) front();
+        if (dense) {
             PhaseTimer ts(this, kFwdSolve);
-            const double* F = K > 0 ? d_F_.p : nullptr;
-            if (dense) {
-                iter_residual_dense(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, d_r_.p);
-                dense_solve(precision, d_r_.p, d_qprev_.p, d_dval_full_.p, nullptr, d_q_.p);
-            } else if (precision == 1) {
-                iter_residual<float>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w32_);
-                spmv_rows<float>(w32_, y32_, part32_, V32_.p);
-            } else {
-                iter_residual<double>(true, d_qtilde_.p, d_q_.p, d_qprev_.p, inv_h2m, F, w64_);
-                spmv_rows<double>(w64_, y64_, part64_, V64_.p);
-            }
+            dense_solve(precision, d_r_.p, d_qprev_.p, d_dval_full_.p, nullptr, d_q_.p);
         }
         if (K > 0) {
             PhaseTimer tc(this, kFwdContact);
@@ -2331,7 +2353,9 @@ void Body::forward_impl(const double* q, const double* v, const double* f_ext, d
         double gd[4];
         {
             PhaseTimer ta(this, kFwdAA);
-            iterate(aa, true, d_qprev_.p, d_q_.p, 0.0, gd, nullptr);
+            queued = run_ahead && iter + 1 < max_pd_iter;
+            iterate(aa, true, d_qprev_.p, d_q_.p, 0.0, gd, nullptr,
+                    queued ? std::function<void()>(front) : std::function<void()>());
         }
         PhaseTimer tg(this, kFwdGate);
         const double abs_err = std::sqrt(gd[0]), rhs_norm = std::sqrt(gd[1]), rc = std::sqrt(gd[2]), rr = std::sqrt(gd[3]);
@@ -2558,12 +2582,11 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
         DevAnderson aa;
         aa.init(aa_window, n3, d_hist_q_, d_hist_g_);
         int it_used = 0;
-        for (int i = 0; i < max_it; ++i) {
-            // s_prev = s; r = rhs + K s - A s
+        // s_prev = s; r = rhs + K s - A s and its solve, up to where s is written
+        auto front = [&] {
             kpd_elements(d_s.p, precision);
             if (dense) {
                 iter_residual_dense(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, d_r_.p);
-                dense_solve(precision, d_r_.p, d_sprev.p, nullptr, nb > 0 ? d_uC_.p : nullptr, d_s.p);
             } else if (precision == 1) {
                 iter_residual<float>(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, w32_);
                 spmv_rows<float>(w32_, y32_, part32_, V32_.p);
@@ -2571,6 +2594,11 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
                 iter_residual<double>(false, d_rhs.p, d_s.p, d_sprev.p, 0.0, nullptr, w64_);
                 spmv_rows<double>(w64_, y64_, part64_, V64_.p);
             }
+        };
+        bool queued = false;  // this iteration's front is queued already
+        for (int i = 0; i < max_it; ++i) {
+            if (!queued) front();
+            if (dense) dense_solve(precision, d_r_.p, d_sprev.p, nullptr, nb > 0 ? d_uC_.p : nullptr, d_s.p);
             if (nb > 0) {
                 // s <- s + A^-1 r - A^-1 J^T G^-1 J (A^-1 r + s) on the device: project the
                 // candidate vectors on the basis, apply G^-1 (formed once per frame, FP32
@@ -2597,11 +2625,14 @@ void Body::backward(const double* q, const double* v, const double* f_ext, doubl
             // safe_clip (backward_gpu.cpp:809-816) before and after the Anderson
             // step: non-finite entries to 0, then |s| <= clip
             double ss, gg;
-            const bool combined = iterate(aa, false, d_sprev.p, d_s.p, clip, &ss, &gg);
+            queued = i + 1 < max_it && timing_level < 2;  // phase times: each by itself
+            const bool combined = iterate(aa, false, d_sprev.p, d_s.p, clip, &ss, &gg,
+                                          queued ? std::function<void()>(front) : std::function<void()>());
             const double err = std::sqrt(gg);
             double sn = std::sqrt(ss);
             if (combined && clip > 0 && std::isfinite(sn) && sn > clip) {
                 launch_scale(stream_, n3, clip / sn, d_s.p);
+                queued = false;  // its front saw the unscaled s
                 sn = clip;
             }
             it_used = i + 1;

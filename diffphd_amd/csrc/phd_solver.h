@@ -6,6 +6,7 @@
 
 #include <array>
 #include <deque>
+#include <functional>
 #include <cstdint>
 #include <map>
 #include <memory>
@@ -321,6 +322,7 @@ private:
     void upload_plan();  // plan_ buffers and the partial-sum arrays sized by it
     int device_ = 0;
     hipStream_t stream_ = nullptr;
+    hipEvent_t ev_iter_ = nullptr;  // the end of an iteration (iterate)
     void* scratch_ = nullptr;  // device address of the library's scratch array on device_
     template <class TV>
     void ainv_passes(const double* b_dev, double* x_dev, int refine, char* scr);
@@ -520,7 +522,8 @@ private:
     // clip > 0 (adjoint): xnew is scaled to that norm first. Returns whether x'
     // was combined: not with fewer than two iterates, nor after a restart
     // (|gamma| >= 10), which drops the history, the current iterate included.
-    bool iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew, double clip, double* sums, double* gg);
+    bool iterate(DevAnderson& aa, bool fwd, const double* xprev, double* xnew, double clip, double* sums, double* gg,
+                 const std::function<void()>& ahead);
     // r = b - A x of one iteration into w (see IterResidual)
     IterResidual iter_args(const double* rhs, double* x, double* xprev, double inv_h2m, const double* F);
     template <class TV>
