@@ -1851,9 +1851,10 @@ void Body::apply_ainv(double dt, const double* b, double* x, int precision, int 
     d_q_.download(x, dofs_);
 }
 
-// x = A^-1 r with the FP64 factor on device vectors (the baseline's global solve).
+// x = A^-1 r with the FP64 factor on device vectors (the baseline's global solve), in
+// the form its step chose.
 void Body::ainv64(const double* r, double* x) {
-    if (nv_ <= kDenseMaxVertices) {
+    if (bl_dense_) {
         ensure_dense(0);
         launch_dense_apply<double>(stream_, nv_, nv_, inv_ld_, d_inv64_.p, r, nullptr, nullptr, nullptr, nullptr, nullptr, x);
         return;
@@ -2065,9 +2066,13 @@ void Body::iter_residual_dense(bool fwd, const double* rhs, double* x, double* x
 // Explicit inverse of a small body (phd_small.hip).
 // ---------------------------------------------------------------------------
 bool Body::dense_inverse(const std::map<std::string, double>& opt, int precision) {
-    if (nv_ > kDenseMaxVertices || opt_or(opt, "phd_dense_inverse", 1.0) == 0.0) return false;
+    if (!dense_option(opt)) return false;
     ensure_dense(precision);
     return true;
+}
+
+bool Body::dense_option(const std::map<std::string, double>& opt) const {
+    return nv_ <= kDenseMaxVertices && opt_or(opt, "phd_dense_inverse", 1.0) != 0.0;
 }
 
 void Body::ensure_dense(int precision) {

@@ -537,6 +537,7 @@ private:
     // iteration amplifies the round-off between the two forms).
     static constexpr int kDenseMaxVertices = 4096;
     bool dense_inverse(const std::map<std::string, double>& opt, int precision);
+    bool dense_option(const std::map<std::string, double>& opt) const;  // the same without forming it
     void ensure_dense(int precision);
     // x = x_prev + A^-1 r (uC: A^-1 r at the candidates, may be null), and
     // x += (A^-1)_C f; dval as in launch_dense_apply
@@ -556,6 +557,10 @@ private:
     // oldest first); tmp: scratch
     void lbfgs_direction(const std::deque<int>& sh, const std::deque<int>& yh, const double* g, double* tmp, double* dir,
                          const std::vector<int>& frozen);
+    // The baseline's global solve takes the explicit inverse (set by each of its steps
+    // from its options). The columns of A^-1 at frozen nodes and their factored block
+    // stay from whichever form a step used first: they differ in round-off only.
+    bool bl_dense_ = false;
     void ainv64(const double* r, double* x);
     void pd_lhs_solve(const double* r, double* x, const std::vector<int>& frozen);
     int pd_nonlinear_solve(const double* q_init, double inv_h2m, const double* rhs, const std::vector<int>& frozen,

@@ -5,9 +5,11 @@ Dirichlet conditions, contact adjoints, both precisions, and the largest body th
 takes it beside the first that does not."""
 import numpy as np
 import pytest
+import torch  # before the library is loaded: both use the same HIP runtime
 
 from diffphd_amd import scenes
 from helpers import backward_frame, product_body, rel_err, rollout
+from test_oracle_baseline import BASELINE_OPT
 from test_oracle_dirichlet import slider
 
 pytestmark = pytest.mark.gpu
@@ -78,3 +80,43 @@ def test_contact_adjoint_hex_and_tet(precision):
         errs = [rel_err(res[0][i], res[1][i]) for i in (0, 1, 3, 4)]
         print(spec["name"], "contacts", len(acts[1]), errs)
         assert max(errs) < (1e-8 if precision == 0 else 1e-4)
+
+
+def _baseline_step(spec, opt, frames):
+    body = product_body(spec)
+    q, v, acts = rollout(body, spec, frames, opt, method="pd_eigen_pcg")
+    g = np.random.default_rng(6).standard_normal(body.dofs())
+    out = backward_frame(body, spec, q, v, acts, frames - 1, g, 0 * g, opt, method="pd_eigen_pcg")
+    return [q[-1]] + [out[i] for i in (0, 1, 3, 4)], acts[-1]
+
+
+@pytest.mark.parametrize("scene", ["beam", "napkin"])
+def test_baseline_takes_the_option(scene):
+    """L-BFGS stops at rel_tol 1e-12 with either form, so results agree to a small
+    multiple of it; they are not the same bits, which shows that two forms ran."""
+    if scene == "beam":
+        spec, frames = scenes.actuated_cantilever(cells=(6, 3, 2)), 1
+    else:  # at rest on the sphere: frozen contact nodes, so the columns of A^-1 as well
+        spec, frames = scenes.napkin(), 48
+    opt = dict(BASELINE_OPT, rel_tol=1e-12, abs_tol=1e-12, max_pd_iter=20000)
+    (a, ca), (b, cb) = (_baseline_step(spec, dict(opt, phd_dense_inverse=d), frames) for d in (1, 0))
+    errs = [rel_err(x, y) for x, y in zip(a, b)]
+    print(scene, "contacts", len(ca), errs)
+    assert ca == cb and (scene == "beam" or len(ca) > 0)
+    assert max(errs) < 1e-8
+    assert not all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def test_baseline_without_the_option_allocates_no_inverse():
+    """4,096 vertices: the FP64 inverse is 128 MiB."""
+    spec = scenes.actuated_cantilever(cells=(15, 15, 15))
+    used = {}
+    for dense in (0, 1):
+        body = product_body(spec)
+        body.factor_build(spec["dt"])
+        free = torch.cuda.mem_get_info()[0]
+        opt = dict(BASELINE_OPT, rel_tol=0.5, phd_dense_inverse=dense)
+        rollout(body, spec, 1, opt, method="pd_eigen_pcg")
+        used[dense] = (free - torch.cuda.mem_get_info()[0]) / 2.0**20
+    print("MiB", used)
+    assert used[0] < 64 and used[1] >= 128
