@@ -2,10 +2,9 @@
 // full matrix in vertex order, and its products.
 //
 // The two products with S are four dependent launches (chunk partials, their sums,
-// column-tile partials, their sums) whose units each walk a chain of rows: 55 us at
-// 425 vertices and 60 us at 2,673, where the values themselves are 0.2 and 2.8 MB.
-// One product with the full inverse is one launch without a chain (6 us and 9 us),
-// at the price of n^2 values; Body::ensure_dense states up to which n that pays.
+// column-tile partials, their sums). One product with the full inverse is one launch
+// without a chain (4 us at 425 vertices in FP64, 14 us at 2,673 in FP32), at the price of
+// n^2 values; Body::kDenseMaxVertices states up to which n that pays, with both sides.
 #include <hip/hip_runtime.h>
 
 #include "phd_kernels.h"

@@ -535,9 +535,24 @@ private:
     // phd_dense_inverse = 0 keeps the products with S): the adjoint of every small
     // body, the forward of one without a frictional boundary (with one, the
     // iteration amplifies the round-off between the two forms).
+    //
+    // The inverse reads n^2 values where S reads its nonzeros in four launches. us per
+    // iteration, inverse / S (forward; adjoint; cantilevers):
+    //   vertices      FP64                       mixed
+    //     425    37 / 52;  24 / 40          37 / 48;  27 / 39
+    //   2,028    47 / 56;  47 / 55          43 / 50;  39 / 47
+    //   2,744    52 / 56;  44 / 54          50 / 50;  41 / 44
+    //   2,880    52 / 56;  54 / 62          51 / 50;  51 / 51
+    //   4,096    61 / 66;  60 / 68          59 / 57;  59 / 58
+    //   5,184    79 / 71;  74 / 70          76 / 65;  71 / 62
+    // An adjoint's constrained iteration, which adds the gather and the scatter of
+    // the contacts to S, takes 75 / 94 (FP64) and 73 / 80 (mixed) at 2,880 and 84 / 97
+    // and 77 / 88 at 4,096. So a mixed body without contacts changes over earlier.
+    // Forming the inverse takes 0.2 to 1.2 ms up to there.
     static constexpr int kDenseMaxVertices = 4096;
+    static constexpr int kDenseMaxMixedFree = 2816;  // mixed precision, no frictional boundary
     bool dense_inverse(const std::map<std::string, double>& opt, int precision);
-    bool dense_option(const std::map<std::string, double>& opt) const;  // the same without forming it
+    bool dense_option(const std::map<std::string, double>& opt, int precision) const;  // the same without forming it
     void ensure_dense(int precision);
     // x = x_prev + A^-1 r (uC: A^-1 r at the candidates, may be null), and
     // x += (A^-1)_C f; dval as in launch_dense_apply
