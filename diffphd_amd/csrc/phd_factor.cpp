@@ -359,7 +359,7 @@ void Factor::build(int n_, const std::vector<int>& Ap, const std::vector<int>& A
     factor_seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t1).count();
 }
 
-void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w) {
+void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w, int min_fine_items, size_t fine_units) {
     chunk_w = group_chunk_w;
     const int n = f.n;
     const int ntiles = (n + 63) / 64;
@@ -386,7 +386,7 @@ void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w) {
             c += (cu_i1[tile_unit_ptr[t + 1] - 1] - cu_i0[tile_unit_ptr[t]] + h - 1) / h;
         return c;
     };
-    while (fine_items > 64 && count(fine_items) < 4096) fine_items /= 2;
+    while (fine_items > min_fine_items && count(fine_items) < fine_units) fine_items /= 2;
     fu_tile.clear(); fu_i0.clear(); fu_i1.clear(); tile_fine_ptr.clear();
     if (fine_items < unit_items) {
         tile_fine_ptr.assign(ntiles + 1, 0);
@@ -436,14 +436,14 @@ void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w) {
 // Host emulation of the device data path for small systems (tests): expands
 // S = L^-1 column by column, checks S^T S A = I, the subtree-range structure,
 // and replays the two SpMV plans against dense products.
-// out: [0] max |S^T S A - I|, [1] max |plan(S w) - S w|, [2] max |plan(S^T y) - S^T y|,
+// out: [0] max |S^T S A - I|, [1] max |plan(S w) - S w|, [2] max |plan(S^T y) - S^T y| (both unit lists),
 //      [3] nnz(S), [4] max depth, [5] nnz(L), [6] structural violations.
 void host_factor_check(int n, const std::vector<int>& Ap, const std::vector<int>& Ai, const std::vector<double>& Ax,
                        const std::vector<double>& X, double* out) {
     Factor f;
     f.build(n, Ap, Ai, Ax, X, 2);
     SpmvPlan plan;
-    plan.build(f, 5, 16);  // small chunks so that rows split and chains split
+    plan.build(f, 5, 16, 2);  // small chunks and units, so that rows, chains and the shorter units split
     std::vector<double> V(f.v_len, 0.0);
     std::vector<double> x(n);
     double viol = 0;
@@ -511,17 +511,17 @@ void host_factor_check(int n, const std::vector<int>& Ap, const std::vector<int>
         }
     };
     cols(plan.cu_tile, plan.cu_i0, plan.cu_i1, xpl);
-    if (!plan.fu_tile.empty()) {
-        std::vector<double> xfl(n, 0.0);
-        cols(plan.fu_tile, plan.fu_i0, plan.fu_i1, xfl);
-        for (size_t t = 0; t + 1 < plan.tile_fine_ptr.size(); ++t)
-            for (int u = plan.tile_fine_ptr[t]; u < plan.tile_fine_ptr[t + 1]; ++u)
-                if (plan.fu_tile[u] != (int)t) viol += 1;
-        for (int j = 0; j < n; ++j)
-            if (std::fabs(xfl[j] - xref[j]) > std::fabs(xpl[j] - xref[j])) xpl[j] = xfl[j];
-    }
+    // the shorter units: there, each tile's its own and no longer than asked for, and the
+    // same product
+    std::vector<double> xfl(n, 0.0);
+    cols(plan.fu_tile, plan.fu_i0, plan.fu_i1, xfl);
+    if (plan.fu_tile.empty() || plan.tile_fine_ptr.back() != (int)plan.fu_tile.size()) viol += 1;
+    for (size_t t = 0; t + 1 < plan.tile_fine_ptr.size(); ++t)
+        for (int u = plan.tile_fine_ptr[t]; u < plan.tile_fine_ptr[t + 1]; ++u)
+            if (plan.fu_tile[u] != (int)t || plan.fu_i1[u] - plan.fu_i0[u] > 2) viol += 1;
     double e1 = 0, e2 = 0;
     for (int k = 0; k < n; ++k) { e1 = std::max(e1, std::fabs(ypl[k] - yref[k])); e2 = std::max(e2, std::fabs(xpl[k] - xref[k])); }
+    for (int k = 0; k < n; ++k) e2 = std::max(e2, std::fabs(xfl[k] - xref[k]));
     out[0] = err; out[1] = e1; out[2] = e2; out[3] = (double)f.nnz; out[4] = f.max_depth; out[5] = (double)f.Lx.size();
     out[6] = viol;
 }

@@ -67,7 +67,8 @@ struct SpmvPlan {
     int row_group = 64;
     int chunk_w = 1024;
     std::vector<int> gu_group, gu_chunk, rbase;
-    void build(const Factor& f, int unit_items, int group_chunk_w = 1024);
+    // min_fine_items, fine_units: the fewest rows of a shorter unit, and the units that are enough
+    void build(const Factor& f, int unit_items, int group_chunk_w = 1024, int min_fine_items = 64, size_t fine_units = 4096);
 };
 
 void host_factor_check(int n, const std::vector<int>& Ap, const std::vector<int>& Ai, const std::vector<double>& Ax,
