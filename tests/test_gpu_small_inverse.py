@@ -59,12 +59,15 @@ def test_per_dof_dirichlet(precision):
     _compare(spec, opt, 1e-9 if precision == 0 else 1e-4)
 
 
+# Vertices and candidates: 168 and 42, 125 and 25 (one row per workgroup); 1,287 and 143,
+# 1,331 and 121 (four rows, the last group and every last vector ragged).
+@pytest.mark.parametrize("beam_cells,tet_n", [((5, 6, 3), 4), ((12, 10, 8), 10)])
 @pytest.mark.parametrize("precision", [0, 1])
-def test_contact_adjoint_hex_and_tet(precision):
+def test_contact_adjoint_hex_and_tet(precision, beam_cells, tet_n):
     """Bodies with a boundary keep S in the forward, so q is the same bit for bit; the
     adjoint (backbone and contact-basis correction) takes the inverse."""
-    beam = scenes.beam(cells=(5, 6, 3), E=1e5, nu=0.4, seed=2)
-    tet = scenes.tet_block(n=4, seed=2)
+    beam = scenes.beam(cells=beam_cells, E=1e5, nu=0.4, seed=2)
+    tet = scenes.tet_block(n=tet_n, seed=2)
     tet["v0"] = np.tile([0.0, 0.0, -4.5], tet["V"].shape[1])  # reaches the ground this frame
     for spec in (beam, tet):
         opt = dict(spec["options"], max_pd_iter=12, rel_tol=0.0, abs_tol=0.0, phd_precision=precision,
@@ -72,6 +75,7 @@ def test_contact_adjoint_hex_and_tet(precision):
         a = product_body(spec)
         qa, _, acts = rollout(a, spec, 1, opt)
         qb, _, _ = rollout(product_body(spec), spec, 1, dict(opt, phd_dense_inverse=0))
+        print(spec["name"], "vertices", a.dofs() // 3, "candidates", len(spec["boundary"][2]))
         assert len(acts[1]) > 0 and np.array_equal(qa[1], qb[1])
         bopt = dict(opt, max_pd_iter=400, rel_tol=1e-12, abs_tol=1e-14)
         g = np.random.default_rng(4).standard_normal(a.dofs())
