@@ -221,11 +221,6 @@ void launch_contact_gather(hipStream_t s, const ContactPieces& pc, const int* cp
 template <class TV>
 void launch_contact_scatter(hipStream_t s, const ContactPieces& pc, const int* rc_row, const int* rc_c, const TV* rc_val,
                             const double* f, double* part, int n, TV* y);
-// M[i][j] = om_i (n_i . n_j) H[i][j] om_j + (i == j) E_i  (row-major, TM = float or double)
-template <class TM>
-void launch_assemble_msys(hipStream_t s, int K, const double* H, const double* nrm, const double* om, const double* E, TM* M);
-// out[3c + d] = sum_j H[c][j] f[3j + d]
-void launch_h_apply(hipStream_t s, int K, const double* H, const double* f, double* out);
 
 void launch_gather_vals(hipStream_t s, int64_t m, const int* rows, const int* cols, const int64_t* base,
                         const double* V64, double* o64, float* o32);
@@ -281,10 +276,6 @@ template <class TH>
 void launch_h_apply_idx(hipStream_t s, int nr, const int* rows, int nc, const int* cols, const TH* H, int K,
                         const double* f, double* out);
 void launch_to_float(hipStream_t s, int64_t n, const double* a, float* b);
-// contact system restricted to the index set J (row-major nJ x nJ)
-template <class TM>
-void launch_assemble_msys_idx(hipStream_t s, int nJ, const int* J, const double* H, int K, const double* nrm,
-                              const double* om, const double* E, TM* M);
 
 // streaming copy of n16 16-byte words (byte-counter calibration)
 void launch_copy(hipStream_t s, int64_t n16, const void* a, void* b);

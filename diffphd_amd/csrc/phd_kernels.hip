@@ -1130,34 +1130,6 @@ __global__ void k_contact_scatter_fin(int nrows, const int* __restrict__ piece_p
     y[2 * n + k] += (TV)a2;
 }
 
-template <class TM>
-__global__ void k_assemble_msys(int K, const double* __restrict__ H, const double* __restrict__ nrm,
-                                const double* __restrict__ om, const double* __restrict__ E, TM* __restrict__ M) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)K * K) return;
-    const int i = (int)(idx / K), j = (int)(idx % K);
-    const double nd = nrm[3 * i] * nrm[3 * j] + nrm[3 * i + 1] * nrm[3 * j + 1] + nrm[3 * i + 2] * nrm[3 * j + 2];
-    double v = om[i] * nd * H[idx] * om[j];
-    if (i == j) v += E[i];
-    M[idx] = (TM)v;
-}
-
-__global__ void k_h_apply(int K, const double* __restrict__ H, const double* __restrict__ f, double* __restrict__ out) {
-    const int c = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-    const int lane = threadIdx.x % WAVE;
-    if (c >= K) return;
-    const double* Hr = H + (int64_t)c * K;
-    double a0 = 0, a1 = 0, a2 = 0;
-    for (int j = lane; j < K; j += WAVE) {
-        const double h = Hr[j];
-        a0 += h * f[3 * j];
-        a1 += h * f[3 * j + 1];
-        a2 += h * f[3 * j + 2];
-    }
-    a0 = wave_sum(a0); a1 = wave_sum(a1); a2 = wave_sum(a2);
-    if (lane == 0) { out[3 * c] = a0; out[3 * c + 1] = a1; out[3 * c + 2] = a2; }
-}
-
 // -----------------------------------------------------------------------------
 // Backward: per-sample 9x9 proximal-map Jacobians (SetupProjectiveDynamicsLocalStepDifferential,
 // deformable_projective_dynamics_backward.cpp:10-80) and their matrix-free application
@@ -1667,21 +1639,6 @@ __global__ __launch_bounds__(kHWaves * WAVE) void k_h_apply_idx(int nr, const in
     if (a0 >= nr) return;  // uniform over the workgroup
     h_apply_rows<TH>(a0, nr, rows, nc, cols, H, K, f, out);
 }
-// Compressed contact system on the index set J: M[a][b] = om_i (n_i . n_j) H[i][j] om_j + (a == b) E_i.
-template <class TM>
-__global__ void k_assemble_msys_idx(int nJ, const int* __restrict__ J, const double* __restrict__ H, int K,
-                                    const double* __restrict__ nrm, const double* __restrict__ om,
-                                    const double* __restrict__ E, TM* __restrict__ M) {
-    const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (int64_t)nJ * nJ) return;
-    const int a = (int)(idx / nJ), b = (int)(idx % nJ);
-    const int i = J[a], j = J[b];
-    const double nd = nrm[3 * i] * nrm[3 * j] + nrm[3 * i + 1] * nrm[3 * j + 1] + nrm[3 * i + 2] * nrm[3 * j + 2];
-    double v = om[i] * nd * H[(int64_t)i * K + j] * om[j];
-    if (a == b) v += E[i];
-    M[idx] = (TM)v;
-}
-
 // Plain streaming copy (calibration of the HBM byte counters).
 // Four 16-byte loads in flight per lane, one pass over the data.
 __global__ void __launch_bounds__(256) k_copy(int64_t n, const float4* __restrict__ a, float4* __restrict__ b) {
@@ -1978,32 +1935,9 @@ void launch_to_float(hipStream_t s, int64_t n, const double* a, float* b) {
     if (n == 0) return;
     hipLaunchKernelGGL(k_to_float, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, a, b);
 }
-template <class TM>
-void launch_assemble_msys_idx(hipStream_t s, int nJ, const int* J, const double* H, int K, const double* nrm,
-                              const double* om, const double* E, TM* M) {
-    if (nJ == 0) return;
-    hipLaunchKernelGGL(k_assemble_msys_idx<TM>, dim3(blocks_for((int64_t)nJ * nJ, 256)), dim3(256), 0, s, nJ, J, H, K,
-                       nrm, om, E, M);
-}
-template void launch_assemble_msys_idx<float>(hipStream_t, int, const int*, const double*, int, const double*,
-                                              const double*, const double*, float*);
-template void launch_assemble_msys_idx<double>(hipStream_t, int, const int*, const double*, int, const double*,
-                                               const double*, const double*, double*);
 void launch_copy(hipStream_t s, int64_t n16, const void* a, void* b) {
     hipLaunchKernelGGL(k_copy, dim3((unsigned)((n16 + 1023) / 1024)), dim3(256), 0, s, n16, (const float4*)a, (float4*)b);
 }
-template <class TM>
-void launch_assemble_msys(hipStream_t s, int K, const double* H, const double* nrm, const double* om, const double* E, TM* M) {
-    if (K == 0) return;
-    hipLaunchKernelGGL(k_assemble_msys<TM>, dim3(blocks_for((int64_t)K * K, 256)), dim3(256), 0, s, K, H, nrm, om, E, M);
-}
-template void launch_assemble_msys<float>(hipStream_t, int, const double*, const double*, const double*, const double*, float*);
-template void launch_assemble_msys<double>(hipStream_t, int, const double*, const double*, const double*, const double*, double*);
-void launch_h_apply(hipStream_t s, int K, const double* H, const double* f, double* out) {
-    if (K == 0) return;
-    hipLaunchKernelGGL(k_h_apply, dim3(blocks_for(K, 4)), dim3(256), 0, s, K, H, f, out);
-}
-
 template <class TW>
 void launch_kpd_build(hipStream_t s, const DevMaterials& m, const double* kc, const double* kv, const double* const* kn,
                       const double* q, int filter, double theta, double lo, int* nfilt, TW* W) {

@@ -91,24 +91,6 @@ static double nrm2(const std::vector<double>& v) {
     for (double x : v) s += x * x;
     return std::sqrt(s);
 }
-// Dense symmetric solve by LDL^T (small systems: AA Gram). Row-major.
-static std::vector<double> small_ldlt_solve(std::vector<double> M, int n, std::vector<double> x) {
-    std::vector<double> d(n);
-    for (int j = 0; j < n; ++j) {
-        double djj = M[j * n + j];
-        for (int k = 0; k < j; ++k) djj -= M[j * n + k] * M[j * n + k] * d[k];
-        d[j] = djj;
-        for (int i = j + 1; i < n; ++i) {
-            double s = M[i * n + j];
-            for (int k = 0; k < j; ++k) s -= M[i * n + k] * M[j * n + k] * d[k];
-            M[i * n + j] = djj != 0 ? s / djj : 0;
-        }
-    }
-    for (int i = 0; i < n; ++i) for (int k = 0; k < i; ++k) x[i] -= M[i * n + k] * x[k];
-    for (int i = 0; i < n; ++i) x[i] = d[i] != 0 ? x[i] / d[i] : 0;
-    for (int i = n - 1; i >= 0; --i) for (int k = i + 1; k < n; ++k) x[i] -= M[k * n + i] * x[k];
-    return x;
-}
 static double det3(const double* A) {  // column-major
     return A[0] * (A[4] * A[8] - A[7] * A[5]) - A[3] * (A[1] * A[8] - A[7] * A[2]) + A[6] * (A[1] * A[5] - A[4] * A[2]);
 }
@@ -1037,11 +1019,9 @@ void Body::setup(double dt, int threads) {
     pverts_.clear();
     dval_full_.assign(dofs_, 0.0);
     ddof_.clear();
-    dval_.clear();
     for (auto& kv : dirichlet_) {
         dval_full_[kv.first] = kv.second;
         ddof_.push_back(kv.first);
-        dval_.push_back(kv.second);
     }
     for (int v = 0; v < nv_; ++v) {
         const int nfix = (int)dirichlet_.count(3 * v) + (int)dirichlet_.count(3 * v + 1) + (int)dirichlet_.count(3 * v + 2);
@@ -1184,8 +1164,6 @@ void Body::setup(double dt, int threads) {
         d_Axe_.upload(ax);
     }
     d_dmask_.upload(dmask_);
-    d_ddof_.upload(ddof_);
-    d_dval_.upload(dval_);
     d_dval_full_.upload(dval_full_);
     d_fix_.release();
     if (!ddof_.empty()) {
@@ -1255,7 +1233,7 @@ void Body::setup(double dt, int threads) {
     d_inc_idx_.upload(inc);
     build_materials();
     // work vectors
-    for (auto* b : {&d_q_, &d_qprev_, &d_qtilde_, &d_b_, &d_r_, &d_pdrhs_, &d_pdrhs_prev_, &d_g_, &d_tmp_, &d_kz_})
+    for (auto* b : {&d_q_, &d_qprev_, &d_qtilde_, &d_b_, &d_r_, &d_pdrhs_, &d_pdrhs_prev_, &d_tmp_})
         b->alloc(dofs_);
     d_elem_.alloc((size_t)ne_ * edim_ * 3);
     d_dot_partial_.alloc(dots_partial_size());
@@ -1308,7 +1286,6 @@ void Body::setup_contact(int threads) {
     d_cp_val64_.alloc(m);
     d_cp_val32_.alloc(m);
     launch_gather_vals(stream_, m, drow.p, dcol.p, d_base_.p, V64_.p, d_cp_val64_.p, d_cp_val32_.p);
-    d_cp_ptr_.upload(cp_ptr);
     d_cp_row_.upload(cp_row);
     // row-compact transpose
     std::vector<int> rowid(nv_, -1), urows;
@@ -1334,7 +1311,6 @@ void Body::setup_contact(int threads) {
     d_rc_val64_.alloc(m);
     d_rc_val32_.alloc(m);
     launch_gather_vals(stream_, m, dr2.p, dc2.p, d_base_.p, V64_.p, d_rc_val64_.p, d_rc_val32_.p);
-    d_rc_ptr_.upload(rc_ptr);
     d_rc_row_.upload(rc_rowk);
     d_rc_c_.upload(rc_c);
     rc_nrows_ = R;
@@ -1392,11 +1368,10 @@ void Body::setup_contact(int threads) {
     for (auto* b : {&d_nrm_, &d_t1_, &d_t2_, &d_F_, &d_dF_, &d_uC_, &d_tmpK3_, &d_qframeC_, &d_Fg_, &d_Fn_, &d_hprev_})
         b->alloc((size_t)3 * K_);
     for (auto* b : {&d_delta_, &d_om_, &d_E_, &d_rhsK_, &d_rprec_, &d_lambda_, &d_lt1_, &d_lt2_, &d_hvec_}) b->alloc(K_);
-    for (auto* b : {&d_idxJ_, &d_idxP_, &d_idxF_, &d_posJ_, &d_posL_}) b->alloc(K_);
+    for (auto* b : {&d_posJ_, &d_posL_}) b->alloc(K_);
     d_ncp_lists_.alloc((size_t)6 * K_);
     d_ncp_counts_.alloc(8);
     d_ncp_flags_.alloc(K_);
-    d_rhsK32_.alloc(K_);
     d_info_.alloc(1);
 }
 
@@ -1584,7 +1559,7 @@ Body::TuneResult Body::autotune(double dt, int threads, int reps) {
             launch_spmv_cols<float>(stream_, (int)plan_.cu_tile.size(), d_cu_tile_.p, d_cu_i0_.p, d_cu_i1_.p, d_items_.p,
                                     d_fd_.p, d_base_.p, V32_.p, y32_.p, nv_, xpart32_.p);
             launch_spmv_cols_fin<float>(stream_, nv_, d_tile_unit_ptr_.p, xpart32_.p, d_perm_.p, nullptr, nullptr,
-                                        nullptr, d_g_.p);
+                                        nullptr, d_r_.p);
         });
         if (res.cols_ms[i] < res.cols_ms[best]) best = i;
     }
@@ -1800,11 +1775,8 @@ void Body::warm_start(const double* v, double dt, double inv_h2m, bool learned) 
               "warm start");
 }
 
-// Contact system M dl = rhs on the index set J (already in d_idxJ_, with
-// d_om_ / d_E_ / d_nrm_ current): assembled and solved by the blocked
-// Cholesky of phd_dense.hip. rhs (host, n) is overwritten with the solution.
-// Returns false when a pivot was not positive.
-// The compressed contact system on the candidates J (n rows): its right-hand
+// The compressed contact system on the candidates J (n rows), with d_om_ / d_E_ / d_nrm_
+// current: assembled and solved by the blocked Cholesky of phd_dense.hip. Its right-hand
 // side is in d_rhsK_, the solution stays on the device (d_cx32_ / d_cx64_);
 // only the pivot flag comes back. False when a pivot was not positive.
 bool Body::solve_contact_system(int n, int precision, const int* J, bool plain_w) {

@@ -414,7 +414,7 @@ private:
     // (t, o may be null: zero)
     void partial_dirichlet(double* y, const double* t, const double* o);
     std::vector<int> ddof_;
-    std::vector<double> dval_, dval_full_;
+    std::vector<double> dval_full_;
     std::vector<double> c_dir_;
     // device
     DevBuf<double> V64_;
@@ -427,8 +427,7 @@ private:
     DevBuf<int> d_Aie_;
     DevBuf<double> d_Axe_;
     DevBuf<unsigned char> d_dmask_;
-    DevBuf<int> d_ddof_;
-    DevBuf<double> d_dval_, d_dval_full_;
+    DevBuf<double> d_dval_full_;
     DevBuf<double> d_c_dir_;
     DevBuf<int> d_elems_, d_inc_ptr_, d_inc_idx_;
     DevBuf<double> d_G_, d_wc_, d_wv_, d_wn_[4];
@@ -440,7 +439,7 @@ private:
     bool has_cor_ = false, has_vol_ = false;
     bool kpd_exact_ = false;
     // work vectors (3N FP64)
-    DevBuf<double> d_q_, d_qprev_, d_qtilde_, d_b_, d_r_, d_pdrhs_, d_pdrhs_prev_, d_elem_, d_g_, d_tmp_, d_kz_;
+    DevBuf<double> d_q_, d_qprev_, d_qtilde_, d_b_, d_r_, d_pdrhs_, d_pdrhs_prev_, d_elem_, d_tmp_;
     // warm start: network, per-vertex feature inputs, guesses
     std::unique_ptr<WarmStartNet> net_;
     DevBuf<float> d_logk_, d_cflag_, d_cdist_, d_feat_, d_mlpout_, d_fmean_, d_fstd_, d_adiag_;
@@ -463,7 +462,7 @@ private:
     DevBuf<double> d_H_;
     DevBuf<float> d_H32_;  // FP32 copy of H for the mixed path's applies and assembly        // A^-1 restricted to the candidates (K x K, FP64)
     std::vector<double> Hdiag_;
-    DevBuf<int> d_cp_ptr_, d_cp_row_, d_rc_ptr_, d_rc_row_, d_rc_c_;
+    DevBuf<int> d_cp_row_, d_rc_row_, d_rc_c_;
     DevBuf<double> d_cp_val64_, d_rc_val64_;
     DevBuf<float> d_cp_val32_, d_rc_val32_;
     int rc_nrows_ = 0;
@@ -481,9 +480,7 @@ private:
     DevBuf<double> d_C64_, d_cy64_, d_cx64_;  // dense contact system (blocked Cholesky layout)
     DevBuf<float> d_C32_, d_cy32_, d_cx32_;
     DevBuf<double> d_rhsK_;
-    DevBuf<float> d_rhsK32_;
     DevBuf<int> d_info_;
-    DevBuf<int> d_idxJ_, d_idxP_, d_idxF_;
     void* blas_ = nullptr;
     std::vector<hipEvent_t> ev_pool_;
     size_t ev_used_ = 0;
