@@ -250,6 +250,9 @@ public:
     // Times `reps` launches of each candidate on this body's factor and mesh
     // and keeps the fastest: the column-chunk width of S w (FP32, the mixed
     // path's product), the unit height of S^T y, the local step's block size.
+    // The height is timed on the list that apply_ainv and frictional forward steps use;
+    // the shorter units of the other solves (SpmvPlan::fu_*) follow from it by their own
+    // rule, and a body that takes the explicit inverse uses neither there.
     struct TuneResult {
         int chunk_w = 0, unit_items = 0, local_block = 0;
         double rows_ms[3] = {0}, cols_ms[4] = {0}, local_ms[3] = {0};

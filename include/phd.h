@@ -218,7 +218,9 @@ int phd_factor_info(phd_ctx ctx, double* out, int cap);
  * times `reps` launches of each candidate on this body and keeps the fastest
  * of the column-chunk width of S w (512, 1024, 2048; FP32 product), the unit
  * height of S^T y (256, 512, 1024, 2048 rows) and the local step's block size
- * (64, 128, 256). Results are independent of the choice up to the summation
+ * (64, 128, 256). The height is timed on the units of phd_apply_ainv and of
+ * frictional forward steps; adjoints and contact-free steps derive shorter
+ * units from it where these are too few. Results are independent of the choice up to the summation
  * order of the partial sums. out: [0] chunk width, [1] unit height, [2] block,
  * [3..5] ms per S w, [6..9] ms per S^T y, [10..12] ms per local step, one per
  * candidate (up to `cap` values; out may be NULL). */
