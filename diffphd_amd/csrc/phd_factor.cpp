@@ -388,7 +388,7 @@ void SpmvPlan::build(const Factor& f, int unit_items, int group_chunk_w, int min
     };
     while (fine_items > min_fine_items && count(fine_items) < fine_units) fine_items /= 2;
     fu_tile.clear(); fu_i0.clear(); fu_i1.clear(); tile_fine_ptr.clear();
-    if (fine_items < unit_items) {
+    if (fine_items < unit_items && count(fine_items) > cu_tile.size()) {
         tile_fine_ptr.assign(ntiles + 1, 0);
         for (int t = 0; t < ntiles; ++t) {
             const int i0 = cu_i0[tile_unit_ptr[t]], i1 = cu_i1[tile_unit_ptr[t + 1] - 1];
@@ -511,11 +511,14 @@ void host_factor_check(int n, const std::vector<int>& Ap, const std::vector<int>
         }
     };
     cols(plan.cu_tile, plan.cu_i0, plan.cu_i1, xpl);
-    // the shorter units: there, each tile's its own and no longer than asked for, and the
-    // same product
+    // the shorter units: there where a unit has to be split and only there, each tile's its
+    // own and no longer than asked for, and the same product
     std::vector<double> xfl(n, 0.0);
-    cols(plan.fu_tile, plan.fu_i0, plan.fu_i1, xfl);
-    if (plan.fu_tile.empty() || plan.tile_fine_ptr.back() != (int)plan.fu_tile.size()) viol += 1;
+    bool split = false;
+    for (size_t u = 0; u < plan.cu_tile.size(); ++u) split |= plan.cu_i1[u] - plan.cu_i0[u] > 2;
+    if (split != !plan.fu_tile.empty()) viol += 1;
+    if (split) cols(plan.fu_tile, plan.fu_i0, plan.fu_i1, xfl); else xfl = xpl;
+    if (!plan.fu_tile.empty() && plan.tile_fine_ptr.back() != (int)plan.fu_tile.size()) viol += 1;
     for (size_t t = 0; t + 1 < plan.tile_fine_ptr.size(); ++t)
         for (int u = plan.tile_fine_ptr[t]; u < plan.tile_fine_ptr[t + 1]; ++u)
             if (plan.fu_tile[u] != (int)t || plan.fu_i1[u] - plan.fu_i0[u] > 2) viol += 1;

@@ -53,9 +53,9 @@ struct SpmvPlan {
     // (the adjoint and bodies without a frictional boundary; the frictional forward
     // iteration amplifies round-off and keeps the order above): halved until they give
     // every CU 16 waves or have 64 rows, one batch. Empty where the units above are
-    // that many. A unit of 512 rows is walked by one wave while most of the chip is
-    // idle: 66 us at 5,040 vertices in FP64 and 35 us at 9,261 in FP32, with units of
-    // 64 rows 15 and 10 us; 56 and 52 us at 35,301 in FP32.
+    // that many or that short. A unit of 512 rows is walked by one wave while most of the
+    // chip is idle: 66 us at 5,040 vertices in FP64 and 35 us at 9,261 in FP32, with units
+    // of 64 rows 15 and 10 us; 56 and 52 us at 35,301 in FP32.
     std::vector<int> fu_tile, fu_i0, fu_i1, tile_fine_ptr;
     // S w by units of (group of row_group consecutive rows, chunk of chunk_w
     // columns): each unit stages w[chunk] once for all rows of the group that
