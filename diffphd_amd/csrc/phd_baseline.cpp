@@ -348,7 +348,7 @@ void Body::forward_baseline(const std::string& method, const double* q, const do
     require((int)act_.size() == act_dofs_, "Inconsistent actuation size.");
     setup(dt, threads);
     require(pverts_.empty(), "The baseline forward supports whole-vertex Dirichlet conditions only.");
-    bl_dense_ = dense_option(opt, 0);
+    bl_dense_ = dense_option(opt);
     if (kpd_exact_) { kpd_exact_ = false; build_materials(); }  // energies read each energy's stiffness()
     last_baseline = BaselineStats();
     const int n3 = dofs_;
@@ -473,7 +473,7 @@ void Body::backward_baseline(const double* q, const double* v, const double* f_e
     require((int)act_.size() == act_dofs_, "Inconsistent actuation size.");
     setup(dt, threads);
     require(pverts_.empty(), "The baseline backward supports whole-vertex Dirichlet conditions only.");
-    bl_dense_ = dense_option(opt, 0);
+    bl_dense_ = dense_option(opt);
     if (kpd_exact_) { kpd_exact_ = false; build_materials(); }
     const int n3 = dofs_, nE = (int)energies_.size();
     const double h = dt, inv_h = 1 / h, mass = element_volume_ * density_, h2m = h * h / mass, inv_h2m = mass / (h * h);

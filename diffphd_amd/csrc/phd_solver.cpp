@@ -2038,14 +2038,13 @@ void Body::iter_residual_dense(bool fwd, const double* rhs, double* x, double* x
 // Explicit inverse of a small body (phd_small.hip).
 // ---------------------------------------------------------------------------
 bool Body::dense_inverse(const std::map<std::string, double>& opt, int precision) {
-    if (!dense_option(opt, precision)) return false;
+    if (!dense_option(opt)) return false;
     ensure_dense(precision);
     return true;
 }
 
-bool Body::dense_option(const std::map<std::string, double>& opt, int precision) const {
-    return nv_ <= (precision == 1 && K_ == 0 ? kDenseMaxMixedFree : kDenseMaxVertices) &&
-           opt_or(opt, "phd_dense_inverse", 1.0) != 0.0;
+bool Body::dense_option(const std::map<std::string, double>& opt) const {
+    return nv_ <= kDenseMaxVertices && opt_or(opt, "phd_dense_inverse", 1.0) != 0.0;
 }
 
 void Body::ensure_dense(int precision) {

@@ -537,22 +537,25 @@ private:
     // iteration amplifies the round-off between the two forms).
     //
     // The inverse reads n^2 values where S reads its nonzeros in four launches. us per
-    // iteration, inverse / S (forward; adjoint; cantilevers):
-    //   vertices      FP64                       mixed
-    //     425    37 / 52;  24 / 40          37 / 48;  27 / 39
-    //   2,028    47 / 56;  47 / 55          43 / 50;  39 / 47
-    //   2,744    52 / 56;  44 / 54          50 / 50;  41 / 44
-    //   2,880    52 / 56;  54 / 62          51 / 50;  51 / 51
-    //   4,096    61 / 66;  60 / 68          59 / 57;  59 / 58
-    //   5,184    79 / 71;  74 / 70          76 / 65;  71 / 62
+    // iteration, inverse / S (forward; adjoint):
+    //   vertices            FP64                  mixed
+    //     425          37 / 52;  24 / 40     37 / 48;  27 / 39
+    //   2,100          50 / 59;  55 / 63     48 / 54;  50 / 54
+    //   2,744          53 / 60;  58 / 67     52 / 54;  54 / 55
+    //   3,200          57 / 63;  61 / 71     57 / 57;  58 / 61
+    //   3,330          58 / 64;  62 / 71     58 / 58;  59 / 59
+    //   3,700          60 / 65;  61 / 69     60 / 58;  59 / 58
+    //   4,096 (cube)   63 / 68;  69 / 73     60 / 60;  63 / 64
+    //   4,096 (beam)   63 / 65;  64 / 68     59 / 57;  58 / 58
+    //   5,184          79 / 71;  74 / 70     76 / 65;  71 / 62
     // An adjoint's constrained iteration, which adds the gather and the scatter of
     // the contacts to S, takes 75 / 94 (FP64) and 73 / 80 (mixed) at 2,880 and 84 / 97
-    // and 77 / 88 at 4,096. So a mixed body without contacts changes over earlier.
-    // Forming the inverse takes 0.2 to 1.2 ms up to there.
+    // and 77 / 88 at 4,096. Mixed bodies without contacts are even from 3,300 on (S from
+    // 4.6% faster to 2.6% slower, by shape), so one limit serves all. Forming the inverse
+    // takes 0.2 to 1.2 ms.
     static constexpr int kDenseMaxVertices = 4096;
-    static constexpr int kDenseMaxMixedFree = 2816;  // mixed precision, no frictional boundary
     bool dense_inverse(const std::map<std::string, double>& opt, int precision);
-    bool dense_option(const std::map<std::string, double>& opt, int precision) const;  // the same without forming it
+    bool dense_option(const std::map<std::string, double>& opt) const;  // the same without forming it
     void ensure_dense(int precision);
     // x = x_prev + A^-1 r (uC: A^-1 r at the candidates, may be null), and
     // x += (A^-1)_C f; dval as in launch_dense_apply
